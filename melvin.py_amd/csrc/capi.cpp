@@ -195,9 +195,8 @@ struct mlv_plan {
   int fully, dtype, fd_order;
   double lx, lz, dx, dz, fx, fz, fx2, fz2;
   const void* tw;
-  void* work;     // 2-D: (nx, nm) complex intermediate; FD-z: Thomas d' (nn, nz) complex128
-  double* cp;     // FD-z Thomas factors (nn, nz)
-  double* rden;
+  void* work;     // 2-D: (nx, nm) complex intermediate; FD-z: Thomas d' (long rows only)
+  double2* fac;   // FD-z Thomas factors (cp, 1/den), laid out as thomas_layout says
   double lower;
   double* red_part;
   std::map<int, void*> basis_mats;  // dense per-axis transforms, built on first use
@@ -266,11 +265,15 @@ int mlv_plan_create(mlv_plan** out, int nx, int nz, double lx, double lz, int di
   } else {
     // Thomas factors of LaplacianSolver.py:21-52, built as a NumPy sweep would
     const int nn = p->nn;
-    std::vector<double> cp((size_t)nn * nz), rden((size_t)nn * nz);
+    int nt, K;
+    thomas_layout(nz, &nt, &K);
+    const size_t rowlen = nt ? (size_t)nt * K : (size_t)nz;
+    std::vector<double2> fac((size_t)nn * rowlen, make_double2(0.0, 1.0));
     const double inv_dz2 = 1.0 / (p->dz * p->dz);
     const double ddx = two_pi / lx;
     for (int n = 0; n < nn; ++n) {
       const double diag = -((n * ddx) * (n * ddx) + 2.0 / (p->dz * p->dz));
+      double2* row = fac.data() + (size_t)n * rowlen;
       double cprev = 0.0;
       for (int j = 0; j < nz; ++j) {
         const double dj = (j == 0 || j == nz - 1) ? 1.0 : diag;
@@ -278,18 +281,14 @@ int mlv_plan_create(mlv_plan** out, int nx, int nz, double lx, double lz, int di
         const double uj = (j == 0 || j == nz - 1) ? 0.0 : inv_dz2;
         const double den = j == 0 ? dj : dj - lj * cprev;
         const double c = uj / den;
-        cp[(size_t)n * nz + j] = c;
-        rden[(size_t)n * nz + j] = 1.0 / den;
+        row[nt ? (size_t)(j % K) * nt + j / K : (size_t)j] = make_double2(c, 1.0 / den);
         cprev = c;
       }
     }
     p->lower = inv_dz2;
-    HIP_TRY(hipMalloc(&p->work, (size_t)nn * nz * 16), "hipMalloc workspace");
-    HIP_TRY(hipMalloc((void**)&p->cp, cp.size() * sizeof(double)), "hipMalloc thomas");
-    HIP_TRY(hipMalloc((void**)&p->rden, rden.size() * sizeof(double)), "hipMalloc thomas");
-    HIP_TRY(hipMemcpy(p->cp, cp.data(), cp.size() * sizeof(double), hipMemcpyHostToDevice),
-            "upload thomas");
-    HIP_TRY(hipMemcpy(p->rden, rden.data(), rden.size() * sizeof(double), hipMemcpyHostToDevice),
+    if (!nt) HIP_TRY(hipMalloc(&p->work, (size_t)nn * nz * 16), "hipMalloc workspace");
+    HIP_TRY(hipMalloc((void**)&p->fac, fac.size() * sizeof(double2)), "hipMalloc thomas");
+    HIP_TRY(hipMemcpy(p->fac, fac.data(), fac.size() * sizeof(double2), hipMemcpyHostToDevice),
             "upload thomas");
   }
   HIP_TRY(hipMalloc((void**)&p->red_part, reduce_partials_bytes()), "hipMalloc partials");
@@ -308,8 +307,7 @@ int mlv_plan_create(mlv_plan** out, int nx, int nz, double lx, double lz, int di
 int mlv_plan_destroy(mlv_plan* p) {
   if (!p) return MLV_OK;
   if (p->work) (void)hipFree(p->work);
-  if (p->cp) (void)hipFree(p->cp);
-  if (p->rden) (void)hipFree(p->rden);
+  if (p->fac) (void)hipFree(p->fac);
   if (p->red_part) (void)hipFree(p->red_part);
   for (auto& kv : p->basis_mats) (void)hipFree(kv.second);
   delete p;
@@ -571,10 +569,10 @@ int mlv_poisson(mlv_plan* p, const void* rhs, void* out, void* stream) {
   CHECK_PTR(out);
   if (p->fully) return mlv_spec_op(p, MLV_SPEC_POISSON, rhs, out, stream);
   hipError_t e = DISPATCH(p,
-                          launch_thomas<float>(rhs, out, p->work, p->cp, p->rden, p->lower, 1.0,
+                          launch_thomas<float>(rhs, out, nullptr, p->work, p->fac, p->lower, 1.0, 0.0,
                                                p->nn, p->nz, (hipStream_t)stream),
-                          launch_thomas<double>(rhs, out, p->work, p->cp, p->rden, p->lower, 1.0,
-                                                p->nn, p->nz, (hipStream_t)stream));
+                          launch_thomas<double>(rhs, out, nullptr, p->work, p->fac, p->lower, 1.0,
+                                                0.0, p->nn, p->nz, (hipStream_t)stream));
   if (e != hipSuccess) return hip_fail(e, "poisson");
   return MLV_OK;
 }
@@ -678,10 +676,11 @@ int mlv_velocity(mlv_plan* p, const void* w, void* psi, void* ux_spec, void* uz_
   }
   if (ux_spec) return fail(MLV_ERR_ARG, "FD-z: ux comes from the physical z-derivative of psi");
   e = DISPATCH(p,
-               launch_thomas<float>(w, psi, p->work, p->cp, p->rden, p->lower, -1.0, p->nn, p->nz, s),
-               launch_thomas<double>(w, psi, p->work, p->cp, p->rden, p->lower, -1.0, p->nn, p->nz, s));
+               launch_thomas<float>(w, psi, uz_spec, p->work, p->fac, p->lower, -1.0, p->fx, p->nn,
+                                    p->nz, s),
+               launch_thomas<double>(w, psi, uz_spec, p->work, p->fac, p->lower, -1.0, p->fx, p->nn,
+                                     p->nz, s));
   if (e != hipSuccess) return hip_fail(e, "velocity poisson");
-  if (uz_spec) return mlv_spec_op(p, MLV_SPEC_DDX, psi, uz_spec, stream);
   return MLV_OK;
 }
 

@@ -44,9 +44,24 @@ hipError_t launch_combine(const void* hist, void* out, size_t n, int q, int curr
 template <typename T>
 hipError_t launch_velocity(const void* w, void* psi, void* ux, void* uz, int rows, int cols, int nn,
                            double fx, double fz, double fx2, double fz2, hipStream_t s);
+// Tridiagonal Poisson solve per x mode: out = solve(sign rhs) and, with uz,
+// uz = i fx n out.  fac holds (cp_j, 1/den_j) per element, rows of K nt
+// entries in the chunk-major layout of thomas_layout(nz) -- entry i nt + t is
+// element t K + i, padding (0, 1) -- or row-major where nt = 0 (dwork then
+// holds (nn, nz) complex128).
 template <typename T>
-hipError_t launch_thomas(const void* rhs, void* out, void* dwork, const double* cp,
-                         const double* rden, double lower, double sign, int nn, int nz,
-                         hipStream_t s);
+hipError_t launch_thomas(const void* rhs, void* out, void* uz, void* dwork, const double2* fac,
+                         double lower, double sign, double fx, int nn, int nz, hipStream_t s);
+// Threads per row and elements per thread of the solve: the fewest threads
+// that hold the row at kThomasKT elements each (about as many wavefronts as
+// the modes of one plan leave the chip room for), 0 threads for rows beyond
+// 1024 threads' reach, which one thread per mode sweeps.
+constexpr int kThomasKT = 4;
+inline void thomas_layout(int nz, int* nt, int* K) {
+  int n = 64;
+  while (n <= 1024 && n * kThomasKT < nz) n *= 2;
+  *nt = n <= 1024 ? n : 0;
+  *K = n <= 1024 ? (nz + n - 1) / n : 0;
+}
 
 }  // namespace mlv
