@@ -175,6 +175,17 @@ int mlv_combine(mlv_plan* plan, int moulton, int order, double dt, const void* h
  * may be NULL except psi. */
 int mlv_velocity(mlv_plan* plan, const void* w, void* psi, void* ux_spec, void* uz_spec,
                  void* stream);
+/* All of calc_velocity_from_vorticity (utility.py:62-79): mlv_velocity and the
+ * physical ux and uz.  FD-z also needs psi_phys (written), and ux_spec must
+ * be NULL there; psi_phys is not used in a fully spectral plan, whose outputs
+ * must not overwrite w. */
+int mlv_velocity_physical(mlv_plan* plan, const void* w, void* psi, void* ux_spec, void* uz_spec,
+                          void* psi_phys, void* ux_phys, void* uz_phys, void* stream);
+/* Variable.vec_dot_nabla (Variable.py:119-128): f_phys = to_physical(f_spec)
+ * unless f_spec is NULL, then out_spec = to_spectral(pddx(ux f) + pddz(uz f));
+ * ux, uz, f_phys are physical fields. */
+int mlv_advect(mlv_plan* plan, const void* ux, const void* uz, const void* f_spec, void* f_phys,
+               void* out_spec, void* stream);
 /* FP64 reduction of n values of type dtype (b used by SUMSQ2/DOT); writes
  * scale * result to out_f64 (device).  plan may be NULL: the call then uses
  * its device's shared partials buffer, which the first *_create call on the

@@ -4,11 +4,16 @@ operator: physical-space FD flux divergence of u*f, then a forward
 transform (Variable.py:119-128)."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
+import torch
 
 from . import _lib, hip
-from ._arrays import as_input
+from ._arrays import as_input, plain
 from ._plans import plan_for, ptr
+from .BasisFunctions import BasisFunctions
+from .SpectralTransformer import SpectralTransformer
 
 
 class Variable:
@@ -93,6 +98,8 @@ class Variable:
     def vec_dot_nabla(self, ux, uz, out=None, convert_to_physical=True):
         pl = plan_for(self._params)
         if out is None:
+            if self._fourier(pl):
+                return self._advect(pl, ux, uz, convert_to_physical)
             out = hip.zeros_like(self._pdata)
         if convert_to_physical:
             self.to_physical()
@@ -105,6 +112,27 @@ class Variable:
         if dst is not out:
             out.copy_(dst)
         return self._st.to_spectral(out, basis_functions=self._basis_functions)
+
+    def _fourier(self, pl):
+        """Whether this is a field of Fourier (or Fourier-x / FD-z) modes held
+        as the plan's kernels take it, transformed by this package."""
+        bx, bz = self._basis_functions
+        return (isinstance(self._st, SpectralTransformer) and self._st._plan is pl
+                and bx is BasisFunctions.COMPLEX_EXP
+                and bz is (BasisFunctions.COMPLEX_EXP if pl.fully else BasisFunctions.FDM)
+                and plain(self._sdata, pl.cplx, (pl.rows, pl.cols))
+                and plain(self._pdata, pl.real, (pl.nx, pl.nz)))
+
+    def _advect(self, pl, ux, uz, convert_to_physical):
+        """vec_dot_nabla whose flux divergence is formed inside the forward
+        transform, so the caller's ``out`` is the only thing it leaves out."""
+        a = as_input(ux, pl.real, (pl.nx, pl.nz))
+        b = as_input(uz, pl.real, (pl.nx, pl.nz))
+        spec = torch.empty((pl.rows, pl.cols), dtype=pl.cplx, device=self._pdata.device)
+        _lib.call("mlv_advect", pl.handle, ptr(a), ptr(b),
+                  ptr(self._sdata) if convert_to_physical else ctypes.c_void_p(0),
+                  ptr(self._pdata), ptr(spec), _lib.stream_handle())
+        return spec
 
     def save(self, dump_counter):
         np.save(self._dump_name + f"{dump_counter:04d}.npy", hip.asnumpy(self._pdata))

@@ -19,15 +19,22 @@ def as_input(a, dtype, shape=None):
 
 
 def output(out, dtype, shape, device=None):
-    """(tensor to write, tensor to return) for an optional ``out``."""
+    """(tensor to write, tensor to return) for an optional ``out``; the
+    operators write every element, so a new one starts uninitialised."""
     if out is None:
-        t = torch.zeros(shape, dtype=dtype, device=device or hip.device())
+        t = torch.empty(shape, dtype=dtype, device=device or hip.device())
         return t, t
     if tuple(out.shape) != tuple(shape):
         raise ValueError(f"out has shape {tuple(out.shape)}, expected {tuple(shape)}")
     if out.dtype == dtype and out.is_contiguous():
         return out, out
     return torch.empty(shape, dtype=dtype, device=out.device), out
+
+
+def plain(t, dtype, shape):
+    """Whether a kernel can read and write ``t`` in place as such an array."""
+    return (t.is_cuda and t.dtype == dtype and tuple(t.shape) == tuple(shape)
+            and t.is_contiguous())
 
 
 def finish(tmp, out):

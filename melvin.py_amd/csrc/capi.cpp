@@ -195,7 +195,7 @@ struct mlv_plan {
   int fully, dtype, fd_order;
   double lx, lz, dx, dz, fx, fz, fx2, fz2;
   const void* tw;
-  void* work;     // 2-D: (nx, nm) complex intermediate; FD-z: Thomas d' (long rows only)
+  void* work;     // 2-D: two (nx, nm) complex intermediates; FD-z: Thomas d' (long rows only)
   double2* fac;   // FD-z Thomas factors (cp, 1/den), laid out as thomas_layout says
   double lower;
   double* red_part;
@@ -261,7 +261,8 @@ int mlv_plan_create(mlv_plan** out, int nx, int nz, double lx, double lz, int di
     return rc;
   }
   if (p->fully) {
-    HIP_TRY(hipMalloc(&p->work, (size_t)nx * p->nm * cplx_bytes(dtype)), "hipMalloc workspace");
+    // (two: mlv_velocity_physical transforms ux and uz together)
+    HIP_TRY(hipMalloc(&p->work, 2 * (size_t)nx * p->nm * cplx_bytes(dtype)), "hipMalloc workspace");
   } else {
     // Thomas factors of LaplacianSolver.py:21-52, built as a NumPy sweep would
     const int nn = p->nn;
@@ -292,10 +293,8 @@ int mlv_plan_create(mlv_plan** out, int nx, int nz, double lx, double lz, int di
             "upload thomas");
   }
   HIP_TRY(hipMalloc((void**)&p->red_part, reduce_partials_bytes()), "hipMalloc partials");
-  size_t lds_need = dtype == MLV_F64 ? fft_lds_bytes<double>(lnx) : fft_lds_bytes<float>(lnx);
-  if (lnz > 0)
-    lds_need = std::max(lds_need, dtype == MLV_F64 ? fft_lds_bytes_row<double>(lnz)
-                                                   : fft_lds_bytes_row<float>(lnz));
+  const int lmax = std::max(lnx, lnz);
+  const size_t lds_need = dtype == MLV_F64 ? tr_lds_max<double>(lmax) : tr_lds_max<float>(lmax);
   if (lds_need > max_lds_per_block(p->device)) {
     mlv_plan_destroy(p);
     return fail(MLV_ERR_UNSUPPORTED, "transform does not fit the LDS of this device");
@@ -339,12 +338,14 @@ int mlv_to_physical(mlv_plan* p, const void* spec, void* phys, void* stream) {
     e = DISPATCH(p, launch_xinv<float>(p->lognx, spec, p->work, p->nn, p->nm, p->tw, s),
                  launch_xinv<double>(p->lognx, spec, p->work, p->nn, p->nm, p->tw, s));
     if (e != hipSuccess) return hip_fail(e, "to_physical x pass");
-    e = DISPATCH(p, launch_zc2r<float>(p->lognz, p->work, phys, p->nx, p->nm, p->tw, s),
-                 launch_zc2r<double>(p->lognz, p->work, phys, p->nx, p->nm, p->tw, s));
+    const Two a = {{p->work, nullptr}, {phys, nullptr}, 1};
+    e = DISPATCH(p, launch_zc2r<float>(p->lognz, a, p->nx, p->nm, p->tw, s),
+                 launch_zc2r<double>(p->lognz, a, p->nx, p->nm, p->tw, s));
     if (e != hipSuccess) return hip_fail(e, "to_physical z pass");
   } else {
-    e = DISPATCH(p, launch_xc2r_cols<float>(p->lognx, spec, phys, p->nn, p->nz, p->tw, s),
-                 launch_xc2r_cols<double>(p->lognx, spec, phys, p->nn, p->nz, p->tw, s));
+    const Two a = {{spec, nullptr}, {phys, nullptr}, 1};
+    e = DISPATCH(p, launch_xc2r_cols<float>(p->lognx, a, p->nn, p->nz, p->tw, s),
+                 launch_xc2r_cols<double>(p->lognx, a, p->nn, p->nz, p->tw, s));
     if (e != hipSuccess) return hip_fail(e, "to_physical x pass");
   }
   return MLV_OK;
@@ -400,10 +401,8 @@ static int fft_setup(int dtype, int axes, int nx, int nz, int* lognx, int* lognz
   int device = 0;
   HIP_TRY(hipGetDevice(&device), "hipGetDevice");
   const bool f64 = dtype == MLV_F64;
-  size_t lds = 0;
-  if (*lognx) lds = f64 ? fft_lds_bytes<double>(*lognx) : fft_lds_bytes<float>(*lognx);
-  if (*lognz)
-    lds = std::max(lds, f64 ? fft_lds_bytes_row<double>(*lognz) : fft_lds_bytes_row<float>(*lognz));
+  const int lmax = std::max(*lognx, *lognz);
+  const size_t lds = f64 ? tr_lds_max<double>(lmax) : tr_lds_max<float>(lmax);
   if (lds > max_lds_per_block(device)) return fail(MLV_ERR_UNSUPPORTED, "transform too long for LDS");
   return get_twiddles(device, dtype, tw);
 }
@@ -423,8 +422,8 @@ int mlv_rfft(int dtype, int axes, int nx, int nz, const void* in, void* out, voi
     e = f64 ? launch_xr2c_cols<double>(lx, in, out, nx / 2 + 1, nz, 1.0, tw, s)
             : launch_xr2c_cols<float>(lx, in, out, nx / 2 + 1, nz, 1.0, tw, s);
   } else if (axes == MLV_FFT_AXIS1) {
-    e = f64 ? launch_zr2c<double>(lz, in, out, nx, nz / 2 + 1, tw, s)
-            : launch_zr2c<float>(lz, in, out, nx, nz / 2 + 1, tw, s);
+    e = f64 ? launch_zr2c<double>(lz, in, out, nx, nz / 2 + 1, tw, s, false)
+            : launch_zr2c<float>(lz, in, out, nx, nz / 2 + 1, tw, s, false);
   } else {
     CHECK_PTR(work);
     const int nm = nz / 2 + 1;
@@ -451,21 +450,23 @@ int mlv_irfft(int dtype, int axes, int nx, int nz, const void* in, void* out, vo
   hipError_t e = hipSuccess;
   if (axes == MLV_FFT_AXIS0) {
     const double sc = 1.0 / nx;
-    e = f64 ? launch_xc2r_cols<double>(lx, in, out, nx / 2 + 1, nz, tw, s, sc)
-            : launch_xc2r_cols<float>(lx, in, out, nx / 2 + 1, nz, tw, s, sc);
+    const Two a = {{in, nullptr}, {out, nullptr}, 1};
+    e = f64 ? launch_xc2r_cols<double>(lx, a, nx / 2 + 1, nz, tw, s, sc)
+            : launch_xc2r_cols<float>(lx, a, nx / 2 + 1, nz, tw, s, sc);
   } else if (axes == MLV_FFT_AXIS1) {
     const double sc = 1.0 / nz;
-    e = f64 ? launch_zc2r<double>(lz, in, out, nx, nz / 2 + 1, tw, s, sc)
-            : launch_zc2r<float>(lz, in, out, nx, nz / 2 + 1, tw, s, sc);
+    const Two a = {{in, nullptr}, {out, nullptr}, 1};
+    e = f64 ? launch_zc2r<double>(lz, a, nx, nz / 2 + 1, tw, s, sc, false)
+            : launch_zc2r<float>(lz, a, nx, nz / 2 + 1, tw, s, sc, false);
   } else {
     CHECK_PTR(work);
     const int nm = nz / 2 + 1;
     const double sc = 1.0 / ((double)nx * (double)nz);
     e = f64 ? launch_xinv<double>(lx, in, work, nx / 2, nm, tw, s, nx, sc)
             : launch_xinv<float>(lx, in, work, nx / 2, nm, tw, s, nx, sc);
+    const Two a = {{work, nullptr}, {out, nullptr}, 1};
     if (e == hipSuccess)
-      e = f64 ? launch_zc2r<double>(lz, work, out, nx, nm, tw, s)
-              : launch_zc2r<float>(lz, work, out, nx, nm, tw, s);
+      e = f64 ? launch_zc2r<double>(lz, a, nx, nm, tw, s) : launch_zc2r<float>(lz, a, nx, nm, tw, s);
   }
   if (e != hipSuccess) return hip_fail(e, "irfft");
   return MLV_OK;
@@ -681,6 +682,82 @@ int mlv_velocity(mlv_plan* p, const void* w, void* psi, void* ux_spec, void* uz_
                launch_thomas<double>(w, psi, uz_spec, p->work, p->fac, p->lower, -1.0, p->fx, p->nn,
                                      p->nz, s));
   if (e != hipSuccess) return hip_fail(e, "velocity poisson");
+  return MLV_OK;
+}
+
+int mlv_velocity_physical(mlv_plan* p, const void* w, void* psi, void* ux_spec, void* uz_spec,
+                          void* psi_phys, void* ux_phys, void* uz_phys, void* stream) {
+  CHECK_PLAN(p);
+  CHECK_PTR(w);
+  CHECK_PTR(psi);
+  CHECK_PTR(uz_spec);
+  CHECK_PTR(ux_phys);
+  CHECK_PTR(uz_phys);
+  hipStream_t s = (hipStream_t)stream;
+  hipError_t e;
+  if (p->fully) {
+    CHECK_PTR(ux_spec);
+    // ux's and uz's blocks read w side by side with the spectra's stores
+    if (psi == w || ux_spec == w || uz_spec == w) return fail(MLV_ERR_ARG, "outputs overwrite w");
+    const VelArgs v = {w, psi, ux_spec, uz_spec, p->fx, p->fz, p->fx2, p->fz2};
+    e = DISPATCH(p, launch_xinv_vel<float>(p->lognx, v, p->work, p->nn, p->nm, p->tw, s),
+                 launch_xinv_vel<double>(p->lognx, v, p->work, p->nn, p->nm, p->tw, s));
+    if (e != hipSuccess) return hip_fail(e, "velocity x pass");
+    const char* work = static_cast<const char*>(p->work);
+    const Two a = {{work, work + (size_t)p->nx * p->nm * cplx_bytes(p->dtype)}, {ux_phys, uz_phys}, 2};
+    e = DISPATCH(p, launch_zc2r<float>(p->lognz, a, p->nx, p->nm, p->tw, s),
+                 launch_zc2r<double>(p->lognz, a, p->nx, p->nm, p->tw, s));
+    if (e != hipSuccess) return hip_fail(e, "velocity z pass");
+    return MLV_OK;
+  }
+  CHECK_PTR(psi_phys);
+  if (ux_spec) return fail(MLV_ERR_ARG, "FD-z: ux comes from the physical z-derivative of psi");
+  const int rc = mlv_velocity(p, w, psi, nullptr, uz_spec, stream);
+  if (rc) return rc;
+  const Two a = {{psi, uz_spec}, {psi_phys, uz_phys}, 2};
+  e = DISPATCH(p, launch_xc2r_cols<float>(p->lognx, a, p->nn, p->nz, p->tw, s),
+               launch_xc2r_cols<double>(p->lognx, a, p->nn, p->nz, p->tw, s));
+  if (e != hipSuccess) return hip_fail(e, "velocity x pass");
+  // -pddz: the stencil over a negated spacing
+  e = DISPATCH(p,
+               launch_fd<float>(psi_phys, ux_phys, p->nx, p->nz, 1, MLV_FD_DDZ, p->fd_order, 0,
+                                -p->dz, s),
+               launch_fd<double>(psi_phys, ux_phys, p->nx, p->nz, 1, MLV_FD_DDZ, p->fd_order, 0,
+                                 -p->dz, s));
+  if (e != hipSuccess) return hip_fail(e, "velocity z difference");
+  return MLV_OK;
+}
+
+int mlv_advect(mlv_plan* p, const void* ux, const void* uz, const void* f_spec, void* f_phys,
+               void* out_spec, void* stream) {
+  CHECK_PLAN(p);
+  CHECK_PTR(ux);
+  CHECK_PTR(uz);
+  CHECK_PTR(f_phys);
+  CHECK_PTR(out_spec);
+  hipStream_t s = (hipStream_t)stream;
+  // the stencils wrap at most once
+  if (p->nz < 5) return fail(MLV_ERR_ARG, "FD axis shorter than 5 points");
+  if (f_spec) {
+    const int rc = mlv_to_physical(p, f_spec, f_phys, stream);
+    if (rc) return rc;
+  }
+  const FluxArgs a = {ux, uz, f_phys, p->fd_order, p->fully, p->dx, p->dz};
+  hipError_t e;
+  if (p->fully) {
+    const double scale = 1.0 / ((double)p->nx * (double)p->nz);
+    e = DISPATCH(p, launch_zr2c_flux<float>(p->lognz, a, p->work, p->nx, p->nm, p->tw, s),
+                 launch_zr2c_flux<double>(p->lognz, a, p->work, p->nx, p->nm, p->tw, s));
+    if (e != hipSuccess) return hip_fail(e, "advection z pass");
+    e = DISPATCH(p, launch_xfwd<float>(p->lognx, p->work, out_spec, p->nn, p->nm, scale, p->tw, s),
+                 launch_xfwd<double>(p->lognx, p->work, out_spec, p->nn, p->nm, scale, p->tw, s));
+  } else {
+    const double scale = 1.0 / (double)p->nx;
+    e = DISPATCH(
+        p, launch_xr2c_cols_flux<float>(p->lognx, a, out_spec, p->nn, p->nz, scale, p->tw, s),
+        launch_xr2c_cols_flux<double>(p->lognx, a, out_spec, p->nn, p->nz, scale, p->tw, s));
+  }
+  if (e != hipSuccess) return hip_fail(e, "advection x pass");
   return MLV_OK;
 }
 

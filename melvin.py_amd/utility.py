@@ -9,6 +9,7 @@ import numpy as np
 from numpy.random import default_rng
 
 from . import _lib, hip
+from ._arrays import plain
 from ._plans import plan_for, ptr
 from .BasisFunctions import BasisFunctions
 
@@ -36,8 +37,9 @@ def calc_kinetic_energy(ux, uz, xp=hip, params=None):
 def calc_velocity_from_vorticity(vorticity, streamfunction, ux, uz,
                                  laplacian_solver=None):
     """psi = solve(-w); ux = -d(psi)/dz, uz = d(psi)/dx in physical space
-    (utility.py:62-79).  The spectral part is one HIP kernel (or the FD-z
-    tridiagonal solve); the physical fields come from the transforms."""
+    (utility.py:62-79).  The spectral part is formed inside the velocity's
+    inverse transform (or by the FD-z tridiagonal solve), and both velocities
+    are transformed in one launch per pass."""
     params = vorticity._params
     pl = plan_for(params)
     w = vorticity.gets()
@@ -46,6 +48,16 @@ def calc_velocity_from_vorticity(vorticity, streamfunction, ux, uz,
     if not (w.is_contiguous() and psi.is_contiguous()):
         raise ValueError("vorticity and streamfunction must be contiguous")
     fdm_z = streamfunction._basis_functions[1] is BasisFunctions.FDM
+    one = ((vorticity, streamfunction, ux, uz) if fdm_z or not pl.fully else (ux, uz))
+    if (all(v._fourier(pl) for v in one) and plain(w, pl.cplx, (pl.rows, pl.cols))
+            and plain(psi, pl.cplx, (pl.rows, pl.cols))
+            and len({w.data_ptr(), psi.data_ptr(), ux._sdata.data_ptr(),
+                     uz._sdata.data_ptr()}) == 4):
+        _lib.call("mlv_velocity_physical", pl.handle, ptr(w), ptr(psi),
+                  null if fdm_z else ptr(ux._sdata), ptr(uz._sdata),
+                  ptr(streamfunction._pdata) if fdm_z else null, ptr(ux._pdata),
+                  ptr(uz._pdata), _lib.stream_handle())
+        return
     _lib.call("mlv_velocity", pl.handle, ptr(w), ptr(psi),
               null if fdm_z else ptr(ux._sdata), ptr(uz._sdata),
               _lib.stream_handle())
