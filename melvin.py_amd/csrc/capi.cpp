@@ -1000,204 +1000,199 @@ int mlv_job_work_bytes(int problem, int nfield, int nx, int nz, int dtype, size_
   return MLV_OK;
 }
 
+}  // extern "C"
+
 // Host plan of a batch: the device job table and every launch table of
 // the job set, ready for one upload (mlv_batch_create, mlv_batch_rebuild).
 struct BatchPlan {
   std::vector<char> host;  // JobDev table
-  std::vector<int> pA[3][2], pB[2][BV_COUNT], pC[2], pCn[2], pCm[2];  // pA[shape][stage]
+  std::vector<int> pA[3][2], pC[3][2], pB[2][BV_COUNT];  // pA[shape][stage]
   BatchLaunch bl{};        // block counts and LDS sizes; pointers set by upload_batch
-  size_t ldsCn = 0;
   std::vector<int> nbB;
   std::vector<long long> loops0;
   std::string signature;
   int nstage = 1;
 };
 
-static int plan_batch(int dtype, const mlv_job_desc* jobs, int njobs, int device, BatchPlan& P) {
-  int rc = MLV_OK;
-  const size_t lds_max = max_lds_per_block(device);
-  const size_t jsz = dtype == MLV_F64 ? sizeof(JobDev<double>) : sizeof(JobDev<float>);
-  std::vector<char>& host = P.host;
-  host.assign(jsz * njobs, 0);
-  auto& pA = P.pA;
-  auto& pB = P.pB;
-  auto& pC = P.pC;
-  auto& pCn = P.pCn;
-  size_t& ldsCn = P.ldsCn;
-  for (int s = 0; s < 2; ++s) {
-    for (int a = 0; a < 3; ++a) pA[a][s].assign(njobs + 1, 0);
-    pC[s].assign(njobs + 1, 0);
-    pCn[s].assign(njobs + 1, 0);
-    P.pCm[s].assign(njobs + 1, 0);
-    for (int v = 0; v < BV_COUNT; ++v) pB[s][v].assign(njobs + 1, 0);
+// What the launch tables need of a job.
+struct JobShape {
+  int nstage, lognx, lognz, nm, nx;
+  int nA[2], neq[2], bvar[2];
+};
+
+template <typename T>
+static JobShape job_shape(const JobDev<T>& J) {
+  JobShape r{};
+  r.nstage = J.nstage;
+  r.lognx = J.lognx;
+  r.lognz = J.lognz;
+  r.nm = J.nm;
+  r.nx = J.nx;
+  for (int s = 0; s < J.nstage; ++s) {
+    r.nA[s] = J.st[s].nA;
+    r.neq[s] = J.st[s].neq;
+    r.bvar[s] = J.st[s].bvar;
   }
+  return r;
+}
+
+// Threads per block: `most`, halved while the launch has fewer than `want`
+// blocks and a half is still at least `least`.
+template <typename F>
+static int fill_threads(int most, int least, int want, F blocks_of) {
+  int nt = most;
+  while (nt / 2 >= least && blocks_of(nt) < want) nt /= 2;
+  return nt;
+}
+
+template <typename T>
+static int plan_batch_t(const mlv_job_desc* jobs, int njobs, int device, BatchPlan& P) {
+  constexpr bool f64 = sizeof(T) == 8;
+  const size_t lds_max = max_lds_per_block(device);
+  P.host.assign(sizeof(JobDev<T>) * njobs, 0);
+  JobDev<T>* J = reinterpret_cast<JobDev<T>*>(P.host.data());
+  std::vector<JobShape> sh(njobs);
   BatchLaunch& bl = P.bl;
   std::memset(&bl, 0, sizeof(bl));
   bl.njobs = njobs;
-  bl.okA[0] = bl.okA[1] = bl.okA[2] = 1;
-  bl.okC[0] = bl.okC[1] = bl.okC[2] = 1;
-  size_t ldsCm = 0;
-  bl.lognx_all = bl.lognz_all = 0;
+  bl.okA[2] = !f64;
+  // threads per block at least: one column of any job, two where the block
+  // is shrunk to fill the chip (a single column's rows move in runs of 8 or
+  // 16 bytes)
+  int one = 64, two = 64, mean = 64;
   for (int j = 0; j < njobs; ++j) {
-    int nstage, lognx, lognz, nm, nx;
-    int nA[2], neq[2], bvar[2];
-    if (dtype == MLV_F64) {
-      JobDev<double>& J = reinterpret_cast<JobDev<double>*>(host.data())[j];
-      rc = build_job<double>(jobs[j], J, j);
-      if (rc) break;
-      nstage = J.nstage;
-      lognx = J.lognx;
-      lognz = J.lognz;
-      nm = J.nm;
-      nx = J.nx;
-      for (int s = 0; s < nstage; ++s) {
-        nA[s] = J.st[s].nA;
-        neq[s] = J.st[s].neq;
-        bvar[s] = J.st[s].bvar;
-      }
-    } else {
-      JobDev<float>& J = reinterpret_cast<JobDev<float>*>(host.data())[j];
-      rc = build_job<float>(jobs[j], J, j);
-      if (rc) break;
-      nstage = J.nstage;
-      lognx = J.lognx;
-      lognz = J.lognz;
-      nm = J.nm;
-      nx = J.nx;
-      for (int s = 0; s < nstage; ++s) {
-        nA[s] = J.st[s].nA;
-        neq[s] = J.st[s].neq;
-        bvar[s] = J.st[s].bvar;
-      }
+    const int rc = build_job<T>(jobs[j], J[j], j);
+    if (rc) return rc;
+    sh[j] = job_shape(J[j]);
+    const JobShape& r = sh[j];
+    bl.lognx_all = (j == 0 || bl.lognx_all == r.lognx) ? r.lognx : -1;
+    bl.lognz_all = (j == 0 || bl.lognz_all == r.lognz) ? r.lognz : -1;
+    bl.lognx_max = std::max(bl.lognx_max, r.lognx);
+    one = std::max(one, xp_tps<T>(r.lognx));
+    two = std::max(two, 2 * xp_tps<T>(r.lognx));
+    if (J[j].split) {
+      bl.split = 1;
+      while (!mean_fits(r.lognz, mean)) mean *= 2;
     }
-    const bool f64 = dtype == MLV_F64;
-    bl.lognx_all = (j == 0 || bl.lognx_all == lognx) ? lognx : -1;
-    bl.lognz_all = (j == 0 || bl.lognz_all == lognz) ? lognz : -1;
-    // x passes: narrow (n) and wide (w) points policies, see fused_points
-    const int sla = f64 ? xinv_cols_host<double>(lognx) : xinv_cols_host<float>(lognx);
-    const size_t ldsa = f64 ? xinv_lds_bytes<double>(lognx) : xinv_lds_bytes<float>(lognx);
-    // kernel A's smaller block shape, where the job's transform fits it
-    const int sla1 = f64 ? xinv_cols_host<double>(lognx, 1) : xinv_cols_host<float>(lognx, 1);
-    const size_t ldsa1 = f64 ? xinv_lds_bytes<double>(lognx, 1) : xinv_lds_bytes<float>(lognx, 1);
-    if (sla1 < 1) bl.okA[1] = 0;
-    // kernel A's mixed tiles (stepA_mixed): every stage's ops, kMixCols
-    // columns of each, in shape 0's block
-    {
-      int max_nA = 0;
-      for (int s = 0; s < nstage; ++s) max_nA = std::max(max_nA, nA[s]);
-      if (f64 || !xmix_fits<float>(lognx, max_nA)) bl.okA[2] = 0;
+    int max_nA = 0;
+    for (int s = 0; s < r.nstage; ++s) max_nA = std::max(max_nA, r.nA[s]);
+    if (!f64 && !xmix_fits(r.lognx, max_nA)) bl.okA[2] = 0;
+    P.nstage = std::max(P.nstage, r.nstage);
+  }
+  if (!fixed_logn(bl.lognx_all)) bl.okA[2] = 0;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+      cus <= 0)
+    cus = 256;
+  // blocks of a stage at nt threads
+  auto blocksA = [&](const JobShape& r, int s, int nt) {
+    return r.nA[s] * ((r.nm + xp_cols<T>(r.lognx, nt) - 1) / xp_cols<T>(r.lognx, nt));
+  };
+  auto blocksC = [&](const JobShape& r, int s, int nt) {
+    return r.neq[s] * ((r.nm + xp_cols<T>(r.lognx, nt) - 1) / xp_cols<T>(r.lognx, nt));
+  };
+  auto total = [&](auto blocks, int nt) {
+    int n = 0;
+    for (const JobShape& r : sh) n += blocks(r, 0, nt);
+    return n;
+  };
+  // LDS a job's kernels need at nt threads, and whether the block holds a column
+  auto fits = [&](int nt) {
+    for (const JobShape& r : sh)
+      if (!xp_fits<T>(r.lognx, nt) || xp_lds_bytes<T>(r.lognx, nt) > lds_max) return false;
+    return true;
+  };
+  // Two blocks per CU: below that a launch is the chain of one block, and a
+  // block of half the columns has the same chain on twice the CUs (256^2 FP64
+  // update: 256 threads, 11 blocks, 8.6 us; 64 threads, 43 blocks, 6.8).
+  const int want = 2 * cus;
+  const int leastA = std::max(two, mean), mostA = f64 ? 256 : 512;
+  int ntA0 = fill_threads(std::max(mostA, one), leastA, want, [&](int nt) { return total(blocksA, nt); });
+  while (!fits(ntA0) && ntA0 / 2 >= std::max(one, mean)) ntA0 /= 2;
+  bl.ntA[0] = ntA0;
+  bl.ntA[1] = ntA0 / 2 >= std::max(one, mean) ? ntA0 / 2 : ntA0;
+  bl.ntA[2] = bl.okA[2] ? xmix_nt(bl.lognx_all) : 0;
+  int ntC0 = fill_threads(std::max(256, one), two, want, [&](int nt) { return total(blocksC, nt); });
+  while (!fits(ntC0) && ntC0 / 2 >= one) ntC0 /= 2;
+  bl.ntC[0] = ntC0;
+  bl.ntC[1] = bl.ntC[2] = fits(512) ? 512 : ntC0;
+  bl.okA[0] = bl.okA[1] = bl.okC[0] = bl.okC[1] = 1;
+  bl.okC[2] = !f64 && fixed_logn(bl.lognx_all);
+  if (!fits(bl.ntA[0]) || !fits(bl.ntC[0]))
+    return fail(MLV_ERR_UNSUPPORTED, "grid too large for LDS");
+  for (int s = 0; s < 2; ++s) {
+    for (int a = 0; a < 3; ++a) {
+      P.pA[a][s].assign(njobs + 1, 0);
+      P.pC[a][s].assign(njobs + 1, 0);
     }
-    const int sln = f64 ? fused_cols_host<double>(lognx, 0) : fused_cols_host<float>(lognx, 0);
-    const int slw = f64 ? fused_cols_host<double>(lognx, 1) : fused_cols_host<float>(lognx, 1);
-    const size_t ldsn = f64 ? fused_lds_bytes<double>(lognx, 0) : fused_lds_bytes<float>(lognx, 0);
-    const size_t ldsw = f64 ? fused_lds_bytes<double>(lognx, 1) : fused_lds_bytes<float>(lognx, 1);
-    // kernel C's 512-thread narrow shape (cshape_threads): single precision
-    const int slm = (cshape_threads(2) * 16) >> lognx;
-    const size_t ldsm = (size_t)slm * fft_ldsn(1 << lognx) * 8;
-    if (f64 || slm < 1 || slm > cshape_threads(2) || ldsm > lds_max) bl.okC[2] = 0;
+    for (int v = 0; v < BV_COUNT; ++v) P.pB[s][v].assign(njobs + 1, 0);
+  }
+  for (int j = 0; j < njobs; ++j) {
+    const JobShape& r = sh[j];
     // z pass: points per thread by program (bpoints); the largest LDS any
     // of the job's programs takes is checked here
     auto zslots = [&](int v) {
-      const int p = f64 ? bpoints<double>(lognz, bvar_nin(v), bvar_neq(v))
-                        : bpoints<float>(lognz, bvar_nin(v), bvar_neq(v));
-      return (kNT * p) >> lognz;
+      return (kNT * bpoints<T>(r.lognz, bvar_nin(v), bvar_neq(v))) >> r.lognz;
     };
     auto zlds = [&](int v) {
-      return (size_t)bslots_used(bvar_nin(v), bvar_neq(v), zslots(v)) * fft_ldsn(1 << lognz) *
-             (f64 ? 16 : 8);
+      return (size_t)bslots_used(bvar_nin(v), bvar_neq(v), zslots(v)) * fft_ldsn(1 << r.lognz) *
+             sizeof(cx<T>);
     };
-    size_t ldsz = 0;
-    for (int s = 0; s < nstage; ++s) ldsz = std::max(ldsz, zlds(bvar[s]));
-    if (ldsa > lds_max || ldsn > lds_max || ldsw > lds_max || ldsz > lds_max || sla < 1 ||
-        sln < 1 || slw < 1) {
-      rc = fail(MLV_ERR_UNSUPPORTED, "job " + std::to_string(j) + ": grid too large for LDS");
-      break;
-    }
-    if (nstage > P.nstage) P.nstage = nstage;
     for (int s = 0; s < 2; ++s) {
-      int a = 0, a1 = 0, a2 = 0, c = 0, cn = 0, cm = 0, bb = 0, bv = 0;
-      if (s < nstage) {
-        const int nin_v = bvar_nin(bvar[s]), neq_v = bvar_neq(bvar[s]);
-        const int slz = zslots(bvar[s]);
-        if (!bfits(nin_v, neq_v, slz)) {
-          rc = fail(MLV_ERR_UNSUPPORTED,
-                    "job " + std::to_string(j) + ": problem does not fit the z-pass LDS at this nz");
-          break;
-        }
-        const int rb = brows(nin_v, neq_v, slz);
-        a = nA[s] * ((nm + sla - 1) / sla);
-        a1 = sla1 >= 1 ? nA[s] * ((nm + sla1 - 1) / sla1) : 0;
-        a2 = (nm + kMixCols - 1) / kMixCols;
-        if (f64 ? bsplit_fits<double>(lognz, bvar[s]) : bsplit_fits<float>(lognz, bvar[s]))
-          bl.splitB = 1;
-        c = neq[s] * ((nm + slw - 1) / slw);
-        cn = neq[s] * ((nm + sln - 1) / sln);
-        cm = slm >= 1 ? neq[s] * ((nm + slm - 1) / slm) : 0;
-        bb = (nx + rb - 1) / rb;
-        bv = bvar[s];
+      const bool on = s < r.nstage;
+      for (int a = 0; a < 3; ++a) {
+        const int na = !on ? 0
+                       : a == 2 ? (r.nm + kMixCols - 1) / kMixCols
+                                : blocksA(r, s, bl.ntA[a]);
+        P.pA[a][s][j + 1] = P.pA[a][s][j] + na;
+        P.pC[a][s][j + 1] = P.pC[a][s][j] + (on ? blocksC(r, s, bl.ntC[a]) : 0);
+        if (bl.okA[a])
+          bl.ldsAp[a] = std::max(bl.ldsAp[a], xp_lds_bytes<T>(r.lognx, bl.ntA[a]));
+        bl.ldsCp[a] = std::max(bl.ldsCp[a], xp_lds_bytes<T>(r.lognx, bl.ntC[a]));
+        if (on && J[j].split && bl.okA[a])
+          bl.ldsAp[a] = std::max(bl.ldsAp[a], mean_lds_bytes(r.lognz, bl.ntA[a]));
+      }
+      int bb = 0, bv = 0;
+      if (on) {
+        bv = r.bvar[s];
+        const int slz = zslots(bv);
+        if (!bfits(bvar_nin(bv), bvar_neq(bv), slz) || zlds(bv) > lds_max)
+          return fail(MLV_ERR_UNSUPPORTED, "job " + std::to_string(j) +
+                                               ": problem does not fit the z-pass LDS at this nz");
+        const int rb = brows(bvar_nin(bv), bvar_neq(bv), slz);
+        bb = (r.nx + rb - 1) / rb;
+        if (bsplit_fits<T>(r.lognz, bv)) bl.splitB = 1;
         bl.ldsB[bv] = std::max(bl.ldsB[bv], zlds(bv));
       }
       if (s == 0) {
         P.nbB.push_back(bb);
         P.loops0.push_back(jobs[j].loops);
       }
-      pA[0][s][j + 1] = pA[0][s][j] + a;
-      pA[1][s][j + 1] = pA[1][s][j] + a1;
-      pA[2][s][j + 1] = pA[2][s][j] + a2;
-      pC[s][j + 1] = pC[s][j] + c;
-      pCn[s][j + 1] = pCn[s][j] + cn;
-      P.pCm[s][j + 1] = P.pCm[s][j] + cm;
-      for (int v = 0; v < BV_COUNT; ++v) pB[s][v][j + 1] = pB[s][v][j] + (v == bv ? bb : 0);
+      for (int v = 0; v < BV_COUNT; ++v)
+        P.pB[s][v][j + 1] = P.pB[s][v][j] + (v == bv ? bb : 0);
     }
-    if (rc) break;
-    bl.ldsAp[0] = std::max(bl.ldsAp[0], ldsa);
-    if (sla1 >= 1) bl.ldsAp[1] = std::max(bl.ldsAp[1], ldsa1);
-    ldsCm = std::max(ldsCm, ldsm);
-    bl.ldsAp[2] = bl.ldsAp[0];
-    // kernel M (single precision mean profiles): one LDS slot of nz
-    if (!f64 && jobs[j].mean_split)
-      bl.ldsM = std::max(bl.ldsM, (size_t)fft_ldsn(1 << lognz) * 8);
-    bl.ldsC = std::max(bl.ldsC, ldsw);
-    ldsCn = std::max(ldsCn, ldsn);
   }
-  if (!rc) {
-    // Kernel C: single precision always runs narrow -- 16 points per thread,
-    // the stencil's neighbours read through the cache, 112 VGPRs, so four
-    // blocks (16 wavefronts) share a CU and their loads overlap the others'
-    // transforms (measured on MI355X, KH 1024^2: -7 % kernel time at 8 and
-    // at 32 jobs against the wide form).  Double precision needs the
-    // register file either way and runs wide when its grid covers the
-    // device's block slots twice over at two blocks per CU.
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
-        cus <= 0)
-      cus = 256;
-    bl.wideC = (dtype == MLV_F64 && pC[0][njobs] >= 4 * cus) ? 1 : 0;
-    // the mixed tiles and the 512-thread update run in the kernels compiled
-    // for one x size; where it applies, the 512-thread update is the default
-    // (64 x 1024^2 FP32: 556 against 578 us per launch for the 256-thread
-    // narrow shape -- Px and Pz rows read in runs of 8 columns, not 4)
-    if (!fixed_logn(bl.lognx_all)) bl.okA[2] = bl.okC[2] = 0;
-    if (bl.okC[2]) bl.wideC = 2;
-    // kernel A: the default block shape; kernel B: the split-pass plan
-    bl.shapeA = 0;
-    bl.planB = kPlanSplit;
-    // choices picked by mlv_batch_autotune for the same set of jobs win
-    P.signature = batch_signature(dtype, jobs, njobs);
-    {
-      std::lock_guard<std::mutex> lk(g_tuned_mu);
-      auto it = g_tuned.find(P.signature);
-      if (it != g_tuned.end()) {
-        bl.shapeA = bl.okA[it->second.shapeA] ? it->second.shapeA : 0;
-        bl.planB = it->second.planB;
-        bl.wideC = bl.okC[it->second.wideC] ? it->second.wideC : bl.wideC;
-      }
-    }
-    bl.ldsCp[1] = bl.ldsC;
-    bl.ldsCp[0] = ldsCn;
-    bl.ldsCp[2] = bl.okC[2] ? ldsCm : 0;
+  bl.planB = kPlanSplit;
+  // defaults: 256-thread blocks in both kernels (single precision kernel A's
+  // shape 1: 38 against 43 us on a mixed batch up to 2048^2, 73 and 74 at 16 x
+  // 1024^2; FP64's shape 0 at 1024^2: 14.3 against 15.1)
+  bl.shapeA = f64 ? 0 : 1;
+  bl.wideC = 0;
+  // choices picked by mlv_batch_autotune for the same set of jobs win
+  P.signature = batch_signature(f64 ? MLV_F64 : MLV_F32, jobs, njobs);
+  std::lock_guard<std::mutex> lk(g_tuned_mu);
+  auto it = g_tuned.find(P.signature);
+  if (it != g_tuned.end()) {
+    bl.shapeA = bl.okA[it->second.shapeA] ? it->second.shapeA : 0;
+    bl.planB = it->second.planB;
+    bl.wideC = bl.okC[it->second.wideC] ? it->second.wideC : bl.wideC;
   }
-  return rc;
+  return MLV_OK;
+}
+
+static int plan_batch(int dtype, const mlv_job_desc* jobs, int njobs, int device, BatchPlan& P) {
+  return dtype == MLV_F64 ? plan_batch_t<double>(jobs, njobs, device, P)
+                          : plan_batch_t<float>(jobs, njobs, device, P);
 }
 
 // The tables of plan P on the device: the job table (with each job's
@@ -1218,9 +1213,7 @@ static int upload_batch(BatchHost* b, BatchPlan& P, const mlv_job_desc* jobs, in
     arrays.push_back({&P.pA[0][s], &bl.prefAp[0][s]});
     arrays.push_back({&P.pA[1][s], &bl.prefAp[1][s]});
     arrays.push_back({&P.pA[2][s], &bl.prefAp[2][s]});
-    arrays.push_back({&P.pC[s], &bl.prefCp[1][s]});
-    arrays.push_back({&P.pCn[s], &bl.prefCp[0][s]});
-    arrays.push_back({&P.pCm[s], &bl.prefCp[2][s]});
+    for (int c = 0; c < 3; ++c) arrays.push_back({&P.pC[c][s], &bl.prefCp[c][s]});
     for (int v = 0; v < BV_COUNT; ++v) arrays.push_back({&P.pB[s][v], &bl.prefB[s][v]});
   }
   std::vector<size_t> aoff;
@@ -1243,9 +1236,7 @@ static int upload_batch(BatchHost* b, BatchPlan& P, const mlv_job_desc* jobs, in
     bl.nAp[0][s] = P.pA[0][s][njobs];
     bl.nAp[1][s] = P.pA[1][s][njobs];
     bl.nAp[2][s] = P.pA[2][s][njobs];
-    bl.nCp[1][s] = P.pC[s][njobs];
-    bl.nCp[0][s] = P.pCn[s][njobs];
-    bl.nCp[2][s] = P.pCm[s][njobs];
+    for (int c = 0; c < 3; ++c) bl.nCp[c][s] = P.pC[c][s][njobs];
     for (int v = 0; v < BV_COUNT; ++v) bl.nB[s][v] = P.pB[s][v][njobs];
   }
   // diagnostics: the buffer not in use now, grown when needed
@@ -1319,6 +1310,8 @@ static void free_batch_memory(BatchHost* b) {
   b->tables = nullptr;
   b->diag_buf[0] = b->diag_buf[1] = nullptr;
 }
+
+extern "C" {
 
 int mlv_batch_create(mlv_batch** out, int dtype, const mlv_job_desc* jobs, int njobs) {
   if (!out || !jobs || njobs <= 0) return fail(MLV_ERR_ARG, "bad batch arguments");

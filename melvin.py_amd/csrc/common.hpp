@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace mlv {
 
 // Largest supported transform length (log2).  One twiddle table of this
@@ -31,6 +33,14 @@ using gptr = T*;
 template <typename T>
 __device__ __forceinline__ gptr<T> glb(T* p) { return (gptr<T>)p; }
 
+// Element of an array at a 32-bit byte offset: with a uniform pointer that is
+// one address register per access and no 64-bit arithmetic.
+template <typename V>
+__device__ __forceinline__ V& at32(V* p, uint32_t bytes) {
+  using C = std::conditional_t<std::is_const_v<V>, const char, char>;
+  return *reinterpret_cast<V*>(reinterpret_cast<C*>(p) + bytes);
+}
+
 template <typename T>
 __device__ __forceinline__ cx<T> mk(T re, T im) {
   cx<T> r;
@@ -42,9 +52,15 @@ template <typename T>
 __device__ __forceinline__ cx<T> cadd(cx<T> a, cx<T> b) { return mk<T>(a.x + b.x, a.y + b.y); }
 template <typename T>
 __device__ __forceinline__ cx<T> csub(cx<T> a, cx<T> b) { return mk<T>(a.x - b.x, a.y - b.y); }
+// a b + c with one rounding.  Where a sum of two products leaves the compiler
+// the choice which of them to fuse, it may choose differently in two
+// instantiations of one body; spelled out, every block shape of a kernel
+// gives the same bits.
+__device__ __forceinline__ float fma1(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma1(double a, double b, double c) { return __builtin_fma(a, b, c); }
 template <typename T>
 __device__ __forceinline__ cx<T> cmul(cx<T> a, cx<T> b) {
-  return mk<T>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return mk<T>(fma1(a.x, b.x, -(a.y * b.y)), fma1(a.x, b.y, a.y * b.x));
 }
 template <typename T>
 __device__ __forceinline__ cx<T> cscale(cx<T> a, T s) { return mk<T>(a.x * s, a.y * s); }

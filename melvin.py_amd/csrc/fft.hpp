@@ -51,7 +51,7 @@ __device__ __forceinline__ cx<T> rot(int k, cx<T> x) {
   const int j = k * (16 / R);
   const T c = T(kCos16[j]);
   const T s = T(DIR) * T(kCos16[(j + 12) & 15]);
-  return mk<T>(x.x * c - x.y * s, x.x * s + x.y * c);
+  return mk<T>(fma1(x.x, c, -(x.y * s)), fma1(x.x, s, x.y * c));
 }
 
 // In-register radix-R DFT, R a power of two <= 16 (recursive radix-2 DIT).

@@ -23,15 +23,17 @@
 namespace mlv {
 
 // Passes, and the radix (log2) and sub-transform length (log2) of pass p:
-// as few passes as E allows, the larger radices first.
-__host__ __device__ constexpr int rf_passes(int logn, int loge) { return (logn + loge - 1) / loge; }
-__host__ __device__ constexpr int rf_logr(int logn, int loge, int p) {
-  const int np = rf_passes(logn, loge);
+// as few passes as the largest radix 2^logm allows, the larger radices
+// first.  The radices alone decide a transform's rounding: two splits with
+// the same logm give the same bits.
+__host__ __device__ constexpr int rf_passes(int logn, int logm) { return (logn + logm - 1) / logm; }
+__host__ __device__ constexpr int rf_logr(int logn, int logm, int p) {
+  const int np = rf_passes(logn, logm);
   return logn / np + (p < logn % np ? 1 : 0);
 }
-__host__ __device__ constexpr int rf_logns(int logn, int loge, int p) {
+__host__ __device__ constexpr int rf_logns(int logn, int logm, int p) {
   int s = 0;
-  for (int i = 0; i < p; ++i) s += rf_logr(logn, loge, i);
+  for (int i = 0; i < p; ++i) s += rf_logr(logn, logm, i);
   return s;
 }
 // LDS position of point i: one spare element every E, so the first
@@ -59,14 +61,16 @@ __device__ __forceinline__ void rf_sync() {
 // the thread in the transform, NT the threads that synchronise together.
 // Before the call nobody still reads or writes the region; after it the last
 // reads of the region may be pending (rf_sync before writing it again).
-template <typename T, int LOGN, int LOGE, int DIR, int STRIDE, int NT, int PASS = 0>
+template <typename T, int LOGN, int LOGE, int DIR, int STRIDE, int NT,
+          int LOGM = (LOGE < 4 ? LOGE : 4), int PASS = 0>
 __device__ __forceinline__ void rf_fft(cx<T> (&v)[1 << LOGE], cx<T>* __restrict__ lds, int t,
                                        const cx<T>* __restrict__ tw) {
   constexpr int N = 1 << LOGN, E = 1 << LOGE, TPS = N / E;
-  constexpr int LOGR = rf_logr(LOGN, LOGE, PASS), R = 1 << LOGR;
-  constexpr int LOGNS = rf_logns(LOGN, LOGE, PASS), NS = 1 << LOGNS;
+  static_assert(LOGM <= LOGE && LOGM <= 4, "a butterfly is one thread's, radix 16 at most");
+  constexpr int LOGR = rf_logr(LOGN, LOGM, PASS), R = 1 << LOGR;
+  constexpr int LOGNS = rf_logns(LOGN, LOGM, PASS), NS = 1 << LOGNS;
   constexpr int B = E / R;  // butterflies per thread
-  constexpr bool LAST = PASS == rf_passes(LOGN, LOGE) - 1;
+  constexpr bool LAST = PASS == rf_passes(LOGN, LOGM) - 1;
   cx<T> u[B][R];
 #pragma unroll
   for (int i = 0; i < B; ++i) {
@@ -102,7 +106,7 @@ __device__ __forceinline__ void rf_fft(cx<T> (&v)[1 << LOGE], cx<T>* __restrict_
     rf_sync<NT>();
 #pragma unroll
     for (int m = 0; m < E; ++m) v[m] = lds[rf_pad<LOGE>(t + m * TPS) * STRIDE];
-    rf_fft<T, LOGN, LOGE, DIR, STRIDE, NT, PASS + 1>(v, lds, t, tw);
+    rf_fft<T, LOGN, LOGE, DIR, STRIDE, NT, LOGM, PASS + 1>(v, lds, t, tw);
   }
 }
 

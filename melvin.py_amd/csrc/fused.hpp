@@ -180,80 +180,75 @@ template <> struct BProg<BV_MHD2> {
   }
 };
 
-// Columns per block of the x-pass kernels: every LDS slot, but at most one
-// per thread, so that each thread keeps a single column (kNT % cols == 0).
-template <int LOGN, int P, int NT = kNT>
-__host__ __device__ constexpr int fused_cols() {
-  return fft_slots<LOGN, NT, P>() < NT ? fft_slots<LOGN, NT, P>() : NT;
-}
-// Kernel C's tile shapes (BatchLaunch::wideC): 0 narrow and 1 wide at kNT
-// threads (fused_points), 2 narrow at 512 threads -- twice the columns per
-// block, so each row of Px / Pz is read in runs of 8 (single precision,
-// batches of one x size, fixed_logn).
-__host__ __device__ constexpr int cshape_threads(int shape) { return shape == 2 ? 512 : kNT; }
-__host__ __device__ constexpr int cshape_wide(int shape) { return shape == 1 ? 1 : 0; }
-// Points per thread of the x passes.  wide = 1 is the column-pass policy
-// of fft_points_col (32 points from N = 1024 in single precision: more
-// columns per block); wide = 0 keeps 16 points up to N = 2048 (half the LDS
-// per block, so twice the blocks per CU, and a batch that mixes 2048 with
-// smaller grids keeps the smaller grids' occupancy: the launch's LDS is the
-// largest job's).  The x-inverse always runs narrow;
-// the x-forward/update kernel runs narrow in single precision and, in
-// double precision, wide when its grid fills the device several times over.
+// The x passes (kernels A and C) hold 2^xp_loge points of a column per
+// thread (fft_reg.hpp): 8, and above 1024 points 16 (FP64 at 4096 points 32)
+// where that keeps a block of several columns within its threads.  Sixteen
+// at 1024 points in single precision leave the update two rows' loads in
+// flight per thread instead of four: 180 against 154 us per launch at 16 x
+// 1024^2.  The count depends on the precision and the size alone, so a job
+// computes the same bits in any batch and block shape.
 template <typename T>
-__host__ __device__ constexpr int fused_points(int logn, int wide) {
-  return wide ? fft_points_col<T>(logn) : (logn >= 12 ? 32 : 16);
+__host__ __device__ constexpr int xp_loge(int logn) {
+  return sizeof(T) == 4 ? (logn >= 11 ? 4 : 3) : (logn >= 12 ? 5 : logn >= 11 ? 4 : 3);
 }
 template <typename T>
-inline int fused_cols_host(int logn, int wide) {
-  const int s = (kNT * fused_points<T>(logn, wide)) >> logn;
-  return s < kNT ? s : kNT;
+__host__ __device__ constexpr int xp_tps(int logn) {
+  return 1 << (logn - xp_loge<T>(logn));
+}
+// Columns per block of nt threads, and the LDS they take.
+template <typename T>
+__host__ __device__ constexpr int xp_cols(int logn, int nt) {
+  return nt / xp_tps<T>(logn);
 }
 template <typename T>
-inline size_t fused_lds_bytes(int logn, int wide) {
-  const int s = (kNT * fused_points<T>(logn, wide)) >> logn;
-  return (size_t)s * fft_ldsn(1 << logn) * sizeof(cx<T>);
+__host__ __device__ constexpr size_t xp_lds_bytes(int logn, int nt) {
+  return (size_t)xp_cols<T>(logn, nt) * rf_len(logn, xp_loge<T>(logn)) * sizeof(cx<T>);
+}
+constexpr size_t kLdsMax = 160 * 1024;
+template <typename T>
+__host__ __device__ constexpr bool xp_fits(int logn, int nt) {
+  return xp_cols<T>(logn, nt) >= 1 && xp_lds_bytes<T>(logn, nt) <= kLdsMax;
+}
+// The compact spectrum's row of x among n points, -1 for a truncated mode:
+// nn = (n - 1) / 3 follows from n, so most rows' cases are decided when a
+// size's body is compiled.
+__host__ __device__ constexpr int xp_nn(int n) { return (n - 1) / 3; }
+__device__ __forceinline__ constexpr int xp_row(int x, int n) {
+  return x <= xp_nn(n) ? x : (x >= n - xp_nn(n) ? x - n + 2 * xp_nn(n) + 1 : -1);
+}
+// Whether thread t's point t + m tps (0 <= t < tps) can be kept for some t.
+__host__ __device__ constexpr bool xp_any(int m, int tps, int n) {
+  return m * tps <= xp_nn(n) || (m + 1) * tps - 1 >= n - xp_nn(n);
+}
+// Points per thread (log2) of a mean profile's transform in a block of nt
+// threads, and whether it fits.
+__host__ __device__ constexpr int mean_loge(int logn, int nt) {
+  int e = 3;
+  while ((1 << (logn - e)) > nt) ++e;
+  return e;
+}
+__host__ __device__ constexpr bool mean_fits(int logn, int nt) {
+  return mean_loge(logn, nt) <= 4;
+}
+inline size_t mean_lds_bytes(int logn, int nt) {
+  return (size_t)rf_len(logn, mean_loge(logn, nt)) * sizeof(cx<float>);
 }
 
-// Threads per block of the x-inverse kernel A, by shape (BatchLaunch::
-// shapeA).  Shape 0, the default: single precision takes 512, so that a
-// block holds 8 columns at 1024 points and each interleaved row pair's store
-// is a whole 128-byte line (two such blocks per CU give as many wavefronts
-// as four blocks of 256); with 64-byte runs the stores of neighbouring tiles
-// only merged in L2 when their blocks ran side by side.  Double precision
-// takes 256 (4 columns of 16-byte values already fill a line, and 512 would
-// not fit the LDS at 4096 points).  Shape 1 halves the block (half the
-// columns per block, twice the blocks); shape 2 keeps shape 0's block with
-// every op of the stage side by side (stepA_mixed); the autotuner times
-// them.
-template <typename T, int SHAPE = 0>
-__host__ __device__ constexpr int xinv_threads() {
-  return (sizeof(T) == 4 ? 512 : 256) >> (SHAPE == 1 ? 1 : 0);
-}
-template <typename T, int LOGN, int P, int SHAPE = 0>
-__host__ __device__ constexpr int xinv_cols() {
-  return ((xinv_threads<T, SHAPE>() * P) >> LOGN) < xinv_threads<T, SHAPE>()
-             ? ((xinv_threads<T, SHAPE>() * P) >> LOGN)
-             : xinv_threads<T, SHAPE>();
-}
-template <typename T>
-inline int xinv_cols_host(int logn, int shape = 0) {
-  const int nt = (sizeof(T) == 4 ? 512 : 256) >> (shape == 1 ? 1 : 0);
-  const int s = (nt * fused_points<T>(logn, 0)) >> logn;
-  return s < nt ? s : nt;
-}
-template <typename T>
-inline size_t xinv_lds_bytes(int logn, int shape = 0) {
-  return (size_t)xinv_cols_host<T>(logn, shape) * fft_ldsn(1 << logn) * sizeof(cx<T>);
-}
-// Columns per block of every op in kernel A's mixed tiles (shape 2), and
-// the host check that a job's stages fit them: single precision at 2^9 and
-// 2^10 points, kMixCols x (the most ops of any stage) <= the block's slots.
+// Kernel A's block shapes (BatchLaunch::shapeA): 0, of at most 512 threads in
+// single and 256 in double precision; 1, half of shape 0's; 2, mixed tiles
+// (stepA_body's MIXED), single precision at 2^9 and 2^10 points with xmix_nt
+// threads, when kMixCols columns of every op of any stage fit the block.
+// Kernel C's tile shapes (BatchLaunch::wideC): 0 (narrow) of at most 256
+// threads, 1 (wide) and, single precision in a batch of one x size
+// (fixed_logn), 2, of 512.
+// "At most": a batch whose blocks would leave the chip idle takes smaller
+// ones (fill_threads in capi.cpp).
 constexpr int kMixCols = 2;
-template <typename T>
+__host__ __device__ constexpr int xmix_nt(int logn) {
+  return logn == 9 || logn == 10 ? 1024 : 0;
+}
 inline bool xmix_fits(int logn, int max_nA) {
-  return sizeof(T) == 4 && (logn == 9 || logn == 10) &&
-         kMixCols * max_nA <= xinv_cols_host<T>(logn, 0);
+  return xmix_nt(logn) > 0 && kMixCols * max_nA <= xp_cols<float>(logn, xmix_nt(logn));
 }
 
 // Rows per z-pass block: as many as fit the LDS slots, at most 8.
@@ -351,38 +346,37 @@ inline size_t fused_work_elems(int nin, int neq, int nx, int nz) {
 
 struct BatchLaunch {
   int njobs;
-  int shapeA;                          // block shape of kernel A (xinv_threads)
+  int split;                           // some job carries mean profiles
+  int shapeA;                          // block shape of kernel A
   int planB;                           // plan of kernel B (kPlanSplit / kPlanTwoSweep)
-  int wideC;                           // points policy of kernel C (fused_points)
+  int wideC;                           // tile shape of kernel C
   int nA[2], nB[2][BV_COUNT], nC[2];  // total blocks per launch
   size_t ldsA, ldsB[BV_COUNT], ldsC;
-  size_t ldsM;                         // single precision mean profiles: one slot; 0 = none
   int* prefA[2];                       // device prefix arrays (njobs + 1)
   int* prefB[2][BV_COUNT];
   int* prefC[2];
-  // the tile shapes of kernel C (index = shape, cshape_*; okC[2] = 0 outside
-  // single-precision batches of one x size); wideC / nC / ldsC / prefC
-  // above are the selected one
-  int okC[3];
-  int nCp[3][2];
-  size_t ldsCp[3];
-  int* prefCp[3][2];
-  // the block shapes of kernel A (index = shape; okA[s] = 0 where shape s
-  // does not apply to every job: the smaller block where a job's transform
-  // does not fit it, the mixed tiles outside xmix_fits or in a batch of
-  // several x sizes); nA / ldsA / prefA above are the selected one
-  int okA[3];
-  int nAp[3][2];
+  // the shapes of kernels A and C (index = shape): whether every job takes
+  // it, threads per block, blocks, LDS and prefix arrays; nA / ldsA / prefA
+  // and nC / ldsC / prefC above are the selected one's
+  int okA[3], ntA[3], nAp[3][2];
   size_t ldsAp[3];
   int* prefAp[3][2];
+  int okC[3], ntC[3], nCp[3][2];
+  size_t ldsCp[3];
+  int* prefCp[3][2];
   // whether some job's z pass takes the split-pass plan under kPlanSplit
   int splitB;
   // log2 of the x / z grid size shared by every job of the batch, -1 when
-  // the jobs differ: a batch of one grid size launches kernels compiled for
-  // that size alone (kFixedLogn), whose registers are their own rather than
-  // the largest over every size the generic kernels handle
+  // the jobs differ: a batch of one z size launches z-pass kernels compiled
+  // for that size alone (fixed_logn), whose registers are their own rather
+  // than the largest over every size the generic kernels handle
   int lognx_all, lognz_all;
+  int lognx_max;                       // the largest x size (log2)
 };
+
+// Kernels A and C are compiled for x sizes up to 2^kXpLo and for all: the
+// larger sizes' points per thread would set every size's registers.
+constexpr int kXpLo = 10;
 
 // Grid sizes with kernels compiled for them alone: 2^9 .. 2^11.
 __host__ __device__ constexpr bool fixed_logn(int logn) { return logn >= 9 && logn <= 11; }
@@ -397,7 +391,7 @@ inline void select_a_shape(BatchLaunch& bl, int shape) {
   }
 }
 
-// Select kernel C's tile shape (wide = 1: fused_points' wide policy).
+// Select kernel C's tile shape.
 inline void select_c_policy(BatchLaunch& bl, int shape) {
   bl.wideC = shape;
   bl.ldsC = bl.ldsCp[shape];

@@ -1,97 +1,114 @@
-// Fused step, x-inverse kernels: A (spectral prologue + inverse x pass)
-// and M (single-precision x-mean profiles); the bodies are in fused_xinv.hpp.
+// Fused step, x-inverse kernel A (spectral prologue + inverse x pass, and the
+// single-precision x-mean profiles); the bodies are in fused_xinv.hpp.
 #include "fused_xinv.hpp"
 
 namespace mlv {
 
-template <typename T, int SHAPE>
-__global__ void __launch_bounds__((xinv_threads<T, SHAPE>()))
-    k_stepA(const JobDev<T>* __restrict__ jobs, const int* __restrict__ pref, int njobs,
-            int stage, int step, const cx<T>* __restrict__ tw) {
+// Logical blocks [0, nA) are kernel A's, then kMeanCh / 2 per job for the
+// mean profiles.
+template <typename T, int NT, int LO, bool MIXED>
+__global__ void __launch_bounds__(NT)
+    __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 1)))
+    k_stepA(const JobDev<T>* __restrict__ jobs, const int* __restrict__ pref, int njobs, int nA,
+            int nM, int stage, int step, const cx<T>* __restrict__ tw) {
   extern __shared__ char smem_raw[];
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-  const int lb = xcd_logical(pref[njobs]);
+  int lb = xcd_logical(nA + nM);
   if (lb < 0) return;
-  roleA<T, SHAPE>(jobs, pref, njobs, lb, stage, step, tw, lds);
-}
-
-// A batch whose jobs all have 2^LOGN points along x (fixed_logn).
-template <typename T, int SHAPE, int LOGN>
-__global__ void __launch_bounds__((xinv_threads<T, SHAPE>()))
-    k_stepA_fixed(const JobDev<T>* __restrict__ jobs, const int* __restrict__ pref, int njobs,
-                  int stage, int step, const cx<T>* __restrict__ tw) {
-  extern __shared__ char smem_raw[];
-  cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-  const int lb = xcd_logical(pref[njobs]);
-  if (lb < 0) return;
-  roleA_fixed<T, SHAPE, LOGN>(jobs, pref, njobs, lb, stage, step, tw, lds);
-}
-
-// Grid: jobs x (kMeanCh / 2) op pairs.
-template <typename T>
-__global__ void __launch_bounds__(kNT) k_stepM(const JobDev<T>* __restrict__ jobs, int stage,
-                                               int step, const cx<T>* __restrict__ tw) {
-  extern __shared__ char smem_raw[];
-  cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-  roleM<T>(jobs[blockIdx.x / (kMeanCh / 2)], blockIdx.x % (kMeanCh / 2), stage, step, tw, lds);
+  if (sizeof(T) == 4 && lb >= nA) {
+    lb -= nA;
+    const JobDev<T>& J = jobs[lb / (kMeanCh / 2)];
+    if (stage >= J.nstage || !J.split) return;
+    const int pair = lb % (kMeanCh / 2), par = (J.par0 + step) & 1;
+    switch (J.lognz) {
+#define X(L)                                                               \
+  case L:                                                                  \
+    if constexpr (mean_fits(L, NT))                                        \
+      stepM_body<T, L, NT>(J, J.st[stage], pair, par, tw, lds);            \
+    break;
+      X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
+#undef X
+      default:
+        break;
+    }
+    return;
+  }
+  const int j = find_job(pref, njobs, lb);
+  const JobDev<T>& J = jobs[j];
+  const int local = lb - pref[j], par = (J.par0 + step) & 1;
+  switch (J.lognx) {
+#define X(L)                                                               \
+  case L:                                                                  \
+    if constexpr (L <= LO && xp_fits<T>(L, NT) && (!MIXED || xmix_nt(L) == NT))           \
+      stepA_body<T, L, NT, MIXED>(J, J.st[stage], local, par, tw, lds);    \
+    break;
+    X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
+#undef X
+    default:
+      break;
+  }
 }
 
 // --------------------------------------------------------------------------
 // Launchers
 // --------------------------------------------------------------------------
+template <typename T, int NT, int LO, bool MIXED>
+static void launchA_lo(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int step,
+                    const cx<T>* tw, hipStream_t s) {
+  const int nA = bl.nA[stage], nM = sizeof(T) == 4 && bl.split ? bl.njobs * (kMeanCh / 2) : 0;
+  MLV_SET_LDS_ONCE((k_stepA<T, NT, LO, MIXED>), bl.ldsA);
+  hipLaunchKernelGGL((k_stepA<T, NT, LO, MIXED>), dim3(xcd_grid(nA + nM)), dim3(NT), bl.ldsA, s, jobs,
+                     (const int*)bl.prefA[stage], bl.njobs, nA, nM, stage, step, tw);
+}
+
+template <typename T, int NT, bool MIXED>
+static void launchA(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int step,
+                    const cx<T>* tw, hipStream_t s) {
+  if (bl.lognx_max <= kXpLo)
+    launchA_lo<T, NT, kXpLo, MIXED>(jobs, bl, stage, step, tw, s);
+  else if constexpr (!MIXED)
+    launchA_lo<T, NT, 12, MIXED>(jobs, bl, stage, step, tw, s);
+}
+
 template <typename T>
 void launch_xinv(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int step,
                  const cx<T>* tw, hipStream_t s) {
-  if (bl.nA[stage] > 0) {
-    const dim3 grid(xcd_grid(bl.nA[stage]));
-    const int* pref = bl.prefA[stage];
-    if (fixed_logn(bl.lognx_all)) {
-#define MLV_A_FIXED(SH, L)                                                                  \
-  if (bl.shapeA == SH && bl.lognx_all == L) {                                               \
-    MLV_SET_LDS_ONCE((k_stepA_fixed<T, SH, L>), bl.ldsA);                                   \
-    hipLaunchKernelGGL((k_stepA_fixed<T, SH, L>), grid, dim3(xinv_threads<T, SH>()), bl.ldsA, \
-                       s, jobs, pref, bl.njobs, stage, step, tw);                           \
-  }
-      MLV_A_FIXED(0, 9) MLV_A_FIXED(0, 10) MLV_A_FIXED(0, 11)
-      MLV_A_FIXED(1, 9) MLV_A_FIXED(1, 10) MLV_A_FIXED(1, 11)
-      if constexpr (sizeof(T) == 4) {
-        MLV_A_FIXED(2, 9) MLV_A_FIXED(2, 10)
-      }
-#undef MLV_A_FIXED
-    } else if (bl.shapeA == 1) {
-      MLV_SET_LDS_ONCE((k_stepA<T, 1>), bl.ldsA);
-      hipLaunchKernelGGL((k_stepA<T, 1>), grid, dim3(xinv_threads<T, 1>()), bl.ldsA, s, jobs,
-                         pref, bl.njobs, stage, step, tw);
-    } else {
-      MLV_SET_LDS_ONCE((k_stepA<T, 0>), bl.ldsA);
-      hipLaunchKernelGGL((k_stepA<T, 0>), grid, dim3(xinv_threads<T, 0>()), bl.ldsA, s, jobs,
-                         pref, bl.njobs, stage, step, tw);
-    }
-  }
+  if (bl.nA[stage] == 0) return;
+  const int nt = bl.ntA[bl.shapeA];
   if constexpr (sizeof(T) == 4) {
-    if (bl.ldsM) {
-      MLV_SET_LDS_ONCE(k_stepM<T>, bl.ldsM);
-      hipLaunchKernelGGL(k_stepM<T>, dim3(bl.njobs * (kMeanCh / 2)), dim3(kNT), bl.ldsM, s, jobs,
-                         stage, step, tw);
-    }
+    if (bl.shapeA == 2) return launchA<T, 1024, true>(jobs, bl, stage, step, tw, s);
   }
+  switch (nt) {
+    case 64: return launchA<T, 64, false>(jobs, bl, stage, step, tw, s);
+    case 128: return launchA<T, 128, false>(jobs, bl, stage, step, tw, s);
+    case 256: return launchA<T, 256, false>(jobs, bl, stage, step, tw, s);
+    default: return launchA<T, 512, false>(jobs, bl, stage, step, tw, s);
+  }
+}
+
+template <typename T, int NT>
+static void prepareA(const BatchLaunch& bl, size_t lds) {
+  if (bl.lognx_max <= kXpLo)
+    MLV_SET_LDS_ONCE((k_stepA<T, NT, kXpLo, false>), lds);
+  else
+    MLV_SET_LDS_ONCE((k_stepA<T, NT, 12, false>), lds);
 }
 
 template <typename T>
 void prepare_xinv(const BatchLaunch& bl) {
-  if (bl.ldsAp[0]) MLV_SET_LDS_ONCE((k_stepA<T, 0>), bl.ldsAp[0]);
-  if (bl.okA[1] && bl.ldsAp[1]) MLV_SET_LDS_ONCE((k_stepA<T, 1>), bl.ldsAp[1]);
-#define MLV_A_FIXED(SH, L)                                                   \
-  if (bl.lognx_all == L && bl.ldsAp[SH] && bl.okA[SH])                        \
-    MLV_SET_LDS_ONCE((k_stepA_fixed<T, SH, L>), bl.ldsAp[SH]);
-  MLV_A_FIXED(0, 9) MLV_A_FIXED(0, 10) MLV_A_FIXED(0, 11)
-  MLV_A_FIXED(1, 9) MLV_A_FIXED(1, 10) MLV_A_FIXED(1, 11)
-  if constexpr (sizeof(T) == 4) {
-    MLV_A_FIXED(2, 9) MLV_A_FIXED(2, 10)
-  }
-#undef MLV_A_FIXED
-  if constexpr (sizeof(T) == 4) {
-    if (bl.ldsM) MLV_SET_LDS_ONCE(k_stepM<T>, bl.ldsM);
+  for (int a = 0; a < 3; ++a) {
+    if (!bl.okA[a]) continue;
+    const size_t lds = bl.ldsAp[a];
+    if constexpr (sizeof(T) == 4) {
+      if (a == 2) {
+        MLV_SET_LDS_ONCE((k_stepA<T, 1024, kXpLo, true>), lds);
+        continue;
+      }
+    }
+    if (bl.ntA[a] == 64) prepareA<T, 64>(bl, lds);
+    if (bl.ntA[a] == 128) prepareA<T, 128>(bl, lds);
+    if (bl.ntA[a] == 256) prepareA<T, 256>(bl, lds);
+    if (bl.ntA[a] == 512) prepareA<T, 512>(bl, lds);
   }
 }
 

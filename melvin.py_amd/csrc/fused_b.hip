@@ -26,7 +26,7 @@ static void launchB_plan(const JobDev<T>* jobs, const BatchLaunch& bl, int stage
   const dim3 grid(xcd_grid(bl.nB[stage][V]));
   const int* pref = bl.prefB[stage][V];
   if constexpr (sizeof(T) == 4) {
-    if (bl.ldsM) {  // some job carries mean profiles
+    if (bl.split) {  // some job carries mean profiles
       MLV_SET_LDS_ONCE((k_stepB<T, V, 1, PLAN>), bl.ldsB[V]);
       hipLaunchKernelGGL((k_stepB<T, V, 1, PLAN>), grid, dim3(kNT), bl.ldsB[V], s, jobs, pref,
                          bl.njobs, stage, flags, tw);

@@ -49,7 +49,7 @@ template <typename T, int V>
 static void launch_v(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int flags,
                      const cx<T>* tw, hipStream_t s) {
   // single precision with mean profiles: SPLIT = 1 (as in fused_b.hip)
-  const bool split = sizeof(T) == 4 && bl.ldsM;
+  const bool split = sizeof(T) == 4 && bl.split;
   if (bl.planB == kPlanTwoSweep) {
     if (split)
       launch_logn<T, V, sizeof(T) == 4 ? 1 : 0, kPlanTwoSweep>(jobs, bl, stage, flags, tw, s);

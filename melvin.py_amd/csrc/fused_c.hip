@@ -4,33 +4,17 @@
 
 namespace mlv {
 
-// Narrow single-precision blocks are held to 128 VGPRs (four wavefronts per
-// SIMD, matching the four blocks per CU their LDS allows).
-template <typename T, int WIDE>
-__global__ void __launch_bounds__(kNT)
-    __attribute__((amdgpu_waves_per_eu((WIDE || sizeof(T) == 8) ? 1 : 4)))
+// Single precision is held to 128 VGPRs (four wavefronts per SIMD).
+template <typename T, int NT, int LO>
+__global__ void __launch_bounds__(NT)
+    __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 1)))
     k_stepC(const JobDev<T>* __restrict__ jobs, JobDev<T>* clock, const int* __restrict__ pref,
             int njobs, int stage, int step, const cx<T>* __restrict__ tw) {
   extern __shared__ char smem_raw[];
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int lb = xcd_logical(pref[njobs]);
   if (lb < 0) return;
-  roleC<T, WIDE>(jobs, clock, pref, njobs, lb, stage, step, tw, lds);
-}
-
-// A batch whose jobs all have 2^LOGN points along x (fixed_logn), tile
-// shape SHAPE (cshape_*).
-template <typename T, int SHAPE, int LOGN>
-__global__ void __launch_bounds__(cshape_threads(SHAPE))
-    __attribute__((amdgpu_waves_per_eu((SHAPE == 1 || sizeof(T) == 8) ? 1 : 4)))
-    k_stepC_fixed(const JobDev<T>* __restrict__ jobs, JobDev<T>* clock,
-                  const int* __restrict__ pref, int njobs, int stage, int step,
-                  const cx<T>* __restrict__ tw) {
-  extern __shared__ char smem_raw[];
-  cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
-  const int lb = xcd_logical(pref[njobs]);
-  if (lb < 0) return;
-  roleC_fixed<T, SHAPE, LOGN>(jobs, clock, pref, njobs, lb, stage, step, tw, lds);
+  roleC<T, NT, LO>(jobs, clock, pref, njobs, lb, stage, step, tw, lds);
 }
 
 template <typename T>
@@ -58,53 +42,54 @@ __global__ void __launch_bounds__(kNT) k_diag(JobDev<T>* jobs, double cutoff, in
 // --------------------------------------------------------------------------
 // Launchers
 // --------------------------------------------------------------------------
+template <typename T, int NT, int LO>
+static void launchC_lo(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int step,
+                       const cx<T>* tw, hipStream_t s) {
+  MLV_SET_LDS_ONCE((k_stepC<T, NT, LO>), bl.ldsC);
+  hipLaunchKernelGGL((k_stepC<T, NT, LO>), dim3(xcd_grid(bl.nC[stage])), dim3(NT), bl.ldsC, s, jobs,
+                     const_cast<JobDev<T>*>(jobs), (const int*)bl.prefC[stage], bl.njobs, stage,
+                     step, tw);
+}
+
+template <typename T, int NT>
+static void launchC(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int step,
+                    const cx<T>* tw, hipStream_t s) {
+  if (bl.lognx_max <= kXpLo)
+    launchC_lo<T, NT, kXpLo>(jobs, bl, stage, step, tw, s);
+  else
+    launchC_lo<T, NT, 12>(jobs, bl, stage, step, tw, s);
+}
+
 template <typename T>
 void launch_update(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int step,
                    const cx<T>* tw, hipStream_t s) {
   if (bl.nC[stage] == 0) return;
-  if (fixed_logn(bl.lognx_all)) {
-#define MLV_C_FIXED(W, L)                                                                     \
-  if (bl.wideC == W && bl.lognx_all == L) {                                                   \
-    MLV_SET_LDS_ONCE((k_stepC_fixed<T, W, L>), bl.ldsC);                                      \
-    hipLaunchKernelGGL((k_stepC_fixed<T, W, L>), dim3(xcd_grid(bl.nC[stage])),                \
-                       dim3(cshape_threads(W)),                                               \
-                       bl.ldsC, s, jobs, const_cast<JobDev<T>*>(jobs),                        \
-                       (const int*)bl.prefC[stage], bl.njobs, stage, step, tw);               \
+  switch (bl.ntC[bl.wideC]) {
+    case 64: return launchC<T, 64>(jobs, bl, stage, step, tw, s);
+    case 128: return launchC<T, 128>(jobs, bl, stage, step, tw, s);
+    case 256: return launchC<T, 256>(jobs, bl, stage, step, tw, s);
+    default: return launchC<T, 512>(jobs, bl, stage, step, tw, s);
   }
-    MLV_C_FIXED(0, 9) MLV_C_FIXED(0, 10) MLV_C_FIXED(0, 11)
-    MLV_C_FIXED(1, 9) MLV_C_FIXED(1, 10) MLV_C_FIXED(1, 11)
-    if constexpr (sizeof(T) == 4) {
-      MLV_C_FIXED(2, 9) MLV_C_FIXED(2, 10) MLV_C_FIXED(2, 11)
-    }
-#undef MLV_C_FIXED
-    return;
-  }
-  if (bl.wideC) {
-    MLV_SET_LDS_ONCE((k_stepC<T, 1>), bl.ldsC);
-    hipLaunchKernelGGL((k_stepC<T, 1>), dim3(xcd_grid(bl.nC[stage])), dim3(kNT), bl.ldsC, s,
-                       jobs, const_cast<JobDev<T>*>(jobs), (const int*)bl.prefC[stage], bl.njobs,
-                       stage, step, tw);
-  } else {
-    MLV_SET_LDS_ONCE((k_stepC<T, 0>), bl.ldsC);
-    hipLaunchKernelGGL((k_stepC<T, 0>), dim3(xcd_grid(bl.nC[stage])), dim3(kNT), bl.ldsC, s,
-                       jobs, const_cast<JobDev<T>*>(jobs), (const int*)bl.prefC[stage], bl.njobs,
-                       stage, step, tw);
-  }
+}
+
+template <typename T, int NT>
+static void prepareC(const BatchLaunch& bl, size_t lds) {
+  if (bl.lognx_max <= kXpLo)
+    MLV_SET_LDS_ONCE((k_stepC<T, NT, kXpLo>), lds);
+  else
+    MLV_SET_LDS_ONCE((k_stepC<T, NT, 12>), lds);
 }
 
 template <typename T>
 void prepare_update(const BatchLaunch& bl) {
-  if (bl.ldsCp[1]) MLV_SET_LDS_ONCE((k_stepC<T, 1>), bl.ldsCp[1]);
-  if (bl.ldsCp[0]) MLV_SET_LDS_ONCE((k_stepC<T, 0>), bl.ldsCp[0]);
-#define MLV_C_FIXED(W, L) \
-  if (bl.lognx_all == L && bl.ldsCp[W] && bl.okC[W])                                       \
-    MLV_SET_LDS_ONCE((k_stepC_fixed<T, W, L>), bl.ldsCp[W]);
-  MLV_C_FIXED(0, 9) MLV_C_FIXED(0, 10) MLV_C_FIXED(0, 11)
-  MLV_C_FIXED(1, 9) MLV_C_FIXED(1, 10) MLV_C_FIXED(1, 11)
-  if constexpr (sizeof(T) == 4) {
-    MLV_C_FIXED(2, 9) MLV_C_FIXED(2, 10) MLV_C_FIXED(2, 11)
+  for (int c = 0; c < 3; ++c) {
+    if (!bl.okC[c]) continue;
+    const size_t lds = bl.ldsCp[c];
+    if (bl.ntC[c] == 64) prepareC<T, 64>(bl, lds);
+    if (bl.ntC[c] == 128) prepareC<T, 128>(bl, lds);
+    if (bl.ntC[c] == 256) prepareC<T, 256>(bl, lds);
+    if (bl.ntC[c] == 512) prepareC<T, 512>(bl, lds);
   }
-#undef MLV_C_FIXED
 }
 
 template <typename T>
