@@ -1006,7 +1006,8 @@ int mlv_job_work_bytes(int problem, int nfield, int nx, int nz, int dtype, size_
 // the job set, ready for one upload (mlv_batch_create, mlv_batch_rebuild).
 struct BatchPlan {
   std::vector<char> host;  // JobDev table
-  std::vector<int> pA[3][2], pC[3][2], pB[2][BV_COUNT];  // pA[shape][stage]
+  std::vector<int> pA[3][2], pC[3][2];  // [shape][stage]
+  std::vector<int> pZ[2][2][2][BV_COUNT];  // [register / two-sweep][plan][stage][program]
   BatchLaunch bl{};        // block counts and LDS sizes; pointers set by upload_batch
   std::vector<int> nbB;
   std::vector<long long> loops0;
@@ -1067,6 +1068,7 @@ static int plan_batch_t(const mlv_job_desc* jobs, int njobs, int device, BatchPl
     const JobShape& r = sh[j];
     bl.lognx_all = (j == 0 || bl.lognx_all == r.lognx) ? r.lognx : -1;
     bl.lognz_all = (j == 0 || bl.lognz_all == r.lognz) ? r.lognz : -1;
+    bl.lognz_max = std::max(bl.lognz_max, r.lognz);
     bl.lognx_max = std::max(bl.lognx_max, r.lognx);
     one = std::max(one, xp_tps<T>(r.lognx));
     two = std::max(two, 2 * xp_tps<T>(r.lognx));
@@ -1125,7 +1127,9 @@ static int plan_batch_t(const mlv_job_desc* jobs, int njobs, int device, BatchPl
       P.pA[a][s].assign(njobs + 1, 0);
       P.pC[a][s].assign(njobs + 1, 0);
     }
-    for (int v = 0; v < BV_COUNT; ++v) P.pB[s][v].assign(njobs + 1, 0);
+    for (auto& kind : P.pZ)
+      for (auto& plan : kind)
+        for (int v = 0; v < BV_COUNT; ++v) plan[s][v].assign(njobs + 1, 0);
   }
   for (int j = 0; j < njobs; ++j) {
     const JobShape& r = sh[j];
@@ -1152,24 +1156,45 @@ static int plan_batch_t(const mlv_job_desc* jobs, int njobs, int device, BatchPl
         if (on && J[j].split && bl.okA[a])
           bl.ldsAp[a] = std::max(bl.ldsAp[a], mean_lds_bytes(r.lognz, bl.ntA[a]));
       }
-      int bb = 0, bv = 0;
+      int nreg = 0, nsweep = 0, bv = 0;
+      bool choice = false, sweep = false;  // LDS-staged under kPlanTwoSweep, always
       if (on) {
         bv = r.bvar[s];
         const int slz = zslots(bv);
-        if (!bfits(bvar_nin(bv), bvar_neq(bv), slz) || zlds(bv) > lds_max)
+        sweep = !z_reg_fits<T>(r.lognz, bv);
+        choice = bsplit_fits<T>(r.lognz, bv);
+        if ((sweep || choice) &&
+            (!bfits(bvar_nin(bv), bvar_neq(bv), slz) || zlds(bv) > lds_max))
           return fail(MLV_ERR_UNSUPPORTED, "job " + std::to_string(j) +
                                                ": problem does not fit the z-pass LDS at this nz");
-        const int rb = brows(bvar_nin(bv), bvar_neq(bv), slz);
-        bb = (r.nx + rb - 1) / rb;
-        if (bsplit_fits<T>(r.lognz, bv)) bl.splitB = 1;
-        bl.ldsB[bv] = std::max(bl.ldsB[bv], zlds(bv));
+        if (sweep || choice) {
+          const int rb = brows(bvar_nin(bv), bvar_neq(bv), slz);
+          nsweep = (r.nx + rb - 1) / rb;
+        }
+        if (!sweep) {
+          if (z_lds_bytes<T>(r.lognz, bv) > lds_max)
+            return fail(MLV_ERR_UNSUPPORTED, "job " + std::to_string(j) +
+                                                 ": problem does not fit the z-pass LDS at this nz");
+          nreg = (r.nx + z_rows(r.lognz) - 1) / z_rows(r.lognz);
+        }
+        if (choice) bl.splitB = 1;
       }
       if (s == 0) {
-        P.nbB.push_back(bb);
+        P.nbB.push_back(std::max(nreg, nsweep));
         P.loops0.push_back(jobs[j].loops);
       }
-      for (int v = 0; v < BV_COUNT; ++v)
-        P.pB[s][v][j + 1] = P.pB[s][v][j] + (v == bv ? bb : 0);
+      for (int plan = 0; plan < 2; ++plan) {
+        const bool swept = sweep || (choice && plan == kPlanTwoSweep);
+        for (int v = 0; v < BV_COUNT; ++v) {
+          auto& pr = P.pZ[0][plan][s][v];
+          auto& ps = P.pZ[1][plan][s][v];
+          pr[j + 1] = pr[j] + (on && v == bv && !swept ? nreg : 0);
+          ps[j + 1] = ps[j] + (on && v == bv && swept ? nsweep : 0);
+        }
+        if (on && !swept)
+          bl.z[plan].lds[bv] = std::max(bl.z[plan].lds[bv], z_lds_bytes<T>(r.lognz, bv));
+        if (on && swept) bl.zsweep[plan].lds[bv] = std::max(bl.zsweep[plan].lds[bv], zlds(bv));
+      }
     }
   }
   bl.planB = kPlanSplit;
@@ -1214,7 +1239,11 @@ static int upload_batch(BatchHost* b, BatchPlan& P, const mlv_job_desc* jobs, in
     arrays.push_back({&P.pA[1][s], &bl.prefAp[1][s]});
     arrays.push_back({&P.pA[2][s], &bl.prefAp[2][s]});
     for (int c = 0; c < 3; ++c) arrays.push_back({&P.pC[c][s], &bl.prefCp[c][s]});
-    for (int v = 0; v < BV_COUNT; ++v) arrays.push_back({&P.pB[s][v], &bl.prefB[s][v]});
+    for (int plan = 0; plan < 2; ++plan)
+      for (int v = 0; v < BV_COUNT; ++v) {
+        arrays.push_back({&P.pZ[0][plan][s][v], &bl.z[plan].pref[s][v]});
+        arrays.push_back({&P.pZ[1][plan][s][v], &bl.zsweep[plan].pref[s][v]});
+      }
   }
   std::vector<size_t> aoff;
   for (auto& a : arrays) {
@@ -1237,7 +1266,11 @@ static int upload_batch(BatchHost* b, BatchPlan& P, const mlv_job_desc* jobs, in
     bl.nAp[1][s] = P.pA[1][s][njobs];
     bl.nAp[2][s] = P.pA[2][s][njobs];
     for (int c = 0; c < 3; ++c) bl.nCp[c][s] = P.pC[c][s][njobs];
-    for (int v = 0; v < BV_COUNT; ++v) bl.nB[s][v] = P.pB[s][v][njobs];
+    for (int plan = 0; plan < 2; ++plan)
+      for (int v = 0; v < BV_COUNT; ++v) {
+        bl.z[plan].n[s][v] = P.pZ[0][plan][s][v][njobs];
+        bl.zsweep[plan].n[s][v] = P.pZ[1][plan][s][v][njobs];
+      }
   }
   // diagnostics: the buffer not in use now, grown when needed
   std::vector<size_t> doff(njobs);

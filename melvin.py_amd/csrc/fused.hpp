@@ -110,7 +110,7 @@ __device__ __forceinline__ uint32_t bf2_pack(float re, float im) {
 // means m and fluctuations f (single-precision mean split, see kernel M)
 template <typename T>
 __device__ __forceinline__ T bil(T am, T af, T bm, T bf) {
-  return am * bf + af * bm + af * bf;
+  return fma1(am + af, bf, af * bm);
 }
 
 // Per-variant channel/product description used by kernel B.  products()
@@ -278,18 +278,47 @@ __host__ __device__ constexpr int bpoints(int logn, int nin, int neq) {
 __host__ __device__ constexpr int bvar_nin(int v) { return v <= BV_VORT3 ? v + 3 : 6; }
 __host__ __device__ constexpr int bvar_neq(int v) { return v <= BV_VORT3 ? v + 1 : 1; }
 
-// The split-pass z pass (inverse 16,16,R with the products in its last
-// pass, forward R,16,16) applies at 2^9..2^11 points when the program runs
-// at 16 points per thread and fits the slots.
+// Sizes with a choice of z-pass plan: 2^9..2^11 points when the program runs
+// at 16 points per thread and fits the slots of the two-sweep pass.
 template <typename T>
 __host__ __device__ constexpr bool bsplit_fits(int logn, int v) {
   return logn >= 9 && logn <= 11 && bpoints<T>(logn, bvar_nin(v), bvar_neq(v)) == 16 &&
          bfits(bvar_nin(v), bvar_neq(v), (kNT * 16) >> logn);
 }
-// Plans of the z pass (BatchLaunch::planB): the split-pass plan where it
-// applies, or the two-sweep plan everywhere (16,16,R both ways, the
-// products in a sweep of their own between the transforms).
+// Plans of the z pass (BatchLaunch::planB).  kPlanTwoSweep runs the sizes
+// that bsplit_fits names on the LDS-staged pass in 16,16,R passes both ways,
+// the products in a sweep of their own.  kPlanSplit runs them with the
+// products between the last inverse and the first forward pass (single
+// precision), or on the register pass (double precision, stepZ_body).
 constexpr int kPlanSplit = 0, kPlanTwoSweep = 1;
+
+// The register z pass: 2^logn points over z_tps threads (a wavefront, or
+// part of one: 8 points per thread up to 512, 16 at 1024, 32 at 2048), one
+// wavefront per input channel or output, whichever are more.
+__host__ __device__ constexpr int z_tps(int logn) { return logn >= 9 ? 64 : 1 << (logn - 3); }
+__host__ __device__ constexpr int z_loge(int logn) { return logn >= 9 ? logn - 6 : 3; }
+__host__ __device__ constexpr int z_waves(int v) {
+  const int in = bvar_nin(v), out = 2 * bvar_neq(v);
+  return in > out ? in : out;
+}
+__host__ __device__ constexpr int z_rows(int logn) { return 2 * (64 / z_tps(logn)); }
+template <typename T>
+__host__ __device__ constexpr size_t z_lds_bytes(int logn, int v) {
+  return (size_t)z_waves(v) * (64 / z_tps(logn)) * rf_len(logn, z_loge(logn)) * sizeof(cx<T>);
+}
+// Sizes the register pass takes, in double precision; the rest (4096 points,
+// and programs of six regions at 2048) run the two-sweep pass under either
+// plan.
+template <typename T>
+__host__ __device__ constexpr bool z_reg_fits(int logn, int v) {
+  return sizeof(T) == 8 && logn <= 11 && z_lds_bytes<T>(logn, v) <= kLdsMax;
+}
+// Whether register m of a thread holds a kept coefficient or its mirror.
+__host__ __device__ constexpr bool z_any(int m, int tps, int n) {
+  return m * tps < xp_nn(n) || (m + 1) * tps - 1 > n - xp_nn(n);
+}
+// Kernels compiled for z extents up to 2^kZLo and up to 2^11.
+constexpr int kZLo = 10;
 
 // workspace channel of equation e's Px (k=0) / Pz (k=1) output; the
 // z-pass inputs occupy channels [0, base)
@@ -344,17 +373,25 @@ inline size_t fused_work_elems(int nin, int neq, int nx, int nz) {
   return (size_t)(nin + 2 * neq) * work_chs(nx, nm) + (size_t)(kMeanCh / 2) * nz;
 }
 
+// A z-pass launch's blocks, LDS and device prefix arrays by stage and program.
+struct ZLaunch {
+  int n[2][BV_COUNT];
+  size_t lds[BV_COUNT];
+  int* pref[2][BV_COUNT];
+};
+
 struct BatchLaunch {
   int njobs;
   int split;                           // some job carries mean profiles
   int shapeA;                          // block shape of kernel A
   int planB;                           // plan of kernel B (kPlanSplit / kPlanTwoSweep)
   int wideC;                           // tile shape of kernel C
-  int nA[2], nB[2][BV_COUNT], nC[2];  // total blocks per launch
-  size_t ldsA, ldsB[BV_COUNT], ldsC;
+  int nA[2], nC[2];                    // total blocks per launch
+  size_t ldsA, ldsC;
   int* prefA[2];                       // device prefix arrays (njobs + 1)
-  int* prefB[2][BV_COUNT];
   int* prefC[2];
+  // by plan: the jobs on the register z pass, and those on the LDS-staged pass
+  ZLaunch z[2], zsweep[2];
   // the shapes of kernels A and C (index = shape): whether every job takes
   // it, threads per block, blocks, LDS and prefix arrays; nA / ldsA / prefA
   // and nC / ldsC / prefC above are the selected one's
@@ -366,19 +403,20 @@ struct BatchLaunch {
   int* prefCp[3][2];
   // whether some job's z pass takes the split-pass plan under kPlanSplit
   int splitB;
-  // log2 of the x / z grid size shared by every job of the batch, -1 when
-  // the jobs differ: a batch of one z size launches z-pass kernels compiled
-  // for that size alone (fixed_logn), whose registers are their own rather
-  // than the largest over every size the generic kernels handle
+  // log2 of the x / z size shared by every job, -1 when they differ: a single-
+  // precision batch of one z size launches z-pass kernels compiled for that
+  // size alone (fixed_logn), whose registers are their own rather than the
+  // largest over every size the generic kernels handle
   int lognx_all, lognz_all;
-  int lognx_max;                       // the largest x size (log2)
+  int lognx_max, lognz_max;            // the largest sizes (log2)
 };
 
 // Kernels A and C are compiled for x sizes up to 2^kXpLo and for all: the
 // larger sizes' points per thread would set every size's registers.
 constexpr int kXpLo = 10;
 
-// Grid sizes with kernels compiled for them alone: 2^9 .. 2^11.
+// One-size batches that take kernel C's shape 2, kernel A's mixed tiles and
+// single precision's z-pass kernels of one size.
 __host__ __device__ constexpr bool fixed_logn(int logn) { return logn >= 9 && logn <= 11; }
 
 // Select kernel A's block shape.
@@ -439,12 +477,11 @@ template <typename T>
 void prepare_zpass(const BatchLaunch& bl);
 template <typename T>
 void prepare_update(const BatchLaunch& bl);
-// The z pass of program v for a batch of one z size (fixed_logn), compiled
-// in its own translation unit (fused_b_fixed.hip).
-template <typename T>
-void launch_zpass_fixed(int v, const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int flags,
-                        const cx<T>* tw, hipStream_t s);
-template <typename T>
+
+// Single precision's z pass of program v for a batch of one z size
+// (fixed_logn), compiled in its own translation unit (fused_b_fixed.hip).
+void launch_zpass_fixed(int v, const JobDev<float>* jobs, const BatchLaunch& bl, int stage,
+                        int flags, const cx<float>* tw, hipStream_t s);
 void prepare_zpass_fixed(const BatchLaunch& bl);
 
 }  // namespace mlv

@@ -1,6 +1,5 @@
 // Device bodies of the fused step's z-pass kernel B (c2r of the channel
-// rows, physical products, r2c of the products), launched by fused_b.hip
-// (generic) and fused_b_fixed.hip (one z size).
+// rows, physical products, r2c of the products), launched by fused_b.hip.
 #pragma once
 #include "fused.hpp"
 #include "diag_dev.hpp"
@@ -8,7 +7,223 @@
 
 namespace mlv {
 // --------------------------------------------------------------------------
-// Kernel B: z pass, c2r of the channels, products, r2c of the products
+// Kernel B: z pass, c2r of the channels, products, r2c of the products.
+//
+// A row pair's channels pack both rows into one complex sequence each, and
+// so do its products: output (e, k) holds row a's u_k f_e in the real and
+// row b's in the imaginary part.  One wavefront transforms one channel of a
+// pair (of 64 / TPS pairs where a row takes fewer threads) in registers
+// (fft_reg.hpp), leaves its values in LDS, forms one product with the value
+// that it holds itself and one that it reads, and transforms that back: the
+// two block barriers are around the exchange, and every transform's own
+// exchanges stay inside the wavefront.
+// Double precision's z pass: what bounds it is the chain of one pair at small
+// sizes (256^2 9.8 -> 5.8 us) and its traffic above (1024^2 19.3 -> 19.0 us,
+// 45 MB).
+// --------------------------------------------------------------------------
+// Two consecutive elements (16 bytes in single precision, one load).
+template <typename T>
+__device__ __forceinline__ void load_two(const cx<T>* __restrict__ p, cx<T>& a, cx<T>& b) {
+  if constexpr (sizeof(T) == 4) {
+    const float4 v = *reinterpret_cast<const float4*>(p);
+    a = mk<T>(v.x, v.y);
+    b = mk<T>(v.z, v.w);
+  } else {
+    a = p[0];
+    b = p[1];
+  }
+}
+
+// Running diagnostics partials of a z-pass thread.
+template <typename T>
+struct BDiag {
+  T mux = -INFINITY, muz = -INFINITY;  // NaN-propagating maxima, as np.max
+  double ke = 0.0, ens = 0.0, flux = 0.0;
+};
+
+// A job's partials of the blocks beyond its count (the two plans split a
+// grid into different numbers of blocks) hold no points; the last block
+// writes them.
+template <int NT>
+__device__ __forceinline__ void neutral_parts(double* part, int local, int count, int all) {
+  if (local != count - 1) return;
+  for (int i = count + (int)threadIdx.x; i < all; i += NT) {
+    double* p = part + (size_t)kDiagPart * i;
+    p[0] = p[1] = -INFINITY;
+    for (int q = 2; q < kDiagPart; ++q) p[q] = 0.0;
+  }
+}
+
+// The output a wavefront forms and the channels it multiplies: its own (or,
+// for a wavefront without one, `first`) and `second`.  MHD's outputs take
+// two more (-(u f) + b g).
+struct ZOut {
+  int e, k;           // equation, 0 for Px / 1 for Pz; e < 0: none
+  int first, second;  // channels
+};
+template <int V>
+__device__ __forceinline__ constexpr ZOut z_out(int ch) {
+  if constexpr (V == BV_VORT1) {  // f, ux, uz
+    if (ch == 1) return {0, 0, 1, 0};
+    if (ch == 2) return {0, 1, 2, 0};
+  } else if constexpr (V == BV_VORT2) {  // f0, f1, ux, uz
+    if (ch == 0) return {0, 0, 0, 2};
+    if (ch == 1) return {1, 1, 1, 3};
+    if (ch == 2) return {1, 0, 2, 1};
+    if (ch == 3) return {0, 1, 3, 0};
+  } else if constexpr (V == BV_VORT3) {  // f0, f1, f2, ux, uz
+    if (ch == 0) return {0, 0, 0, 3};
+    if (ch == 1) return {1, 1, 1, 4};
+    if (ch == 2) return {2, 0, 2, 3};
+    if (ch == 3) return {1, 0, 3, 1};
+    if (ch == 4) return {0, 1, 4, 0};
+    if (ch == 5) return {2, 1, 4, 2};
+  } else {  // w, j, ux, uz, bx, bz
+    const int f = V == BV_MHD1 ? 0 : 1;
+    if (ch == 2) return {0, 0, 2, f};
+    if (ch == 3) return {0, 1, 3, f};
+  }
+  return {-1, 0, 0, 0};
+}
+
+template <typename T, int LOGN, int V>
+__device__ __forceinline__ void stepZ_body(const JobDev<T>& J, const StageDev& S, int local,
+                                           int flags, const cx<T>* __restrict__ tw, cx<T>* lds) {
+#pragma clang fp contract(off)
+  using Pg = BProg<V>;
+  constexpr int NIN = Pg::NIN, NW = z_waves(V), NT = 64 * NW;
+  constexpr int N = 1 << LOGN, TPS = z_tps(LOGN), E = N / TPS, PB = 64 / TPS;
+  constexpr int LOGE = z_loge(LOGN), LDSN = rf_len(LOGN, LOGE), nm = xp_nn(N);
+  const int nx = J.nx;
+  const uint32_t chs = (uint32_t)work_chs(nx, nm);
+  const int ch = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, sub = lane / TPS, t = TPS == 1 ? 0 : lane % TPS;
+  const int x0 = 2 * (local * PB + sub);
+  const bool live = x0 < nx;
+  auto region = [&](int c, int sb) { return lds + (c * PB + sb) * LDSN; };
+  cx<T>* __restrict__ mine = region(ch, sub);
+  cx<T>* __restrict__ work = glb(J.work);
+  // the wavefront's product
+  const ZOut o = z_out<V>(ch);
+  const bool out = o.e >= 0;
+  constexpr bool mhd = V == BV_MHD1 || V == BV_MHD2;
+  const int cb = 4 + o.k, cg = V == BV_MHD1 ? 1 : 0;  // MHD's second pair
+  cx<T> v[E];
+  if (ch < NIN) {
+    const uint32_t base = ((uint32_t)ch * chs + (uint32_t)xrow_base(live ? x0 : 0, nm)) * (uint32_t)sizeof(cx<T>);
+    // a wavefront issuing its loads goes ahead of other blocks' arithmetic
+    __builtin_amdgcn_s_setprio(1);
+    cx<T> a[E], b[E];
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      a[m] = b[m] = czero<T>();
+      if (!z_any(m, TPS, N)) continue;
+      const int x = t + m * TPS, k = 2 * x <= N ? x : N - x;
+      if (k < nm) load_two<T>(&at32(work, base + (uint32_t)k * (2 * (uint32_t)sizeof(cx<T>))), a[m], b[m]);
+    }
+    __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const int x = t + m * TPS;
+      v[m] = 2 * x <= N ? mk<T>(a[m].x - b[m].y, a[m].y + b[m].x)
+                        : mk<T>(a[m].x + b[m].y, b[m].x - a[m].y);
+      if (m == 0 && t == 0) v[m] = mk<T>(a[m].x, b[m].x);
+    }
+    rf_fft<T, LOGN, LOGE, +1, 1, 64>(v, mine, t, tw);
+    rf_sync<64>();
+#pragma unroll
+    for (int m = 0; m < E; ++m) mine[rf_pad<LOGE>(t + m * TPS)] = v[m];
+  }
+  __syncthreads();
+  // this job's check loop (J.loops counts the loops before this one)
+  const bool diag = (flags & kDiag) && J.loops % (flags >> kDiagShift) == 0;
+  if (diag || (flags & kWritePhys)) {
+    BDiag<T> d;
+    for (int i = threadIdx.x; i < PB * N; i += NT) {
+      const int sb = i / N, n = i % N, xa = 2 * (local * PB + sb);
+      if (xa >= nx) continue;
+      cx<T> q[NIN];
+#pragma unroll
+      for (int c = 0; c < NIN; ++c) {
+        q[c] = region(c, sb)[rf_pad<LOGE>(n)];
+      }
+      if (diag) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          auto val = [&](int c) { return r ? q[c].y : q[c].x; };
+          const double ux = (double)val(Pg::UX), uz = (double)val(Pg::UZ), w = (double)val(0);
+          d.mux = nan_max(d.mux, val(Pg::UX));
+          d.muz = nan_max(d.muz, val(Pg::UZ));
+          d.ke += uz * uz + ux * ux;
+          d.ens += w * w;
+          if constexpr (Pg::FLUX >= 0) d.flux += (double)val(Pg::FLUX) * uz;
+        }
+      }
+      if (flags & kWritePhys) {
+#pragma unroll
+        for (int c = 0; c < NIN; ++c)
+#pragma unroll
+          for (int p = 0; p < kMaxPhys; ++p)
+            if (S.phys_ch[p] == c) {
+              T* __restrict__ o = glb(J.phys[p]) + (size_t)xa * N + n;
+              o[0] = q[c].x;
+              o[N] = q[c].y;
+            }
+      }
+    }
+    if (diag) {
+      double* part = glb(J.diag);
+      block_diag<NT>((double)d.mux, (double)d.muz, d.ke, d.ens, d.flux,
+                     part + (size_t)kDiagPart * local);
+      neutral_parts<NT>(part, local, (nx + 2 * PB - 1) / (2 * PB), J.nbB);
+    }
+  }
+  if (out) {
+    const cx<T>* __restrict__ sec = region(o.second, sub);
+    const cx<T>* __restrict__ fst = region(o.first, sub);
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const int i = rf_pad<LOGE>(t + m * TPS);
+      const cx<T> a = o.first == ch ? v[m] : fst[i], b = sec[i];
+      const T px = a.x * b.x, py = a.y * b.y;
+      if constexpr (mhd) {
+        const cx<T> c = region(cb, sub)[i], g = region(cg, sub)[i];
+        v[m] = mk<T>(fma1(c.x, g.x, -px), fma1(c.y, g.y, -py));
+      } else {
+        v[m] = mk<T>(-px, -py);
+      }
+    }
+  }
+  // every value is read before any transform writes over it
+  __syncthreads();
+  if (!out) return;
+  rf_fft<T, LOGN, LOGE, -1, 1, 64>(v, mine, t, tw);
+  rf_sync<64>();
+#pragma unroll
+  for (int m = 0; m < E; ++m)
+    if (z_any(m, TPS, N)) mine[rf_pad<LOGE>(t + m * TPS)] = v[m];
+  rf_sync<64>();
+  const uint32_t obase = ((uint32_t)pchan(NIN, o.e, o.k) * chs + (uint32_t)x0 * kPGroup) * (uint32_t)sizeof(cx<T>);
+#pragma unroll
+  for (int m = 0; m <= E / 2; ++m) {
+    if (m * TPS >= nm) continue;
+    const int k = t + m * TPS;
+    if (live && k < nm) {
+      const cx<T> y = mine[rf_pad<LOGE>(k)], ym = mine[rf_pad<LOGE>((N - k) & (N - 1))];
+      const uint32_t at = obase + (uint32_t)pidx(0, k, nx) * (uint32_t)sizeof(cx<T>);
+      at32(work, at) = mk<T>(T(0.5) * (y.x + ym.x), T(0.5) * (y.y - ym.y));
+      at32(work, at + kPGroup * (uint32_t)sizeof(cx<T>)) = mk<T>(T(0.5) * (y.y + ym.y), T(0.5) * (ym.x - y.x));
+    }
+  }
+}
+
+// --------------------------------------------------------------------------
+// The LDS-staged z pass: channel rows staged in LDS, 16 or 32 points per
+// thread.  Single precision runs it at every size (its blocks hold more
+// rows and its products, between two fused passes, cost no LDS trip of their
+// own: 106 against 120 us at 16 x 1024^2 with the register pass, 12 against 15
+// on tearing at 4 x 512^2, 43 against 58 on a mixed batch of double
+// diffusion), double precision the two-sweep plan and z_reg_fits' exceptions.
 // --------------------------------------------------------------------------
 // SPLIT (single precision): jobs with split carry mean profiles (kernel M)
 // and mean-free channels; a batch without such jobs runs SPLIT = 0.
@@ -47,19 +262,6 @@ struct BShape {
   static_assert(SLN <= bslots_used(NIN, NEQ, SL) && NO <= bslots_used(NIN, NEQ, SL),
                 "the launch's LDS holds the slots in use");
 };
-
-// Two consecutive elements (16 bytes in single precision, one load).
-template <typename T>
-__device__ __forceinline__ void load_two(const cx<T>* __restrict__ p, cx<T>& a, cx<T>& b) {
-  if constexpr (sizeof(T) == 4) {
-    const float4 v = *reinterpret_cast<const float4*>(p);
-    a = mk<T>(v.x, v.y);
-    b = mk<T>(v.z, v.w);
-  } else {
-    a = p[0];
-    b = p[1];
-  }
-}
 
 // Load phase: the block's input channel rows into the LDS slots, two real
 // sequences per slot packed as one Hermitian spectrum (zero-padded from nm
@@ -122,13 +324,6 @@ __device__ __forceinline__ void bload(const cx<T>* __restrict__ work, size_t chs
     for (int k = nm + lane + 64 * ssub; k <= N - nm; k += 64 * WPS) z[fft_pad(k)] = czero<T>();
   }
 }
-
-// Running diagnostics partials of a z-pass thread.
-template <typename T>
-struct BDiag {
-  T mux = -INFINITY, muz = -INFINITY;  // NaN-propagating maxima, as np.max
-  double ke = 0.0, ens = 0.0, flux = 0.0;
-};
 
 // The physical work at one point n of the block's rows, v[q] the value of
 // sequence q = row * NIN + channel (a fluctuation when kSplit): the
@@ -264,8 +459,12 @@ __device__ __forceinline__ void stepB_body(const JobDev<T>& J, const StageDev& S
       for (int o = 0; o < RB * NEQ; ++o)
         if (o < nrows * NEQ) lds[o * LDSN + fft_pad(n)] = mk<T>(px[o], pz[o]);
     }
-    if (diag) block_diag<kNT>((double)d.mux, (double)d.muz, d.ke, d.ens, d.flux,
-                              glb(J.diag) + (size_t)kDiagPart * local);
+    if (diag) {
+      double* part = glb(J.diag);
+      block_diag<kNT>((double)d.mux, (double)d.muz, d.ke, d.ens, d.flux,
+                      part + (size_t)kDiagPart * local);
+      neutral_parts<kNT>(part, local, (nx + RB - 1) / RB, J.nbB);
+    }
     __syncthreads();
     fft_lds<T, LOGN, -1, kNT, P, true>(lds, nrows * NEQ, tw);
     bstore<T, Sh>(glb(J.work), chs, nm, nx, x0, nrows, lds);
@@ -399,7 +598,9 @@ __device__ __forceinline__ void roleB(const JobDev<T>* __restrict__ jobs, const 
   switch (J.lognz) {
 #define X(L)                                                          \
   case L:                                                             \
-    if constexpr (PLAN == kPlanSplit && bsplit_ok<T, L, V>())         \
+    if constexpr (sizeof(T) == 8 && L < 9)                            \
+      break; /* the register pass's */                                \
+    else if constexpr (PLAN == kPlanSplit && bsplit_ok<T, L, V>())    \
       stepB_split<T, L, V, SPLIT>(J, J.st[stage], local, flags, tw, lds); \
     else                                                              \
       stepB_body<T, L, V, SPLIT>(J, J.st[stage], local, flags, tw, lds);  \
