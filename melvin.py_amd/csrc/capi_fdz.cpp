@@ -17,14 +17,6 @@ using namespace mlv::abi;
 
 namespace {
 
-// Row kernel variant of a job with wpr wavefronts per row and K elements
-// per thread: the smallest compiled size >= K of that wpr.
-int fdz_variant(int K, int wpr) {
-  for (int v = 0; v < kFdzVariants; ++v)
-    if (kFdzWprs[v] == wpr && kFdzKts[v] >= K) return v;
-  return -1;
-}
-
 struct FdzHost {
   int dtype = 0, njobs = 0, device = 0, nphase = 1;
   void* jobs_dev = nullptr;
@@ -109,7 +101,6 @@ int build_fdz_job(const mlv_fdz_job_desc& d, FdzJob<T>& J, int j) {
   J.nn = (d.nx - 1) / 3;
   J.wpr = fdz_wpr(d.nz);
   J.K = (d.nz + 64 * J.wpr - 1) / (64 * J.wpr);
-  J.kt = kFdzKts[fdz_variant(J.K, J.wpr)];
   J.fd_order = d.fd_order;
   J.scheme = d.scheme;
   J.q = d.ab_order;
@@ -172,14 +163,18 @@ int create_impl(FdzHost* b, const mlv_fdz_job_desc* jobs, int njobs) {
   const int dtype = b->dtype;
   b->host.assign(sizeof(FdzJob<T>) * njobs, 0);
   const size_t lds_max = max_lds_per_block(b->device);
-  std::vector<int> prow[3][kFdzVariants], pcol[2];
-  for (int p = 0; p < 3; ++p)
-    for (int v = 0; v < kFdzVariants; ++v) prow[p][v].assign(njobs + 1, 0);
+  std::vector<int> prow[3], pcol[2];
+  for (int p = 0; p < 3; ++p) prow[p].assign(njobs + 1, 0);
   for (int p = 0; p < 2; ++p) pcol[p].assign(njobs + 1, 0);
   FdzLaunch& fl = b->fl;
   std::memset(&fl, 0, sizeof(fl));
   fl.njobs = njobs;
-  int zmax = 0;
+  {
+    const void* tw64 = nullptr;
+    const int rc = get_twiddles(b->device, MLV_F64, &tw64);
+    if (rc) return rc;
+    fl.tw64 = static_cast<const double2*>(tw64);
+  }
   for (int j = 0; j < njobs; ++j) {
     FdzJob<T>& J = host_job<T>(b, j);
     int rc = build_fdz_job<T>(jobs[j], J, j);
@@ -189,10 +184,11 @@ int create_impl(FdzHost* b, const mlv_fdz_job_desc* jobs, int njobs) {
     if (tc < 1 || ldsc > lds_max)
       return fail(MLV_ERR_UNSUPPORTED, "job " + std::to_string(j) + ": nx too large for LDS");
     fl.ldscol = std::max(fl.ldscol, ldsc);
-    zmax = std::max(zmax, J.nz);
+    // two LDS rows (buf, vrow) per row of a block, odd strides: the rows
+    // start on different banks
+    fl.ldsrow = std::max(fl.ldsrow, (size_t)fdz_rows_per_block(J.wpr) * 2 * (J.nz | 1) * sizeof(double2));
     const int nph = J.scheme == MLV_FDZ_PC ? 2 : 1;
     b->nphase = std::max(b->nphase, nph);
-    const int var = fdz_variant(J.K, J.wpr);
     const int cb = (J.nz + tc - 1) / tc;
     const int rpb = fdz_rows_per_block(J.wpr);
     const int rb2 = (2 * J.nn + rpb - 1) / rpb;
@@ -202,16 +198,10 @@ int create_impl(FdzHost* b, const mlv_fdz_job_desc* jobs, int njobs) {
     b->max_nn = std::max(b->max_nn, J.nn);
     for (int p = 0; p < 3; ++p) {
       const int nb = p == 2 ? rb1 : (p < nph ? rb2 : 0);
-      for (int v = 0; v < kFdzVariants; ++v) prow[p][v][j + 1] = prow[p][v][j] + (v == var ? nb : 0);
+      prow[p][j + 1] = prow[p][j] + nb;
     }
   }
-  fl.zstride = zmax | 1;  // odd stride: the waves' rows start on different banks
-  // two LDS rows (buf, vrow) per row of a block
-  for (int v = 0; v < kFdzVariants; ++v) {
-    fl.ldsrow[v] = (size_t)fdz_rows_per_block(kFdzWprs[v]) * 2 * fl.zstride * sizeof(double2);
-    if (fl.ldsrow[v] > lds_max)
-      return fail(MLV_ERR_UNSUPPORTED, "nz too large for the row kernel LDS");
-  }
+  if (fl.ldsrow > lds_max) return fail(MLV_ERR_UNSUPPORTED, "nz too large for the row kernel LDS");
   auto dalloc = [&](size_t bytes, void** p) -> int {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc fdz batch");
@@ -253,13 +243,11 @@ int create_impl(FdzHost* b, const mlv_fdz_job_desc* jobs, int njobs) {
     int r = upload(pcol[p], &fl.prefcol[p]);
     if (r) return r;
   }
-  for (int p = 0; p < 3; ++p)
-    for (int v = 0; v < kFdzVariants; ++v) {
-      fl.nrow[p][v] = prow[p][v][njobs];
-      if (fl.nrow[p][v] == 0) continue;
-      int r = upload(prow[p][v], &fl.prefrow[p][v]);
-      if (r) return r;
-    }
+  for (int p = 0; p < 3; ++p) {
+    fl.nrow[p] = prow[p][njobs];
+    int r = upload(prow[p], &fl.prefrow[p]);
+    if (r) return r;
+  }
   int r = MLV_OK;
   r = dalloc(b->host.size(), &b->jobs_dev);
   if (r) return r;

@@ -1,6 +1,7 @@
 // Fused Fourier-x / FD-z step kernels over a job table (see fdz.hpp).
 #include <math.h>
 
+#include "affine_scan.hpp"
 #include "diag_dev.hpp"
 #include "fdz.hpp"
 #include "grid.hpp"
@@ -20,19 +21,19 @@ __device__ __forceinline__ cx<T> t2(double2 v) {
 // Tridiagonal solve of one row by its WPR wavefronts, FP64.
 //
 // The system has identity first and last rows and constant interior bands
-// (lower = upper = lo).  fac holds, for element j, (cp_j, 1/den_j) of the
-// Thomas factorisation, stored chunk-major: entry i * LR + t is element
-// j = t K + i, LR = 64 WPR threads per row.  Thread t owns elements
-// [t K, t K + K).
+// (lower = upper = lo).  fc holds, for the thread's element i -- element t K
+// + i of the row -- (cp, 1/den) of the Thomas factorisation, read by
+// row_factors from the chunk-major tables (entry i * LR + t, LR = 64 WPR
+// threads per row).
 //   forward   d_j = (r_j - lower_j d_{j-1}) / den_j
 //   backward  x_j = d_j - cp_j x_{j+1},  x_{nz-1} = d_{nz-1}
 // Each recurrence is an affine map per element; a thread composes the maps
-// of its chunk, an inclusive shuffle scan composes them across a
-// wavefront's lanes, and the thread then replays its chunk from the value
-// entering it.  With two wavefronts per row the value leaving the first
-// wavefront's last element (forward) or entering the second's first
-// element (backward) goes through xch (4 doubles of LDS) between them.
-// buf holds the right-hand side on entry and the solution on exit.
+// of its chunk, a scan composes them across the lanes (affine_scan.hpp: DPP;
+// with shuffles the row kernel took 21.4 us at 1024x513 FP32 predictor-
+// corrector, 20.1 now; eight such jobs 77.9, now 75.9) and, through tot,
+// across the wavefronts, and the thread then replays its chunk from the value
+// entering it.  buf holds the right-hand side on entry and the solution on
+// exit.
 // --------------------------------------------------------------------------
 template <int WPR>
 __device__ __forceinline__ void row_sync() {
@@ -43,130 +44,78 @@ __device__ __forceinline__ void row_sync() {
 }
 
 template <int KT, int WPR>
-__device__ __forceinline__ void row_tridiag(double2* __restrict__ buf,
-                                            gptr<const double2> fac, double lo, int nz, int K,
-                                            int t, double* __restrict__ xch) {
-  static_assert(WPR == 1 || WPR == 2, "one or two wavefronts per row");
-  constexpr int LR = 64 * WPR;
-  const int lane = t & 63, wv = t >> 6;
-  const int j0 = t * K;
-  double2 d[KT], fc[KT];
+__device__ __forceinline__ void row_factors(double2 (&fc)[KT], gptr<const double2> fac, int K,
+                                            int t) {
 #pragma unroll
   for (int i = 0; i < KT; ++i) {
-    const int j = j0 + i;
-    const bool ok = i < K && j < nz;
     fc[i] = make_double2(0.0, 1.0);
+    if (i < K) fc[i] = fac[i * (64 * WPR) + t];
+  }
+}
+
+// The value entering a thread's chunk: the wavefronts' maps before its own,
+// then the lanes' before its own (BACK: after it).
+template <int WPR, bool BACK>
+__device__ __forceinline__ double2 row_scan(const Affine& m, Affine* __restrict__ tot, int t) {
+  Affine all;
+  const Affine e = wave_affine_scan<BACK>(m, all);
+  double px = 0.0, py = 0.0;
+  if constexpr (WPR > 1) {
+    const int wv = t >> 6;
+    if ((t & 63) == 0) tot[wv] = all;
+    __syncthreads();
+    auto step = [&](int w) {
+      px = fma(tot[w].a, px, tot[w].x);
+      py = fma(tot[w].a, py, tot[w].y);
+    };
+    if constexpr (BACK)
+      for (int w = WPR - 1; w > wv; --w) step(w);
+    else
+      for (int w = 0; w < wv; ++w) step(w);
+  }
+  return make_double2(fma(e.a, px, e.x), fma(e.a, py, e.y));
+}
+
+template <int KT, int WPR>
+__device__ __forceinline__ void row_tridiag(double2* __restrict__ buf, const double2 (&fc)[KT],
+                                            double lo, int nz, int K, int t,
+                                            Affine* __restrict__ tot) {
+  const int j0 = t * K;
+  double2 d[KT];
+  Affine m = {1.0, 0.0, 0.0};
+#pragma unroll
+  for (int i = 0; i < KT; ++i) {
+    const int j = j0 + i;
     d[i] = make_double2(0.0, 0.0);
-    if (ok) {
-      fc[i] = fac[i * LR + t];
+    if (i < K && j < nz) {
       d[i] = buf[j];
+      const double l = (j == 0 || j == nz - 1) ? 0.0 : lo;
+      m = aff_after(Affine{-l * fc[i].y, d[i].x * fc[i].y, d[i].y * fc[i].y}, m);
     }
   }
-  // forward elimination
-  double A = 1.0, Bx = 0.0, By = 0.0;
+  double2 p = row_scan<WPR, false>(m, tot, t);
+  m = {1.0, 0.0, 0.0};
 #pragma unroll
   for (int i = 0; i < KT; ++i) {
     const int j = j0 + i;
     if (i < K && j < nz) {
       const double l = (j == 0 || j == nz - 1) ? 0.0 : lo;
-      const double m = -l * fc[i].y;
-      A = m * A;
-      Bx = m * Bx + d[i].x * fc[i].y;
-      By = m * By + d[i].y * fc[i].y;
+      p.x = d[i].x = (d[i].x - l * p.x) * fc[i].y;
+      p.y = d[i].y = (d[i].y - l * p.y) * fc[i].y;
     }
   }
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const double Ao = __shfl_up(A, off, 64);
-    const double Xo = __shfl_up(Bx, off, 64);
-    const double Yo = __shfl_up(By, off, 64);
-    if (lane >= off) {
-      Bx = A * Xo + Bx;
-      By = A * Yo + By;
-      A = A * Ao;
-    }
-  }
-  double px = __shfl_up(Bx, 1, 64), py = __shfl_up(By, 1, 64);
-  if (lane == 0) px = py = 0.0;
-  if constexpr (WPR == 2) {
-    // the second wavefront's lanes continue from the first's last value
-    double ax = __shfl_up(A, 1, 64);
-    if (lane == 0) ax = 1.0;
-    if (t == 63) {
-      xch[0] = Bx;
-      xch[1] = By;
-    }
-    __syncthreads();
-    if (wv == 1) {
-      px = ax * xch[0] + px;
-      py = ax * xch[1] + py;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < KT; ++i) {
-    const int j = j0 + i;
-    if (i < K && j < nz) {
-      const double l = (j == 0 || j == nz - 1) ? 0.0 : lo;
-      d[i].x = (d[i].x - l * px) * fc[i].y;
-      d[i].y = (d[i].y - l * py) * fc[i].y;
-      px = d[i].x;
-      py = d[i].y;
-    }
-  }
-  // back substitution
-  A = 1.0;
-  Bx = 0.0;
-  By = 0.0;
+  for (int i = KT - 1; i >= 0; --i)
+    if (i < K && j0 + i < nz) m = aff_after(Affine{-fc[i].x, d[i].x, d[i].y}, m);
+  p = row_scan<WPR, true>(m, tot + WPR, t);
 #pragma unroll
   for (int i = KT - 1; i >= 0; --i) {
     const int j = j0 + i;
     if (i < K && j < nz) {
-      const double c = fc[i].x;
-      A = -c * A;
-      Bx = d[i].x - c * Bx;
-      By = d[i].y - c * By;
+      p.x = d[i].x - fc[i].x * p.x;
+      p.y = d[i].y - fc[i].x * p.y;
+      buf[j] = p;
     }
-  }
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const double Ao = __shfl_down(A, off, 64);
-    const double Xo = __shfl_down(Bx, off, 64);
-    const double Yo = __shfl_down(By, off, 64);
-    if (lane + off < 64) {
-      Bx = A * Xo + Bx;
-      By = A * Yo + By;
-      A = A * Ao;
-    }
-  }
-  double xx = __shfl_down(Bx, 1, 64), xy = __shfl_down(By, 1, 64);
-  if (lane == 63) xx = xy = 0.0;
-  if constexpr (WPR == 2) {
-    // the first wavefront's lanes continue from the second's first value
-    double ax = __shfl_down(A, 1, 64);
-    if (lane == 63) ax = 1.0;
-    if (t == 64) {
-      xch[2] = Bx;
-      xch[3] = By;
-    }
-    __syncthreads();
-    if (wv == 0) {
-      xx = ax * xch[2] + xx;
-      xy = ax * xch[3] + xy;
-    }
-  }
-#pragma unroll
-  for (int i = KT - 1; i >= 0; --i) {
-    const int j = j0 + i;
-    if (i < K && j < nz) {
-      xx = d[i].x - fc[i].x * xx;
-      xy = d[i].y - fc[i].x * xy;
-      d[i] = make_double2(xx, xy);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < KT; ++i) {
-    const int j = j0 + i;
-    if (i < K && j < nz) buf[j] = d[i];
   }
 }
 
@@ -209,7 +158,8 @@ __device__ __forceinline__ double2 d2dz2_row(const double2* __restrict__ b, int 
 template <typename T, int KT, int WPR>
 __device__ __forceinline__ void fdz_row(const FdzJob<T>& J, int stage, int n, int f, int step,
                                         double2* __restrict__ buf, double2* __restrict__ vrow,
-                                        int t, double* __restrict__ xch) {
+                                        int t, Affine* __restrict__ tot,
+                                        const double2* __restrict__ tw64) {
   constexpr int LR = 64 * WPR;  // threads per row
   const int Z = J.nz, K = J.K;
   const int par = (J.par0 + step) & 1;
@@ -221,10 +171,16 @@ __device__ __forceinline__ void fdz_row(const FdzJob<T>& J, int stage, int n, in
   if (stage != FDZ_PROLOGUE) {
     const int q = J.q;
     const int cur = ring(J.curr0, step, q);
+    const bool expl = J.scheme == MLV_FDZ_EXPLICIT;
+    const int ws = stage == FDZ_CORR ? (cur + 1) % q : cur;  // ring slot written
+    const int s1 = (ws + q - 1) % q, s2 = (ws + q - 2) % q, s3 = (ws + q - 3) % q;
+    const size_t ssz = (size_t)J.nn * Z;
+    cx<T>* __restrict__ hist = glb(J.hist[f]);
     const cx<T>* __restrict__ qx = glb(J.qw[2 * f]) + row;
     const cx<T>* __restrict__ qz = glb(J.qw[2 * f + 1]) + row;
     const cx<T>* __restrict__ vin = glb(J.state[par][f]) + row;
     const cx<T>* __restrict__ cin = J.comp[f] ? glb(J.comp[f]) + row : nullptr;
+    const cx<T>* __restrict__ tsrc = glb(stage == FDZ_CORR ? J.star[1] : J.state[par][1]) + row;
 #pragma unroll
     for (int i = 0; i < KT; ++i) {
       const int j = t + LR * i;
@@ -239,23 +195,18 @@ __device__ __forceinline__ void fdz_row(const FdzJob<T>& J, int stage, int n, in
         vrow[j] = v;
       }
     }
-    row_sync<WPR>();
-    double sx;
+    double sx;  // modified wavenumber of the x difference, sin(2 pi n / nx) from the table
     {
-      const double th = 2.0 * M_PI * (double)n / (double)J.nx;
-      sx = order == 2 ? sin(th) / J.dx : (8.0 * sin(th) - sin(2.0 * th)) / (6.0 * J.dx);
+      const int sh = LOG_NMAX - J.lognx;
+      const double s1x = -tw64[n << sh].y;
+      sx = order == 2 ? s1x / J.dx : (8.0 * s1x + tw64[(2 * n) << sh].y) / (6.0 * J.dx);
     }
+    row_sync<WPR>();
     // -Pr Ra i (2 pi n / lx) T  (rayleigh_benard_convection.py:101-104)
     const double buoy = f == 0 ? J.Pr * J.Ra * (J.fx * (double)n) : 0.0;
-    const cx<T>* __restrict__ tsrc = glb(stage == FDZ_CORR ? J.star[1] : J.state[par][1]) + row;
     const double coeff = f == 0 ? J.Pr : 1.0;
     const double k2 = J.fx2 * (double)n * (double)n;  // -(2 pi n / lx)^2
     const double idz2 = 1.0 / (dz * dz);
-    const bool expl = J.scheme == MLV_FDZ_EXPLICIT;
-    const int ws = stage == FDZ_CORR ? (cur + 1) % q : cur;  // ring slot written
-    const int s1 = (ws + q - 1) % q, s2 = (ws + q - 2) % q, s3 = (ws + q - 3) % q;
-    const size_t ssz = (size_t)J.nn * Z;
-    cx<T>* __restrict__ hist = glb(J.hist[f]);
     const double dt = J.dt;
     double2 inc[KT];
 #pragma unroll
@@ -320,9 +271,10 @@ __device__ __forceinline__ void fdz_row(const FdzJob<T>& J, int stage, int n, in
     if (!expl) {
       // increment form of the theta scheme:
       //   (I - a dt c L) delta = dt c L v + E,  v_new = v + delta
+      double2 fd[KT];
+      row_factors<KT, WPR>(fd, glb(J.fac[1 + f]) + (size_t)n * K * LR, K, t);
       row_sync<WPR>();
-      row_tridiag<KT, WPR>(buf, glb(J.fac[1 + f]) + (size_t)n * K * LR, J.lo[1 + f], Z, K,
-                           t, xch);
+      row_tridiag<KT, WPR>(buf, fd, J.lo[1 + f], Z, K, t, tot);
     }
     row_sync<WPR>();
     // new state and wall writes (rayleigh_benard_convection.py:113-142);
@@ -374,8 +326,10 @@ __device__ __forceinline__ void fdz_row(const FdzJob<T>& J, int stage, int n, in
   if (f != 0) return;
   // psi = solve(-omega) (utility.py:65, LaplacianSolver.py:70-78),
   // ux_s = -pddz(psi), uz_s = i kx psi (utility.py:66-79)
+  double2 fp[KT];
+  row_factors<KT, WPR>(fp, glb(J.fac[0]) + (size_t)n * K * LR, K, t);
   row_sync<WPR>();
-  row_tridiag<KT, WPR>(buf, glb(J.fac[0]) + (size_t)n * K * LR, J.lo[0], Z, K, t, xch);
+  row_tridiag<KT, WPR>(buf, fp, J.lo[0], Z, K, t, tot + 2 * WPR);
   row_sync<WPR>();
   const int vs = stage == FDZ_PRED ? 2 : (stage == FDZ_PROLOGUE ? par : par ^ 1);
   cx<T>* __restrict__ ux = glb(J.vel[vs][0]) + row;
@@ -395,20 +349,27 @@ __device__ __forceinline__ void fdz_row(const FdzJob<T>& J, int stage, int n, in
   }
 }
 
-// Blocks of fdz_rows_per_block(WPR) rows of WPR wavefronts each.
-template <typename T, int KT, int WPR>
-__global__ void __launch_bounds__(fdz_row_threads(WPR))
+// Blocks of 128 threads: two rows of one wavefront, or one row of two.  One
+// launch runs every job's rows, each wavefront taking the branch of its job's
+// K.  (A launch per K left a batch of ragged sizes with up to five launches
+// that each filled a fraction of the chip: six FP64 jobs of nz 33 to 257 took
+// 39.6 us of row kernels per step, 14.4 in one launch.  The kernel holds 124
+// VGPRs: reading all operands and factors up front costs 149 and a wavefront
+// per SIMD, 81.8 against 75.9 us for eight jobs of 1024x513, with no gain for
+// one.)
+template <typename T>
+__global__ void __launch_bounds__(kFdzRowThreads)
     k_fdz_rows(const FdzJob<T>* __restrict__ jobs, FdzJob<T>* clock, const int* __restrict__ pref,
-               int njobs, int phase, int step, int zstride) {
+               int njobs, int phase, int step, const double2* __restrict__ tw64) {
   extern __shared__ char smem_raw[];
-  __shared__ double xch[4];
+  __shared__ Affine tot[2 * 2 * 2];  // two solves, two directions, two wavefronts
   const int lb = xcd_logical(pref[njobs]);
   if (lb < 0) return;
   const int jb = find_job(pref, njobs, lb);
   const FdzJob<T>& J = jobs[jb];
-  constexpr int LR = 64 * WPR;
-  const int rib = threadIdx.x / LR, t = threadIdx.x % LR;  // row in block, thread in row
-  const int lw = (lb - pref[jb]) * fdz_rows_per_block(WPR) + rib;
+  const int wpr = J.wpr, lr = 64 * wpr;
+  const int rib = threadIdx.x / lr, t = threadIdx.x % lr;  // row in block, thread in row
+  const int lw = (lb - pref[jb]) * fdz_rows_per_block(wpr) + rib;
   int stage, nwf;
   if (phase < 0) {
     stage = FDZ_PROLOGUE;
@@ -424,11 +385,26 @@ __global__ void __launch_bounds__(fdz_row_threads(WPR))
     clock[jb].t = clock[jb].t + J.dt;
     clock[jb].loops = clock[jb].loops + 1;
   }
-  // (uniform over a block when WPR > 1: the block is one row)
-  if (lw >= nwf * J.nn || J.kt != KT || J.wpr != WPR) return;
-  const int n = lw / nwf, f = lw % nwf;
+  // (uniform over a block when wpr > 1: the block is one row)
+  if (lw >= nwf * J.nn) return;
+  const int n = lw / nwf, f = lw % nwf, zstride = J.nz | 1;
   double2* buf = reinterpret_cast<double2*>(smem_raw) + (size_t)(2 * rib) * zstride;
-  fdz_row<T, KT, WPR>(J, stage, n, f, step, buf, buf + zstride, t, xch);
+  double2* vrow = buf + zstride;
+#define MLV_ROW(KT, WPR) fdz_row<T, KT, WPR>(J, stage, n, f, step, buf, vrow, t, tot, tw64)
+  if (wpr == 1) {
+    if (J.K <= 1)
+      MLV_ROW(1, 1);
+    else if (J.K <= 2)
+      MLV_ROW(2, 1);
+    else
+      MLV_ROW(4, 1);
+  } else {
+    if (J.K <= 4)
+      MLV_ROW(4, 2);
+    else
+      MLV_ROW(6, 2);
+  }
+#undef MLV_ROW
 }
 
 // --------------------------------------------------------------------------
@@ -743,27 +719,15 @@ __global__ void k_fdz_set_dt(FdzJob<T>* jobs, int j, double dt, double lo_w, dou
 // --------------------------------------------------------------------------
 // Host side
 // --------------------------------------------------------------------------
-template <typename T, int V>
-static void launch_rows(const FdzJob<T>* jobs, const FdzLaunch& fl, const int* pref, int nblocks,
-                        int phase, int step, hipStream_t s) {
-  if (nblocks <= 0) return;
-  constexpr int KT = kFdzKts[V], WPR = kFdzWprs[V];
-  MLV_SET_LDS_ONCE((k_fdz_rows<T, KT, WPR>), fl.ldsrow[V]);
-  hipLaunchKernelGGL((k_fdz_rows<T, KT, WPR>), dim3(xcd_grid(nblocks)), dim3(fdz_row_threads(WPR)),
-                     fl.ldsrow[V], s, jobs, const_cast<FdzJob<T>*>(jobs), pref, fl.njobs, phase,
-                     step, fl.zstride);
-}
-
 template <typename T>
-static void launch_rows_all(const FdzJob<T>* jobs, const FdzLaunch& fl, int phase, int step,
-                            hipStream_t s) {
+static void launch_rows(const FdzJob<T>* jobs, const FdzLaunch& fl, int phase, int step,
+                        hipStream_t s) {
   const int p = phase < 0 ? 2 : phase;
-  launch_rows<T, 0>(jobs, fl, fl.prefrow[p][0], fl.nrow[p][0], phase, step, s);
-  launch_rows<T, 1>(jobs, fl, fl.prefrow[p][1], fl.nrow[p][1], phase, step, s);
-  launch_rows<T, 2>(jobs, fl, fl.prefrow[p][2], fl.nrow[p][2], phase, step, s);
-  launch_rows<T, 3>(jobs, fl, fl.prefrow[p][3], fl.nrow[p][3], phase, step, s);
-  launch_rows<T, 4>(jobs, fl, fl.prefrow[p][4], fl.nrow[p][4], phase, step, s);
-  static_assert(kFdzVariants == 5, "row kernel variants");
+  if (fl.nrow[p] <= 0) return;
+  MLV_SET_LDS_ONCE(k_fdz_rows<T>, fl.ldsrow);
+  hipLaunchKernelGGL(k_fdz_rows<T>, dim3(xcd_grid(fl.nrow[p])), dim3(kFdzRowThreads), fl.ldsrow, s,
+                     jobs, const_cast<FdzJob<T>*>(jobs), (const int*)fl.prefrow[p], fl.njobs,
+                     phase, step, fl.tw64);
 }
 
 template <typename T>
@@ -776,14 +740,14 @@ hipError_t fdz_phase(const FdzJob<T>* jobs, const FdzLaunch& fl, int phase, int 
                        jobs, (const int*)fl.prefcol[phase], fl.njobs, phase, flags, step, tw);
   }
   if (ev) (void)hipEventRecord(ev[1], s);
-  launch_rows_all<T>(jobs, fl, phase, step, s);
+  launch_rows<T>(jobs, fl, phase, step, s);
   if (ev) (void)hipEventRecord(ev[2], s);
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t fdz_prologue(const FdzJob<T>* jobs, const FdzLaunch& fl, int step, hipStream_t s) {
-  launch_rows_all<T>(jobs, fl, -1, step, s);
+  launch_rows<T>(jobs, fl, -1, step, s);
   return hipGetLastError();
 }
 
@@ -805,7 +769,7 @@ template <typename T>
 hipError_t fdz_diag(FdzJob<T>* jobs, int njobs, int max_nn, double cutoff, int cadence,
                     hipStream_t s) {
   hipLaunchKernelGGL(k_fdz_diag<T>, dim3(njobs), dim3(kNT), 0, s, jobs, cutoff, cadence);
-  hipLaunchKernelGGL(k_fdz_refactor<T>, dim3(max_nn, njobs, 2), dim3(128), 0, s,
+  hipLaunchKernelGGL(k_fdz_refactor<T>, dim3(max_nn, njobs, 2), dim3(kFdzRowThreads), 0, s,
                      (const FdzJob<T>*)jobs);
   return hipGetLastError();
 }
@@ -813,10 +777,7 @@ hipError_t fdz_diag(FdzJob<T>* jobs, int njobs, int max_nn, double cutoff, int c
 template <typename T>
 hipError_t fdz_prepare(const FdzLaunch& fl) {
   if (fl.ldscol) MLV_SET_LDS_ONCE(k_fdz_cols<T>, fl.ldscol);
-#define MLV_ROWS_LDS(V) \
-  if (fl.ldsrow[V]) MLV_SET_LDS_ONCE((k_fdz_rows<T, kFdzKts[V], kFdzWprs[V]>), fl.ldsrow[V]);
-  MLV_ROWS_LDS(0) MLV_ROWS_LDS(1) MLV_ROWS_LDS(2) MLV_ROWS_LDS(3) MLV_ROWS_LDS(4)
-#undef MLV_ROWS_LDS
+  MLV_SET_LDS_ONCE(k_fdz_rows<T>, fl.ldsrow);
   return hipGetLastError();
 }
 

@@ -9,7 +9,7 @@
 //         (ux_s + i uz_s) and (omega + i T), the four products ux*f, uz*f
 //         in physical space, two packed forward x transforms, keep
 //         kx < nn, scale 1/nx  ->  Qx_f, Qz_f.
-//   rows  one wavefront per (x mode, field): the flux divergence
+//   rows  one or two wavefronts per (x mode, field): the flux divergence
 //         D = i sx(kx) Qx + Dz(Qz) (the periodic x difference is its exact
 //         modified wavenumber; the z difference acts along the row, and both
 //         commute with the x transform), buoyancy -Pr Ra i kx T for omega,
@@ -24,9 +24,9 @@
 // Schemes: EXPLICIT and SEMI_IMPLICIT run one phase per step; PC runs two
 // (AB predictor into a scratch state, AM corrector from the old state).
 // The tridiagonal solves run in FP64 whatever the state precision: each
-// lane of the wave owns a contiguous chunk of the row, Thomas's two
-// first-order recurrences are composed into affine maps per chunk and
-// scanned across the 64 lanes with shuffles.
+// lane owns a contiguous chunk of the row, Thomas's two first-order
+// recurrences are composed into affine maps per chunk and scanned across
+// the lanes.
 #pragma once
 #include <hip/hip_runtime.h>
 #include "../../include/melvin_hip.h"
@@ -36,29 +36,22 @@
 namespace mlv {
 
 enum FdzStage : int { FDZ_MAIN = 0, FDZ_PRED = 1, FDZ_CORR = 2, FDZ_PROLOGUE = 3 };
-constexpr int kFdzWaves = 4;   // rows (mode, field) per row block of one wavefront per row
-// Row kernel variants: KT row elements per thread and WPR wavefronts per
-// row.  A row of nz <= 256 points takes one wavefront (K = ceil(nz / 64)
-// elements per lane, blocks of kFdzWaves rows); a longer row takes two
-// (K = ceil(nz / 128), a block per row), which halves each wavefront's
-// serial chain of instructions -- a single job has fewer rows than the
-// device has SIMDs, so that chain sets the kernel's time.  The choice
-// depends on the job alone, so a job computes the same bits in any batch.
-// A job runs in the smallest variant of its WPR with KT >= its K.
-constexpr int kFdzVariants = 5;
-constexpr int kFdzKts[kFdzVariants] = {1, 2, 4, 4, 6};
-constexpr int kFdzWprs[kFdzVariants] = {1, 1, 1, 2, 2};
+// Row blocks of 128 threads.  A row of nz <= 256 points takes one wavefront
+// (K = ceil(nz / 64) elements per lane, two rows per block); a longer row
+// takes two (K = ceil(nz / 128), a block per row), which halves each
+// wavefront's serial chain of instructions -- a single job has fewer rows
+// than the device has SIMDs, so that chain sets the kernel's time.  (Four
+// wavefronts per row gained nothing for one 1024x513 FP32 job and took 23.4
+// us instead of 20.5 for an FP64 one.)  The choice depends on the job alone,
+// so a job computes the same bits in any batch.
+constexpr int kFdzRowThreads = 128;
 constexpr int kFdzMaxNz = 768;
 __host__ __device__ constexpr int fdz_wpr(int nz) { return nz > 256 ? 2 : 1; }
-// rows per block and threads per block of a variant with wpr wavefronts per row
-__host__ __device__ constexpr int fdz_rows_per_block(int wpr) { return wpr == 1 ? kFdzWaves : 1; }
-__host__ __device__ constexpr int fdz_row_threads(int wpr) {
-  return 64 * wpr * fdz_rows_per_block(wpr);
-}
+__host__ __device__ constexpr int fdz_rows_per_block(int wpr) { return 2 / wpr; }
 
 template <typename T>
 struct FdzJob {
-  int nx, nz, lognx, nn, K, kt, wpr, fd_order, scheme, q, curr0, par0;
+  int nx, nz, lognx, nn, K, wpr, fd_order, scheme, q, curr0, par0;
   double fx, fx2, dx, dz, dt, alpha, Pr, Ra;
   double lo[3];            // interior off-diagonal of each tridiagonal operator
   cx<T>* state[2][2];      // [buffer][omega, T]
@@ -89,11 +82,11 @@ constexpr int kFdzWritePhys = 1, kFdzDiag = 2, kFdzDiagShift = 8;
 struct FdzLaunch {
   int njobs;
   int ncol[2];                       // column blocks of phases 0 and 1
-  int nrow[3][kFdzVariants];         // row blocks of phases 0, 1 and the prologue
-  size_t ldsrow[kFdzVariants], ldscol;  // LDS of each row variant's blocks
-  int zstride;                       // LDS elements per row of the row kernel
+  int nrow[3];                       // row blocks of phases 0, 1 and the prologue
+  size_t ldsrow, ldscol;
+  const double2* tw64;               // FP64 twiddles exp(-2 pi i k / NMAX)
   int *prefcol[2];
-  int *prefrow[3][kFdzVariants];
+  int *prefrow[3];
 };
 
 // Points per thread of the column kernel: 16 below N = 2048 (two columns
