@@ -54,8 +54,9 @@ class Integrator:
     def set_dt(self, ux, uz):
         """Sets dt based on the CFL limit (signed maxima, as the reference)."""
         with np.errstate(divide="ignore", invalid="ignore"):
-            cfl_dt = min(np.float64(self._dx) / np.float64(hip.max(ux.getp())),
-                         np.float64(self._dz) / np.float64(hip.max(uz.getp())))
+            ux_max, uz_max = hip.max_pair(ux.getp(), uz.getp())
+            cfl_dt = min(np.float64(self._dx) / np.float64(ux_max),
+                         np.float64(self._dz) / np.float64(uz_max))
         if self._dt > cfl_dt or np.isnan(cfl_dt):
             raise Exception("CFL condition breached")
         while self._dt > self._cfl_cutoff * cfl_dt:

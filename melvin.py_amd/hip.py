@@ -34,7 +34,8 @@ _TORCH = {
 
 
 def device():
-    if not torch.cuda.is_available():
+    # (is_available counts the devices again: 1 us of an operator call)
+    if not (torch.cuda.is_initialized() or torch.cuda.is_available()):
         raise _lib.MelvinHipError("melvin_amd.hip needs a GPU (no CPU fallback)")
     return torch.device("cuda", torch.cuda.current_device())
 
@@ -93,7 +94,7 @@ def asnumpy(a):
     return np.asarray(a)
 
 
-def _reduce(op, a, b=None, scale=1.0):
+def _reduce(op, a, b=None, scale=1.0, out=None):
     a = asarray(a).contiguous()
     if a.dtype == torch.float64:
         dt = _lib.F64
@@ -105,7 +106,8 @@ def _reduce(op, a, b=None, scale=1.0):
         b = asarray(b).contiguous()
         if b.dtype != a.dtype or b.shape != a.shape:
             raise ValueError("reduction operands differ in dtype or shape")
-    out = torch.empty(1, dtype=torch.float64, device=a.device)
+    if out is None:
+        out = torch.empty(1, dtype=torch.float64, device=a.device)
     _lib.call("mlv_reduce", None, op, dt, ctypes.c_void_p(a.data_ptr()),
               ctypes.c_void_p(0 if b is None else b.data_ptr()), a.numel(),
               float(scale), ctypes.c_void_p(out.data_ptr()), _lib.stream_handle())
@@ -115,6 +117,15 @@ def _reduce(op, a, b=None, scale=1.0):
 def max(a):  # noqa: A001
     """Signed maximum (NaN-propagating), FP64, as a Python float."""
     return float(_reduce(_lib.RED_MAX, a).item())
+
+
+def max_pair(a, b):
+    """(max(a), max(b)) read back together: one wait instead of two."""
+    a, b = asarray(a), asarray(b)
+    out = torch.empty(2, dtype=torch.float64, device=a.device)
+    _reduce(_lib.RED_MAX, a, out=out)
+    _reduce(_lib.RED_MAX, b, out=out[1:])
+    return tuple(out.tolist())
 
 
 def sum(a):  # noqa: A001
