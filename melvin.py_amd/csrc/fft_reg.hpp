@@ -42,6 +42,28 @@ template <int LOGE>
 __host__ __device__ constexpr int rf_pad(int i) {
   return i + (i >> LOGE);
 }
+// Position of point t + d, d a constant once unrolled.  A multiple of E moves
+// the position by a constant, which becomes the access's immediate offset;
+// as rf_pad(t + d) the compiler keeps a register per point (the 1024-point
+// FP32 column pass of the FD-z step: 171 VGPRs, 126 so).
+template <int LOGE>
+__host__ __device__ constexpr int rf_pad(int t, int d) {
+  return d % (1 << LOGE) == 0 ? rf_pad<LOGE>(t) + rf_pad<LOGE>(d) : rf_pad<LOGE>(t + d);
+}
+// Position of point -(t + m TPS) mod N, the mirror of a thread's point m.
+template <int LOGN, int LOGE>
+__host__ __device__ constexpr int rf_mirror(int t, int m) {
+  constexpr int N = 1 << LOGN, TPS = N >> LOGE;
+  return m == 0 && t == 0 ? 0 : rf_pad<LOGE>(TPS - t, N - (m + 1) * TPS);
+}
+// Position of the neighbour at distance |d| <= 2 of a thread's point m,
+// periodic.
+template <int LOGN, int LOGE>
+__host__ __device__ constexpr int rf_near(int t, int m, int d) {
+  constexpr int N = 1 << LOGN, TPS = N >> LOGE;
+  const bool inside = m * TPS >= 2 && (m + 1) * TPS + 2 <= N;
+  return inside ? rf_pad<LOGE>(t + d, m * TPS) : rf_pad<LOGE>((t + m * TPS + d) & (N - 1));
+}
 __host__ __device__ constexpr int rf_len(int logn, int loge) {
   return (1 << logn) + ((1 << logn) >> loge);
 }
@@ -61,8 +83,9 @@ __device__ __forceinline__ void rf_sync() {
 // the thread in the transform, NT the threads that synchronise together.
 // Before the call nobody still reads or writes the region; after it the last
 // reads of the region may be pending (rf_sync before writing it again).
+// IMM: positions at constant distances (two-argument rf_pad).
 template <typename T, int LOGN, int LOGE, int DIR, int STRIDE, int NT,
-          int LOGM = (LOGE < 4 ? LOGE : 4), int PASS = 0>
+          int LOGM = (LOGE < 4 ? LOGE : 4), bool IMM = true, int PASS = 0>
 __device__ __forceinline__ void rf_fft(cx<T> (&v)[1 << LOGE], cx<T>* __restrict__ lds, int t,
                                        const cx<T>* __restrict__ tw) {
   constexpr int N = 1 << LOGN, E = 1 << LOGE, TPS = N / E;
@@ -71,6 +94,7 @@ __device__ __forceinline__ void rf_fft(cx<T> (&v)[1 << LOGE], cx<T>* __restrict_
   constexpr int LOGNS = rf_logns(LOGN, LOGM, PASS), NS = 1 << LOGNS;
   constexpr int B = E / R;  // butterflies per thread
   constexpr bool LAST = PASS == rf_passes(LOGN, LOGM) - 1;
+  auto at = [](int i, int d) { return IMM ? rf_pad<LOGE>(i, d) : rf_pad<LOGE>(i + d); };
   cx<T> u[B][R];
 #pragma unroll
   for (int i = 0; i < B; ++i) {
@@ -101,12 +125,12 @@ __device__ __forceinline__ void rf_fft(cx<T> (&v)[1 << LOGE], cx<T>* __restrict_
       const int jm = j & (NS - 1);
       const int base = (j - jm) * R + jm;
 #pragma unroll
-      for (int r = 0; r < R; ++r) lds[rf_pad<LOGE>(base + r * NS) * STRIDE] = u[i][r];
+      for (int r = 0; r < R; ++r) lds[at(base, r * NS) * STRIDE] = u[i][r];
     }
     rf_sync<NT>();
 #pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = lds[rf_pad<LOGE>(t + m * TPS) * STRIDE];
-    rf_fft<T, LOGN, LOGE, DIR, STRIDE, NT, LOGM, PASS + 1>(v, lds, t, tw);
+    for (int m = 0; m < E; ++m) v[m] = lds[at(t, m * TPS) * STRIDE];
+    rf_fft<T, LOGN, LOGE, DIR, STRIDE, NT, LOGM, IMM, PASS + 1>(v, lds, t, tw);
   }
 }
 

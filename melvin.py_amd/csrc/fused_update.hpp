@@ -66,12 +66,11 @@ __device__ __forceinline__ void stepC_body(const JobDev<T>& J, const StageDev& S
   const T szc = modk<T>(tw, cok ? col : 0, J.lognz, order, J.dz);
   cx<T>* __restrict__ slot = lds + c;
 #pragma unroll
-  for (int m = 0; m < E; ++m) slot[rf_pad<LOGE>(t + m * TPS) * TC] = v[m];
+  for (int m = 0; m < E; ++m) slot[rf_pad<LOGE>(t, m * TPS) * TC] = v[m];
   rf_sync<NT>();
 #pragma unroll
   for (int m = 0; m < E; ++m) {
-    const int x = t + m * TPS;
-    auto at = [&](int d) { return slot[rf_pad<LOGE>((x + d) & (N - 1)) * TC]; };
+    auto at = [&](int d) { return slot[rf_near<LOGN, LOGE>(t, m, d) * TC]; };
     const cx<T> a1 = at(1), b1 = at(-1);
     cx<T> d;
     if (order == 2) {

@@ -132,7 +132,7 @@ __device__ __forceinline__ void stepZ_body(const JobDev<T>& J, const StageDev& S
     rf_fft<T, LOGN, LOGE, +1, 1, 64>(v, mine, t, tw);
     rf_sync<64>();
 #pragma unroll
-    for (int m = 0; m < E; ++m) mine[rf_pad<LOGE>(t + m * TPS)] = v[m];
+    for (int m = 0; m < E; ++m) mine[rf_pad<LOGE>(t, m * TPS)] = v[m];
   }
   __syncthreads();
   // this job's check loop (J.loops counts the loops before this one)
@@ -183,7 +183,7 @@ __device__ __forceinline__ void stepZ_body(const JobDev<T>& J, const StageDev& S
     const cx<T>* __restrict__ fst = region(o.first, sub);
 #pragma unroll
     for (int m = 0; m < E; ++m) {
-      const int i = rf_pad<LOGE>(t + m * TPS);
+      const int i = rf_pad<LOGE>(t, m * TPS);
       const cx<T> a = o.first == ch ? v[m] : fst[i], b = sec[i];
       const T px = a.x * b.x, py = a.y * b.y;
       if constexpr (mhd) {
@@ -201,7 +201,7 @@ __device__ __forceinline__ void stepZ_body(const JobDev<T>& J, const StageDev& S
   rf_sync<64>();
 #pragma unroll
   for (int m = 0; m < E; ++m)
-    if (z_any(m, TPS, N)) mine[rf_pad<LOGE>(t + m * TPS)] = v[m];
+    if (z_any(m, TPS, N)) mine[rf_pad<LOGE>(t, m * TPS)] = v[m];
   rf_sync<64>();
   const uint32_t obase = ((uint32_t)pchan(NIN, o.e, o.k) * chs + (uint32_t)x0 * kPGroup) * (uint32_t)sizeof(cx<T>);
 #pragma unroll
@@ -209,7 +209,7 @@ __device__ __forceinline__ void stepZ_body(const JobDev<T>& J, const StageDev& S
     if (m * TPS >= nm) continue;
     const int k = t + m * TPS;
     if (live && k < nm) {
-      const cx<T> y = mine[rf_pad<LOGE>(k)], ym = mine[rf_pad<LOGE>((N - k) & (N - 1))];
+      const cx<T> y = mine[rf_pad<LOGE>(t, m * TPS)], ym = mine[rf_mirror<LOGN, LOGE>(t, m)];
       const uint32_t at = obase + (uint32_t)pidx(0, k, nx) * (uint32_t)sizeof(cx<T>);
       at32(work, at) = mk<T>(T(0.5) * (y.x + ym.x), T(0.5) * (y.y - ym.y));
       at32(work, at + kPGroup * (uint32_t)sizeof(cx<T>)) = mk<T>(T(0.5) * (y.y + ym.y), T(0.5) * (ym.x - y.x));

@@ -294,15 +294,14 @@ struct FluxSrc {
         const T da = diff(q[0], q[W - 1], q[W + 1], q[2 * W]);
         const T db = diff(q[1], q[W], q[W + 2], q[2 * W + 1]);
         g[m0 + m] = mk<T>(ina ? da * ihc : T(0), inb ? db * ihc : T(0));
-        lds[rf_pad<LOGE>(t + (m0 + m) * TPS) * STRIDE] =
+        lds[rf_pad<LOGE>(t, (m0 + m) * TPS) * STRIDE] =
             mk<T>(ov[m][0] * fv[m][W], ov[m][1] * fv[m][W + 1]);
       }
     }
     rf_sync<NT>();
 #pragma unroll
     for (int m = 0; m < E; ++m) {
-      const int i = t + m * TPS;
-      auto own = [&](int d) { return lds[rf_pad<LOGE>((i + d) & (N - 1)) * STRIDE]; };
+      auto own = [&](int d) { return lds[rf_near<LOGN, LOGE>(t, m, d) * STRIDE]; };
       const cx<T> m1 = own(-1), p1 = own(1);
       cx<T> m2 = m1, p2 = p1;
       if constexpr (ORDER == 4) {
@@ -330,15 +329,15 @@ __global__ void __launch_bounds__((ZShape<LOGN>::NT))
   rf_fft<T, LOGN, S::LOGE, -1, 1, S::NT>(v, lds, t, tw);
   rf_sync<S::NT>();
 #pragma unroll
-  for (int m = 0; m < S::E; ++m) lds[rf_pad<S::LOGE>(t + m * S::TPS)] = v[m];
+  for (int m = 0; m < S::E; ++m) lds[rf_pad<S::LOGE>(t, m * S::TPS)] = v[m];
   rf_sync<S::NT>();
   // coefficients k <= N / 2 of both rows (a half-spectrum ends at N / 2)
 #pragma unroll
   for (int m = 0; m <= S::E / 2; ++m) {
     const int k = t + m * S::TPS;
     if (live && k < nm) {
-      const cx<T> y = lds[rf_pad<S::LOGE>(k)];
-      const cx<T> ym = lds[rf_pad<S::LOGE>((S::N - k) & (S::N - 1))];
+      const cx<T> y = lds[rf_pad<S::LOGE>(t, m * S::TPS)];
+      const cx<T> ym = lds[rf_mirror<LOGN, S::LOGE>(t, m)];
       const cx<T> a = mk<T>(T(0.5) * (y.x + ym.x), T(0.5) * (y.y - ym.y));
       const cx<T> b = mk<T>(T(0.5) * (y.y + ym.y), T(0.5) * (ym.x - y.x));
       if constexpr (PAIRS) {
@@ -407,14 +406,14 @@ __global__ void __launch_bounds__((XShape<LOGN, TC>::NT))
   rf_fft<T, LOGN, S::LOGE, -1, S::C, S::NT>(v, lds + c, t, tw);
   rf_sync<S::NT>();
 #pragma unroll
-  for (int m = 0; m < S::E; ++m) lds[rf_pad<S::LOGE>(t + m * S::TPS) * S::C + c] = v[m];
+  for (int m = 0; m < S::E; ++m) lds[rf_pad<S::LOGE>(t, m * S::TPS) * S::C + c] = v[m];
   rf_sync<S::NT>();
 #pragma unroll
   for (int m = 0; m <= S::E / 2; ++m) {
     const int k = t + m * S::TPS;
     if (live && k < nn) {
-      const cx<T> y = lds[rf_pad<S::LOGE>(k) * S::C + c];
-      const cx<T> ym = lds[rf_pad<S::LOGE>((S::N - k) & (S::N - 1)) * S::C + c];
+      const cx<T> y = lds[rf_pad<S::LOGE>(t, m * S::TPS) * S::C + c];
+      const cx<T> ym = lds[rf_mirror<LOGN, S::LOGE>(t, m) * S::C + c];
       const T h = T(0.5);
       const size_t o = (size_t)k * nz + za;
       out[o] = cscale<T>(mk<T>(h * (y.x + ym.x), h * (y.y - ym.y)), scale);
