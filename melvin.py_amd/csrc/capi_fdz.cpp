@@ -163,9 +163,10 @@ int create_impl(FdzHost* b, const mlv_fdz_job_desc* jobs, int njobs) {
   const int dtype = b->dtype;
   b->host.assign(sizeof(FdzJob<T>) * njobs, 0);
   const size_t lds_max = max_lds_per_block(b->device);
-  std::vector<int> prow[3], pcol[2];
+  std::vector<int> prow[3], pcol[kFdzColSizes][2];
   for (int p = 0; p < 3; ++p) prow[p].assign(njobs + 1, 0);
-  for (int p = 0; p < 2; ++p) pcol[p].assign(njobs + 1, 0);
+  for (int w = 0; w < kFdzColSizes; ++w)
+    for (int p = 0; p < 2; ++p) pcol[w][p].assign(njobs + 1, 0);
   FdzLaunch& fl = b->fl;
   std::memset(&fl, 0, sizeof(fl));
   fl.njobs = njobs;
@@ -179,21 +180,24 @@ int create_impl(FdzHost* b, const mlv_fdz_job_desc* jobs, int njobs) {
     FdzJob<T>& J = host_job<T>(b, j);
     int rc = build_fdz_job<T>(jobs[j], J, j);
     if (rc) return rc;
-    const int tc = fdz_cols_per_block<T>(J.lognx);
+    const int size = fdz_col_size(J.lognx);
     const size_t ldsc = fdz_cols_lds_bytes<T>(J.lognx);
-    if (tc < 1 || ldsc > lds_max)
+    if (ldsc > lds_max)
       return fail(MLV_ERR_UNSUPPORTED, "job " + std::to_string(j) + ": nx too large for LDS");
-    fl.ldscol = std::max(fl.ldscol, ldsc);
+    fl.ldscol[size] = std::max(fl.ldscol[size], ldsc);
     // two LDS rows (buf, vrow) per row of a block, odd strides: the rows
     // start on different banks
     fl.ldsrow = std::max(fl.ldsrow, (size_t)fdz_rows_per_block(J.wpr) * 2 * (J.nz | 1) * sizeof(double2));
     const int nph = J.scheme == MLV_FDZ_PC ? 2 : 1;
     b->nphase = std::max(b->nphase, nph);
+    const int tc = 2 * fdz_col_pairs(J.lognx);
     const int cb = (J.nz + tc - 1) / tc;
     const int rpb = fdz_rows_per_block(J.wpr);
     const int rb2 = (2 * J.nn + rpb - 1) / rpb;
     const int rb1 = (J.nn + rpb - 1) / rpb;
-    for (int p = 0; p < 2; ++p) pcol[p][j + 1] = pcol[p][j] + (p < nph ? cb : 0);
+    for (int w = 0; w < kFdzColSizes; ++w)
+      for (int p = 0; p < 2; ++p)
+        pcol[w][p][j + 1] = pcol[w][p][j] + (w == size && p < nph ? cb : 0);
     J.nbC = cb;
     b->max_nn = std::max(b->max_nn, J.nn);
     for (int p = 0; p < 3; ++p) {
@@ -238,11 +242,12 @@ int create_impl(FdzHost* b, const mlv_fdz_job_desc* jobs, int njobs) {
       if (r) return r;
     }
   }
-  for (int p = 0; p < 2; ++p) {
-    fl.ncol[p] = pcol[p][njobs];
-    int r = upload(pcol[p], &fl.prefcol[p]);
-    if (r) return r;
-  }
+  for (int w = 0; w < kFdzColSizes; ++w)
+    for (int p = 0; p < 2; ++p) {
+      fl.ncol[w][p] = pcol[w][p][njobs];
+      int r = upload(pcol[w][p], &fl.prefcol[w][p]);
+      if (r) return r;
+    }
   for (int p = 0; p < 3; ++p) {
     fl.nrow[p] = prow[p][njobs];
     int r = upload(prow[p], &fl.prefrow[p]);

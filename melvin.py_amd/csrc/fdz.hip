@@ -408,187 +408,223 @@ __global__ void __launch_bounds__(kFdzRowThreads)
 }
 
 // --------------------------------------------------------------------------
-// Column kernel: TC z columns per block (TC even), two LDS slots per column.
+// Column kernel: PB pairs of adjacent z columns per block, the NT threads in
+// four groups, one per field (ux, uz, omega, T).
 //
 // Two real sequences share one complex transform (a + i b).  The rounding
 // of a transform is relative to the whole complex sequence, so the pair
 // must hold values of similar size: omega is ~Ra times T once convection
 // starts, and packing omega with T would bury T under omega's rounding.
-// Each slot therefore pairs the same field at two adjacent z columns.
+// Each transform therefore pairs the same field at two adjacent z columns.
+//
+// A group transforms its field of the block's pairs in registers
+// (fft_reg.hpp), leaves the values in LDS, forms one product and transforms
+// that back: group 0 ux T', 1 uz T', 2 ux omega, 3 uz omega.  At up to 1024
+// points a transform is one wavefront's, so the two block barriers around the
+// exchange of the values are the only ones.  Consecutive threads take
+// consecutive pairs, so a load covers PB pairs of a row; each mode is loaded
+// once and goes through LDS to its points k and N - k (loaded at both points
+// it would be twice as many scattered 16-byte reads).
+// What bounds it: one chain of loads, two transforms and stores per block, at
+// one block per CU for one 1024x513 job.  Per launch, against columns staged
+// and transformed in LDS: 1024x513 FP32 20.4 -> 17.4 us, FP64 25.4 -> 21.7,
+// 512x257 FP32 14.7 -> 9.0, 256x129 FP64 14.2 -> 8.8, 2048x600 FP64 60.5 ->
+// 49.6; eight 1024x513 FP32 jobs 64.8 -> 55.9 (1.6 TB/s).  Three wavefronts
+// per SIMD in single precision at up to 1024 points: a bound of four costs
+// 66.9 instead of 64.6 us a step there.
 // --------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ void herm_pack(cx<T>* __restrict__ z, int k, int N, cx<T> a, cx<T> b) {
-  // Spectra of two real sequences (k < nn kept) packed into one complex
-  // sequence a + i b; irfft ignores the imaginary part of the k = 0 term.
-  if (k == 0) {
-    z[0] = mk<T>(a.x, b.x);
-  } else {
-    z[fft_pad(k)] = mk<T>(a.x - b.y, a.y + b.x);
-    z[fft_pad(N - k)] = mk<T>(a.x + b.y, b.x - a.y);
-  }
+// Hides where p comes from, so that what is read through it again is read
+// again: the compiler would keep the first transform's twiddles and the
+// velocities' spectra (56 and 24 registers in single precision) to the end of
+// the kernel, and spill them.
+template <typename P>
+__device__ __forceinline__ void opaque(P& p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(p));
+#endif
 }
 
 template <typename T>
-__host__ __device__ constexpr int fdz_tc(int slots) {
-  return slots / 2 > kNT ? kNT : slots / 2;
-}
+struct ColPair {
+  cx<T> a, b;  // two adjacent columns (aligned as one element only)
+};
 
-template <typename T, int LOGN>
+template <typename T, int LOGN, int NT>
 __device__ __forceinline__ void fdz_cols_body(const FdzJob<T>& J, int local, int phase, int flags,
-                                              int step, const cx<T>* __restrict__ tw,
-                                              cx<T>* lds) {
-  constexpr int N = 1 << LOGN;
-  constexpr int P = fdz_points<T>(LOGN);
-  constexpr int SL = fft_slots<LOGN, kNT, P>();
-  constexpr int TC = fdz_tc<T>(SL);
-  if constexpr (TC < 2) {
-    return;  // rejected on the host
-  } else {
-    constexpr int LDSN = fft_ldsn(N);
-    const int Z = J.nz, nn = J.nn;
-    const int par = (J.par0 + step) & 1;
-    const bool corr = J.scheme == MLV_FDZ_PC && phase == 1;
-    const int j0 = local * TC;
-    const int ncol = min(TC, Z - j0);
-    const int npair = (ncol + 1) / 2;
-    const int vs = corr ? 2 : par;
-    // field f of column pair p lives in slot 4 p + f: 0 ux, 1 uz, 2 omega, 3 T
-    const gptr<const cx<T>> src[4] = {glb(J.vel[vs][0]), glb(J.vel[vs][1]),
-                                      glb(corr ? J.star[0] : J.state[par][0]),
-                                      glb(corr ? J.star[1] : J.state[par][1])};
-    // The x mean of T, Tm(z) = Re T[kx=0], is O(1) (the conductive profile)
-    // while the rest is small: transforming T whole in single precision would
-    // spread Tm's rounding over every mode.  Tm is constant along x, so
-    // F_x(u Tm) = Tm F_x(u) exactly; the transforms carry T - Tm and the
-    // Tm u_s term is added per mode after the forward transform.
-    __shared__ T tmean[TC];  // (every size's body has its own)
-    for (int cc = threadIdx.x; cc < ncol; cc += kNT) tmean[cc] = src[3][j0 + cc].x;
-    const int nslot = 4 * npair;
-    const int nzero = N - 2 * nn + 1;
-    for (int e = threadIdx.x; e < nslot * nzero; e += kNT) {
-      const int sl = e / nzero, k = nn + e % nzero;
-      lds[sl * LDSN + fft_pad(k)] = czero<T>();
-    }
-    // one work item = (field, k, pair): both columns' values of one field;
-    // neighbouring threads read neighbouring column pairs
-    const int nfill = npair * 4 * nn;
-    constexpr int U = 4;
-#pragma unroll 1
-    for (int e0 = threadIdx.x; e0 < nfill; e0 += U * kNT) {
-      cx<T> a[U], b[U];
+                                              int step, const cx<T>* tw, cx<T>* lds,
+                                              T* __restrict__ tmean) {
+#pragma clang fp contract(off)
+  constexpr int N = 1 << LOGN, LOGE = fdz_loge(LOGN), E = 1 << LOGE, TPS = N / E;
+  constexpr int GT = NT / 4, PB = GT / TPS;  // threads of a group, pairs of a block
+  constexpr int REG = rf_len(LOGN, LOGE) * PB;
+  constexpr int nn = (N - 1) / 3, KI = (nn + TPS - 1) / TPS;
+  // synchronises a group's transforms: a wavefront's own, or the block's
+  constexpr int ST = GT <= 64 ? 64 : NT;
+  const int Z = J.nz;
+  const int par = (J.par0 + step) & 1;
+  const bool corr = J.scheme == MLV_FDZ_PC && phase == 1;
+  const int vs = corr ? 2 : par;
+  const int f = __builtin_amdgcn_readfirstlane(threadIdx.x / GT);
+  const int g = threadIdx.x % GT, sub = g % PB, t = TPS == 1 ? 0 : g / PB;
+  const int c0 = 2 * (local * PB + sub);  // the pair's first column
+  const bool live = c0 < Z, two = c0 + 1 < Z;
+  auto region = [&](int fld, int sb) { return lds + fld * REG + sb; };
+  cx<T>* __restrict__ mine = region(f, sub);
+  // The x mean of T, Tm(z) = Re T[kx=0], is O(1) (the conductive profile)
+  // while the rest is small: transforming T whole in single precision would
+  // spread Tm's rounding over every mode.  Tm is constant along x, so
+  // F_x(u Tm) = Tm F_x(u) exactly; the transforms carry T - Tm and the
+  // Tm u_s term is added per mode after the forward transform.
+  const gptr<const cx<T>> tsrc = glb(corr ? J.star[1] : J.state[par][1]);
+  gptr<const cx<T>> src =
+      f < 2 ? glb(J.vel[vs][f]) : (f == 3 ? tsrc : glb(corr ? J.star[0] : J.state[par][0]));
+  for (int c = threadIdx.x; c < 2 * PB; c += NT)
+    if (2 * local * PB + c < Z) tmean[c] = tsrc[2 * local * PB + c].x;
+  // A pair is one load of two elements; the last column of an odd row comes
+  // with the one before it, and idle lanes read the row's first two.
+  const int ld = !live ? 0 : (two ? c0 : c0 - 1);
+  cx<T> ka[KI], kb[KI];
+  auto load = [&] {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int e = e0 + u * kNT;
-        const int pr = e % npair, k = (e / npair) % nn, f = e / (npair * nn);
-        const int c0 = 2 * pr;
-        a[u] = czero<T>();
-        b[u] = czero<T>();
-        if (e < nfill) {
-          const size_t idx = (size_t)k * Z + j0 + c0;
-          const bool drop = f == 3 && k == 0;  // T without its x mean
-          if (!drop) {
-            a[u] = src[f][idx];
-            if (c0 + 1 < ncol) b[u] = src[f][idx + 1];
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int e = e0 + u * kNT;
-        if (e < nfill) {
-          const int pr = e % npair, k = (e / npair) % nn, f = e / (npair * nn);
-          herm_pack<T>(lds + (4 * pr + f) * LDSN, k, N, a[u], b[u]);
-        }
-      }
+    for (int i = 0; i < KI; ++i) {
+      const int k = t + i * TPS;
+      const auto p = *reinterpret_cast<gptr<const ColPair<T>>>(src + (k < nn ? k : 0) * Z + ld);
+      ka[i] = two ? p.a : p.b;
+      kb[i] = p.b;
+      // irfft ignores the imaginary part of the kx = 0 term
+      if (k == 0) ka[i].y = kb[i].y = T(0);
     }
-    __syncthreads();
-    fft_lds<T, LOGN, +1, kNT, P>(lds, nslot, tw);
-    const bool wp = (flags & kFdzWritePhys) && !corr;
-    const bool dg = (flags & kFdzDiag) && !corr && J.loops % (flags >> kFdzDiagShift) == 0;
+  };
+  load();
+#pragma unroll
+  for (int i = 0; i < KI; ++i) {
+    const int k = t + i * TPS;
+    if (!live || (f == 3 && k == 0)) ka[i] = czero<T>();  // (T without its x mean)
+    if (!two || (f == 3 && k == 0)) kb[i] = czero<T>();
+    if (k == 0) {
+      mine[0] = mk<T>(ka[i].x, kb[i].x);
+    } else if (k < nn) {
+      mine[rf_pad<LOGE>(t, i * TPS) * PB] = mk<T>(ka[i].x - kb[i].y, ka[i].y + kb[i].x);
+      mine[rf_mirror<LOGN, LOGE>(t, i) * PB] = mk<T>(ka[i].x + kb[i].y, kb[i].x - ka[i].y);
+    }
+  }
+  rf_sync<ST>();
+  cx<T> v[E];
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    const int x = t + m * TPS;
+    v[m] = czero<T>();
+    if (x < nn || x > N - nn) v[m] = mine[rf_pad<LOGE>(t, m * TPS) * PB];
+  }
+  rf_sync<ST>();
+  rf_fft<T, LOGN, LOGE, +1, PB, ST>(v, mine, t, tw);
+  rf_sync<ST>();
+#pragma unroll
+  for (int m = 0; m < E; ++m) mine[rf_pad<LOGE>(t, m * TPS) * PB] = v[m];
+  __syncthreads();
+  const bool wp = (flags & kFdzWritePhys) && !corr;
+  const bool dg = (flags & kFdzDiag) && !corr && J.loops % (flags >> kFdzDiagShift) == 0;
+  if (wp || dg) {
     T mux = -INFINITY, muz = -INFINITY;  // NaN-propagating maxima, as np.max
     double ke = 0.0, ens = 0.0, flux = 0.0;
-    for (int e = threadIdx.x; e < npair * N; e += kNT) {
-      const int pr = e / N, x = e % N;
-      cx<T>* z = lds + (4 * pr) * LDSN + fft_pad(x);
-      const cx<T> vx = z[0], vz = z[LDSN], w = z[2 * LDSN], t = z[3 * LDSN];
-      if (dg) {
-        // the imaginary parts belong to column 2 pr + 1 when it exists
-        const int c0 = 2 * pr;
-        const double t0 = (double)(t.x + tmean[c0]);
-        mux = nan_max(mux, vx.x);
-        muz = nan_max(muz, vz.x);
-        ke += (double)vz.x * (double)vz.x + (double)vx.x * (double)vx.x;
-        ens += (double)w.x * (double)w.x;
-        flux += t0 * (double)vz.x;
-        if (c0 + 1 < ncol) {
-          const double t1 = (double)(t.y + tmean[c0 + 1]);
-          mux = nan_max(mux, vx.y);
-          muz = nan_max(muz, vz.y);
-          ke += (double)vz.y * (double)vz.y + (double)vx.y * (double)vx.y;
-          ens += (double)w.y * (double)w.y;
-          flux += t1 * (double)vz.y;
-        }
-      }
-      // real parts: column 2 pr, imaginary parts: column 2 pr + 1
-      if (wp) {
-        const int c0 = 2 * pr;
-        const size_t o = (size_t)x * Z + j0 + c0;
-        const bool two = c0 + 1 < ncol;
-        const gptr<T> p0 = glb(J.phys[0]), p1 = glb(J.phys[1]), p2 = glb(J.phys[2]),
-                      p3 = glb(J.phys[3]);
-        if (p0) { p0[o] = vx.x; if (two) p0[o + 1] = vx.y; }
-        if (p1) { p1[o] = vz.x; if (two) p1[o + 1] = vz.y; }
-        if (p2) { p2[o] = w.x; if (two) p2[o + 1] = w.y; }
-        if (p3) {
-          p3[o] = t.x + tmean[c0];
-          if (two) p3[o + 1] = t.y + tmean[c0 + 1];
-        }
-      }
-      z[0] = mk<T>(vx.x * w.x, vx.y * w.y);              // ux omega
-      z[LDSN] = mk<T>(vz.x * w.x, vz.y * w.y);           // uz omega
-      z[2 * LDSN] = mk<T>(vx.x * t.x, vx.y * t.y);       // ux T'
-      z[3 * LDSN] = mk<T>(vz.x * t.x, vz.y * t.y);       // uz T'
-    }
-    if (dg) block_diag<kNT>((double)mux, (double)muz, ke, ens, flux, glb(J.diag) + (size_t)kDiagPart * local);
-    __syncthreads();
-    fft_lds<T, LOGN, -1, kNT, P>(lds, nslot, tw);
-    const T hs = (T)(0.5 / (double)N);
-    // one work item = (column, k): the four outputs of that column
-    for (int e = threadIdx.x; e < TC * nn; e += kNT) {
-      const int cc = e % TC, k = e / TC;
-      if (cc >= ncol) continue;
-      const int pr = cc >> 1;
-      const bool hi = cc & 1;
-      const size_t idx = (size_t)k * Z + j0 + cc;
-      cx<T> ov[4];
+    for (int e = threadIdx.x; e < PB * N; e += NT) {
+      const int sb = e % PB, x = e / PB, ca = 2 * (local * PB + sb), at = rf_pad<LOGE>(x) * PB;
+      if (ca >= Z) continue;
+      cx<T> q[4];
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const cx<T>* z = lds + (4 * pr + m) * LDSN;
-        const cx<T> y = z[fft_pad(k)];
-        const cx<T> ym = z[fft_pad((N - k) & (N - 1))];
-        // (y + conj ym) / 2 is the first sequence's spectrum, (y - conj ym) / 2i the second's
-        ov[m] = hi ? mk<T>(hs * (y.y + ym.y), hs * (ym.x - y.x))
-                   : mk<T>(hs * (y.x + ym.x), hs * (y.y - ym.y));
+      for (int c = 0; c < 4; ++c) q[c] = region(c, sb)[at];
+      // real parts: the pair's first column, imaginary parts: its second
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        if (ca + r >= Z) continue;
+        auto val = [&](int c) { return r ? q[c].y : q[c].x; };
+        const T vx = val(0), vz = val(1), w = val(2), tt = val(3) + tmean[2 * sb + r];
+        if (dg) {
+          mux = nan_max(mux, vx);
+          muz = nan_max(muz, vz);
+          ke += (double)vz * (double)vz + (double)vx * (double)vx;
+          ens += (double)w * (double)w;
+          flux += (double)tt * (double)vz;
+        }
+        if (wp) {
+          const size_t o = (size_t)x * Z + ca + r;
+          const gptr<T> p0 = glb(J.phys[0]), p1 = glb(J.phys[1]), p2 = glb(J.phys[2]),
+                        p3 = glb(J.phys[3]);
+          if (p0) p0[o] = vx;
+          if (p1) p1[o] = vz;
+          if (p2) p2[o] = w;
+          if (p3) p3[o] = tt;
+        }
       }
-      cx<T> vx = src[0][idx], vz = src[1][idx];
-      if (k == 0) {  // irfft keeps the real part of the kx = 0 term
-        vx.y = T(0);
-        vz.y = T(0);
-      }
-      const T tm = tmean[cc];
-      glb(J.qw[0])[idx] = ov[0];
-      glb(J.qw[1])[idx] = ov[1];
-      glb(J.qw[2])[idx] = mk<T>(ov[2].x + tm * vx.x, ov[2].y + tm * vx.y);
-      glb(J.qw[3])[idx] = mk<T>(ov[3].x + tm * vz.x, ov[3].y + tm * vz.y);
     }
+    if (dg)
+      block_diag<NT>((double)mux, (double)muz, ke, ens, flux,
+                     glb(J.diag) + (size_t)kDiagPart * local);
+  }
+  // the product: own value times T' (velocities), or ux / uz times omega
+  {
+    const cx<T>* __restrict__ pa = region(f == 3 ? 1 : 0, sub);
+    const cx<T>* __restrict__ pb = region(f < 2 ? 3 : 2, sub);
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const int at = rf_pad<LOGE>(t, m * TPS) * PB;
+      const cx<T> b = pb[at];
+      cx<T> a = v[m];
+      if (f >= 2) a = pa[at];
+      v[m] = mk<T>(a.x * b.x, a.y * b.y);
+    }
+  }
+  // every value is read before any transform writes over it
+  __syncthreads();
+  opaque(tw);
+  rf_fft<T, LOGN, LOGE, -1, PB, ST>(v, mine, t, tw);
+  rf_sync<ST>();
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    const int x = t + m * TPS;
+    if (x < nn || x > N - nn) mine[rf_pad<LOGE>(t, m * TPS) * PB] = v[m];
+  }
+  rf_sync<ST>();
+  if (f < 2) {
+    opaque(src);
+    load();
+  }
+  // group 0 Qx_T, 1 Qz_T, 2 Qx_omega, 3 Qz_omega
+  const gptr<cx<T>> dst = glb(J.qw[f ^ 2]);
+  const T hs = (T)(0.5 / (double)N);
+  const T tm0 = tmean[2 * sub], tm1 = tmean[2 * sub + 1];
+#pragma unroll
+  for (int i = 0; i < KI; ++i) {
+    const int k = t + i * TPS;
+    if (!live || k >= nn) continue;
+    // (y + conj ym) / 2 is the first column's spectrum, (y - conj ym) / 2i
+    // the second's
+    const cx<T> y = mine[rf_pad<LOGE>(t, i * TPS) * PB],
+                ym = mine[rf_mirror<LOGN, LOGE>(t, i) * PB];
+    ColPair<T> p;
+    p.a = mk<T>(hs * (y.x + ym.x), hs * (y.y - ym.y));
+    p.b = mk<T>(hs * (y.y + ym.y), hs * (ym.x - y.x));
+    if (f < 2) {
+      p.a = mk<T>(fma1(tm0, ka[i].x, p.a.x), fma1(tm0, ka[i].y, p.a.y));
+      p.b = mk<T>(fma1(tm1, kb[i].x, p.b.x), fma1(tm1, kb[i].y, p.b.y));
+    }
+    if (two)
+      *reinterpret_cast<gptr<ColPair<T>>>(dst + k * Z + c0) = p;
+    else
+      dst[k * Z + c0] = p.a;
   }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(kNT)
+// NT = 512 runs the jobs of 2048 points, whose transforms take two
+// wavefronts each, 256 all others (a job's blocks are in one of the two
+// launches' prefix arrays).
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT)
+    __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (NT == 256 ? 3 : 4) : 2)))
     k_fdz_cols(const FdzJob<T>* __restrict__ jobs, const int* __restrict__ pref, int njobs,
                int phase, int flags, int step, const cx<T>* __restrict__ tw) {
   extern __shared__ char smem_raw[];
+  __shared__ T tmean[2 * 64];  // two columns of at most 64 pairs
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int lb = xcd_logical(pref[njobs]);
   if (lb < 0) return;
@@ -596,11 +632,12 @@ __global__ void __launch_bounds__(kNT)
   const FdzJob<T>& J = jobs[jb];
   const int local = lb - pref[jb];
   switch (J.lognx) {
-#define X(L)                                                          \
-  case L:                                                             \
-    fdz_cols_body<T, L>(J, local, phase, flags, step, tw, lds);       \
+#define X(L)                                                                   \
+  case L:                                                                      \
+    if constexpr (fdz_col_threads(L) == NT)                                    \
+      fdz_cols_body<T, L, NT>(J, local, phase, flags, step, tw, lds, tmean);   \
     break;
-    X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
+    X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11)
 #undef X
     default:
       break;
@@ -730,15 +767,24 @@ static void launch_rows(const FdzJob<T>* jobs, const FdzLaunch& fl, int phase, i
                      phase, step, fl.tw64);
 }
 
+// Column blocks of the jobs whose blocks have NT threads.
+template <typename T, int NT>
+static void launch_cols(const FdzJob<T>* jobs, const FdzLaunch& fl, int phase, int flags, int step,
+                        const cx<T>* tw, hipStream_t s) {
+  constexpr int w = NT >> 9;
+  if (fl.ncol[w][phase] <= 0) return;
+  MLV_SET_LDS_ONCE((k_fdz_cols<T, NT>), fl.ldscol[w]);
+  hipLaunchKernelGGL((k_fdz_cols<T, NT>), dim3(xcd_grid(fl.ncol[w][phase])), dim3(NT),
+                     fl.ldscol[w], s, jobs, (const int*)fl.prefcol[w][phase], fl.njobs, phase,
+                     flags, step, tw);
+}
+
 template <typename T>
 hipError_t fdz_phase(const FdzJob<T>* jobs, const FdzLaunch& fl, int phase, int flags, int step,
                      const cx<T>* tw, hipStream_t s, hipEvent_t* ev) {
   if (ev) (void)hipEventRecord(ev[0], s);
-  if (fl.ncol[phase] > 0) {
-    MLV_SET_LDS_ONCE(k_fdz_cols<T>, fl.ldscol);
-    hipLaunchKernelGGL(k_fdz_cols<T>, dim3(xcd_grid(fl.ncol[phase])), dim3(kNT), fl.ldscol, s,
-                       jobs, (const int*)fl.prefcol[phase], fl.njobs, phase, flags, step, tw);
-  }
+  launch_cols<T, 256>(jobs, fl, phase, flags, step, tw, s);
+  launch_cols<T, 512>(jobs, fl, phase, flags, step, tw, s);
   if (ev) (void)hipEventRecord(ev[1], s);
   launch_rows<T>(jobs, fl, phase, step, s);
   if (ev) (void)hipEventRecord(ev[2], s);
@@ -776,7 +822,8 @@ hipError_t fdz_diag(FdzJob<T>* jobs, int njobs, int max_nn, double cutoff, int c
 
 template <typename T>
 hipError_t fdz_prepare(const FdzLaunch& fl) {
-  if (fl.ldscol) MLV_SET_LDS_ONCE(k_fdz_cols<T>, fl.ldscol);
+  if (fl.ldscol[0]) MLV_SET_LDS_ONCE((k_fdz_cols<T, 256>), fl.ldscol[0]);
+  if (fl.ldscol[1]) MLV_SET_LDS_ONCE((k_fdz_cols<T, 512>), fl.ldscol[1]);
   MLV_SET_LDS_ONCE(k_fdz_rows<T>, fl.ldsrow);
   return hipGetLastError();
 }

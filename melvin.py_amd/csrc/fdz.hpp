@@ -5,10 +5,10 @@
 // kx in [0, nn), column = z grid point.  One evaluation of the explicit
 // terms ("phase") is two kernels:
 //
-//   cols  per block of z columns: Hermitian-packed inverse x transforms of
-//         (ux_s + i uz_s) and (omega + i T), the four products ux*f, uz*f
-//         in physical space, two packed forward x transforms, keep
-//         kx < nn, scale 1/nx  ->  Qx_f, Qz_f.
+//   cols  per pair of z columns: inverse x transforms of ux, uz, omega and
+//         T, each packing the two columns, the four products ux*f, uz*f in
+//         physical space, four packed forward x transforms, keep kx < nn,
+//         scale 1/nx  ->  Qx_f, Qz_f.
 //   rows  one or two wavefronts per (x mode, field): the flux divergence
 //         D = i sx(kx) Qx + Dz(Qz) (the periodic x difference is its exact
 //         modified wavenumber; the z difference acts along the row, and both
@@ -31,6 +31,7 @@
 #include <hip/hip_runtime.h>
 #include "../../include/melvin_hip.h"
 #include "diag.hpp"
+#include "fft_reg.hpp"
 #include "transforms.hpp"
 
 namespace mlv {
@@ -79,33 +80,38 @@ struct FdzJob {
 // the loops whose count before the loop is a multiple of it)
 constexpr int kFdzWritePhys = 1, kFdzDiag = 2, kFdzDiagShift = 8;
 
+// Column kernel: points per thread (log2), threads per transform, threads
+// per block (four fields, each at least a wavefront) and column pairs per
+// block.  16 points from 1024 on: three passes, which at 1024 stay inside a
+// wavefront (8 points, four passes behind block barriers: 20 against 17 us an
+// evaluation at 1024x513 FP32, 31 against 22 FP64); 8 points below, where
+// they spread a small grid over twice the blocks.
+__host__ __device__ constexpr int fdz_loge(int lognx) { return lognx >= 10 ? 4 : 3; }
+__host__ __device__ constexpr int fdz_tps(int lognx) { return 1 << (lognx - fdz_loge(lognx)); }
+__host__ __device__ constexpr int fdz_col_threads(int lognx) {
+  return fdz_tps(lognx) > 64 ? 4 * fdz_tps(lognx) : 256;
+}
+__host__ __device__ constexpr int fdz_col_pairs(int lognx) {
+  return fdz_col_threads(lognx) / 4 / fdz_tps(lognx);
+}
+constexpr int kFdzColSizes = 2;  // block sizes 256 << i, each a launch of its own jobs
+__host__ __device__ constexpr int fdz_col_size(int lognx) {
+  return fdz_col_threads(lognx) >> 9;
+}
+
 struct FdzLaunch {
   int njobs;
-  int ncol[2];                       // column blocks of phases 0 and 1
+  int ncol[kFdzColSizes][2];         // column blocks of 256 and 512 threads, phases 0 and 1
   int nrow[3];                       // row blocks of phases 0, 1 and the prologue
-  size_t ldsrow, ldscol;
+  size_t ldsrow, ldscol[kFdzColSizes];
   const double2* tw64;               // FP64 twiddles exp(-2 pi i k / NMAX)
-  int *prefcol[2];
+  int *prefcol[kFdzColSizes][2];
   int *prefrow[3];
 };
 
-// Points per thread of the column kernel: 16 below N = 2048 (two columns
-// per block at 1024, so a single job's z columns spread over twice as many
-// CUs as at 32 points), 32 at 2048 (a block must hold a column pair).
-template <typename T>
-__host__ __device__ constexpr int fdz_points(int lognx) {
-  return lognx >= 11 ? 32 : 16;
-}
-// Columns per block of the column kernel (two LDS slots each, in pairs of
-// columns); 0 when the LDS slots do not hold two columns.
-template <typename T>
-inline int fdz_cols_per_block(int lognx) {
-  const int s = ((kNT * fdz_points<T>(lognx)) >> lognx) / 2;
-  return s < 2 ? 0 : (s > kNT ? kNT : s);
-}
 template <typename T>
 inline size_t fdz_cols_lds_bytes(int lognx) {
-  return (size_t)((kNT * fdz_points<T>(lognx)) >> lognx) * fft_ldsn(1 << lognx) * sizeof(cx<T>);
+  return (size_t)4 * fdz_col_pairs(lognx) * rf_len(lognx, fdz_loge(lognx)) * sizeof(cx<T>);
 }
 
 template <typename T>
