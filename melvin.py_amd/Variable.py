@@ -98,7 +98,9 @@ class Variable:
     def vec_dot_nabla(self, ux, uz, out=None, convert_to_physical=True):
         pl = plan_for(self._params)
         if out is None:
-            if self._fourier(pl):
+            if self._fourier(pl) and all(
+                    isinstance(u, torch.Tensor) and plain(u, pl.real, (pl.nx, pl.nz))
+                    for u in (ux, uz)):
                 return self._advect(pl, ux, uz, convert_to_physical)
             out = hip.zeros_like(self._pdata)
         if convert_to_physical:
@@ -115,9 +117,11 @@ class Variable:
 
     def _fourier(self, pl):
         """Whether this is a field of Fourier (or Fourier-x / FD-z) modes held
-        as the plan's kernels take it, transformed by this package."""
+        as the plan's kernels take it, transformed by this package's own
+        methods (a subclass may transform differently)."""
         bx, bz = self._basis_functions
-        return (isinstance(self._st, SpectralTransformer) and self._st._plan is pl
+        return (type(self._st) is SpectralTransformer and self._st._plan is pl
+                and type(self).to_physical is Variable.to_physical
                 and bx is BasisFunctions.COMPLEX_EXP
                 and bz is (BasisFunctions.COMPLEX_EXP if pl.fully else BasisFunctions.FDM)
                 and plain(self._sdata, pl.cplx, (pl.rows, pl.cols))
@@ -125,11 +129,11 @@ class Variable:
 
     def _advect(self, pl, ux, uz, convert_to_physical):
         """vec_dot_nabla whose flux divergence is formed inside the forward
-        transform, so the caller's ``out`` is the only thing it leaves out."""
-        a = as_input(ux, pl.real, (pl.nx, pl.nz))
-        b = as_input(uz, pl.real, (pl.nx, pl.nz))
+        transform, so the caller's ``out`` is the only thing it leaves out.
+        ux and uz are read in place: one may be this field's own physical
+        array, which the conversion writes first."""
         spec = torch.empty((pl.rows, pl.cols), dtype=pl.cplx, device=self._pdata.device)
-        _lib.call("mlv_advect", pl.handle, ptr(a), ptr(b),
+        _lib.call("mlv_advect", pl.handle, ptr(ux), ptr(uz),
                   ptr(self._sdata) if convert_to_physical else ctypes.c_void_p(0),
                   ptr(self._pdata), ptr(spec), _lib.stream_handle())
         return spec

@@ -52,7 +52,8 @@ def calc_velocity_from_vorticity(vorticity, streamfunction, ux, uz,
     if (all(v._fourier(pl) for v in one) and plain(w, pl.cplx, (pl.rows, pl.cols))
             and plain(psi, pl.cplx, (pl.rows, pl.cols))
             and len({w.data_ptr(), psi.data_ptr(), ux._sdata.data_ptr(),
-                     uz._sdata.data_ptr()}) == 4):
+                     uz._sdata.data_ptr()}) == 4
+            and len({v._pdata.data_ptr() for v in (streamfunction, ux, uz)}) == 3):
         _lib.call("mlv_velocity_physical", pl.handle, ptr(w), ptr(psi),
                   null if fdm_z else ptr(ux._sdata), ptr(uz._sdata),
                   ptr(streamfunction._pdata) if fdm_z else null, ptr(ux._pdata),

@@ -81,3 +81,40 @@ def test_velocity_equals_separate_operators(mlv, nx, nz, fdz, precision):
     else:
         assert torch.equal(ux.getp(), st.to_physical(ux.gets(), basis_functions=bfs))
     assert torch.isfinite(ux.getp()).all()
+
+
+@pytest.mark.parametrize("fdz", [False, True])
+def test_velocity_arguments_that_share_the_fields_memory(mlv, fdz):
+    """The field's own physical array as a velocity, as it is and transposed
+    (a view that has to be copied after the conversion, not before)."""
+    import torch
+
+    p, sim, bfs = _make(mlv, 64, 64, fdz, "double", 2)
+    for view in (lambda v: v.getp(), lambda v: v.getp().T):
+        a, b = (sim.make_variable("v", bfs) for _ in range(2))
+        for v in (a, b):
+            v.sets(_random_spectrum(mlv, p, 3))
+            v.getp().fill_(7.0)
+        got = a.vec_dot_nabla(view(a), view(a))
+        want = b.vec_dot_nabla(view(b), view(b), out=torch.empty_like(b.getp()))
+        top = float(a.getp().abs().max()) ** 2
+        bound = 40 * EPS["double"] * top * (1 / p.dx + 1 / p.dz)
+        assert float((got - want).abs().max()) <= bound
+
+
+def test_overridden_transforms_are_used(mlv):
+    """A transformer or variable class of the caller's own keeps its say."""
+    p, sim, bfs = _make(mlv, 32, 32, False, "double", 2)
+
+    class Doubling(mlv.SpectralTransformer):
+        def to_spectral(self, *a, **k):
+            return 2.0 * super().to_spectral(*a, **k)
+
+    ux, uz = (mlv.hip.asarray(np.random.default_rng(k).standard_normal((32, 32))) for k in (1, 2))
+    a, b = (sim.make_variable("v", bfs) for _ in range(2))
+    for v in (a, b):
+        v.sets(_random_spectrum(mlv, p, 4))
+    b._st = Doubling(p, mlv.hip)
+    got, want = a.vec_dot_nabla(ux, uz), b.vec_dot_nabla(ux, uz)
+    scale = float(want.abs().max())
+    assert float((2.0 * got - want).abs().max()) <= 1e-10 * scale
