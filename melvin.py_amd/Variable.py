@@ -10,9 +10,10 @@ import numpy as np
 import torch
 
 from . import _lib, hip
-from ._arrays import as_input, plain
+from ._arrays import as_input, own, plain
 from ._plans import plan_for, ptr
 from .BasisFunctions import BasisFunctions
+from .SpatialDifferentiator import SpatialDifferentiator
 from .SpectralTransformer import SpectralTransformer
 
 
@@ -118,14 +119,21 @@ class Variable:
     def _fourier(self, pl):
         """Whether this is a field of Fourier (or Fourier-x / FD-z) modes held
         as the plan's kernels take it, transformed by this package's own
-        methods (a subclass may transform differently)."""
+        methods (a subclass or an instance may have others)."""
         bx, bz = self._basis_functions
         return (type(self._st) is SpectralTransformer and self._st._plan is pl
-                and type(self).to_physical is Variable.to_physical
+                and own(self._st, SpectralTransformer, "to_physical", "to_spectral")
+                and own(self, Variable, "to_physical")
                 and bx is BasisFunctions.COMPLEX_EXP
                 and bz is (BasisFunctions.COMPLEX_EXP if pl.fully else BasisFunctions.FDM)
                 and plain(self._sdata, pl.cplx, (pl.rows, pl.cols))
                 and plain(self._pdata, pl.real, (pl.nx, pl.nz)))
+
+    def _own_pddz(self, pl):
+        """Whether pddz is this package's difference of this field's own
+        physical array."""
+        return (own(self, Variable, "pddz", "getp") and type(self._sd) is SpatialDifferentiator
+                and self._sd._plan is pl and own(self._sd, SpatialDifferentiator, "pddz", "_fd"))
 
     def _advect(self, pl, ux, uz, convert_to_physical):
         """vec_dot_nabla whose flux divergence is formed inside the forward

@@ -37,6 +37,12 @@ def plain(t, dtype, shape):
             and t.is_contiguous())
 
 
+def own(obj, cls, *names):
+    """Whether these methods of ``obj`` are ``cls``'s: neither a subclass nor
+    the instance puts another in their place."""
+    return all(getattr(getattr(obj, n), "__func__", None) is getattr(cls, n) for n in names)
+
+
 def finish(tmp, out):
     if tmp is not out:
         out.copy_(tmp)

@@ -9,9 +9,10 @@ import numpy as np
 from numpy.random import default_rng
 
 from . import _lib, hip
-from ._arrays import plain
+from ._arrays import own, plain
 from ._plans import plan_for, ptr
 from .BasisFunctions import BasisFunctions
+from .Variable import Variable
 
 
 def sech(x):
@@ -49,7 +50,10 @@ def calc_velocity_from_vorticity(vorticity, streamfunction, ux, uz,
         raise ValueError("vorticity and streamfunction must be contiguous")
     fdm_z = streamfunction._basis_functions[1] is BasisFunctions.FDM
     one = ((vorticity, streamfunction, ux, uz) if fdm_z or not pl.fully else (ux, uz))
-    if (all(v._fourier(pl) for v in one) and plain(w, pl.cplx, (pl.rows, pl.cols))
+    # (FD z forms ux in place of ux.setp(-streamfunction.pddz()))
+    if (all(v._fourier(pl) for v in one)
+            and (not fdm_z or (streamfunction._own_pddz(pl) and own(ux, Variable, "setp")))
+            and plain(w, pl.cplx, (pl.rows, pl.cols))
             and plain(psi, pl.cplx, (pl.rows, pl.cols))
             and len({w.data_ptr(), psi.data_ptr(), ux._sdata.data_ptr(),
                      uz._sdata.data_ptr()}) == 4
