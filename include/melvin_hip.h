@@ -183,7 +183,8 @@ int mlv_velocity_physical(mlv_plan* plan, const void* w, void* psi, void* ux_spe
                           void* psi_phys, void* ux_phys, void* uz_phys, void* stream);
 /* Variable.vec_dot_nabla (Variable.py:119-128): f_phys = to_physical(f_spec)
  * unless f_spec is NULL, then out_spec = to_spectral(pddx(ux f) + pddz(uz f));
- * ux, uz, f_phys are physical fields. */
+ * ux, uz, f_phys are physical fields.  (FD-z plans beyond nx = 1024 are
+ * faster as mlv_to_physical, mlv_flux_divergence and mlv_to_spectral.) */
 int mlv_advect(mlv_plan* plan, const void* ux, const void* uz, const void* f_spec, void* f_phys,
                void* out_spec, void* stream);
 /* FP64 reduction of n values of type dtype (b used by SUMSQ2/DOT); writes

@@ -99,7 +99,14 @@ class Variable:
     def vec_dot_nabla(self, ux, uz, out=None, convert_to_physical=True):
         pl = plan_for(self._params)
         if out is None:
-            if self._fourier(pl) and all(
+            # FD z beyond 1024 points along x: a thread of the transform that
+            # forms the flux holds 16 points with the operands of six to eight
+            # columns and spills (us a call, fused against stencil then
+            # transform: 2048x65 FP64 31 and 23 at order 2, 40 and 23 at order
+            # 4; 2048x700 37 and 39, 49 and 39; 4096x512 100 and 60, 156 and
+            # 62; at 1024x513 20 and 24, 22 and 25)
+            fused = pl.fully or pl.nx <= 1024
+            if fused and self._fourier(pl) and all(
                     isinstance(u, torch.Tensor) and plain(u, pl.real, (pl.nx, pl.nz))
                     for u in (ux, uz)):
                 return self._advect(pl, ux, uz, convert_to_physical)

@@ -1,0 +1,34 @@
+"""Long axes whose calls run as separate operators: the result is theirs bit
+for bit.  (The fused forms round otherwise.)"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _fdz(mlv, nx, nz, precision, order):
+    p = mlv.Parameters(dict(nx=nx, nz=nz, lx=2.0, lz=1.5, final_time=1.0, precision=precision,
+                            spatial_derivative_order=order, integrator="explicit",
+                            discretisation=["spectral", "fdm"]))
+    sim = mlv.Simulation(p, mlv.hip)
+    bfs = [mlv.BasisFunctions.COMPLEX_EXP, mlv.BasisFunctions.FDM]
+    rng = np.random.default_rng(nx + nz)
+    s = rng.standard_normal(p.spectral_shape) + 1j * rng.standard_normal(p.spectral_shape)
+    return p, sim, bfs, mlv.hip.asarray(s.astype(p.complex))
+
+
+@pytest.mark.parametrize("precision", ["double", "single"])
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("nx,nz", [(2048, 64), (4096, 7), (4096, 64)])
+def test_fdz_advection_beyond_1024_points(mlv, nx, nz, order, precision):
+    import torch
+
+    p, sim, bfs, s = _fdz(mlv, nx, nz, precision, order)
+    a, b = (sim.make_variable("v", bfs) for _ in range(2))
+    a.sets(s)
+    b.sets(s)
+    rng = np.random.default_rng(3)
+    ux, uz = (mlv.hip.asarray(rng.standard_normal((nx, nz)).astype(p.float)) for _ in range(2))
+    want = b.vec_dot_nabla(ux, uz, out=torch.empty_like(b.getp()))
+    assert torch.equal(a.vec_dot_nabla(ux, uz), want)
+    assert torch.equal(a.getp(), b.getp())
