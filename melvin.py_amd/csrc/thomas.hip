@@ -6,6 +6,7 @@
 // FP64 throughout; the state type only changes the load and store.
 #include "affine_scan.hpp"
 #include "common.hpp"
+#include "grid.hpp"
 #include "ops.hpp"
 
 namespace mlv {
@@ -163,10 +164,9 @@ __global__ void __launch_bounds__(64) k_thomas_serial(const cx<T>* __restrict__ 
 template <typename T, int NT>
 static void launch_nt(const void* rhs, void* out, void* uz, const double2* fac, double lower,
                       double sign, double fx, int nn, int nz, int K, hipStream_t s) {
+  // (rows near 4096 points take over 64 KB with the wavefronts' totals)
   const size_t lds = (size_t)nz * sizeof(double2);
-  if (lds > 65536)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_thomas<T, NT>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  MLV_SET_LDS_ONCE((&k_thomas<T, NT>), lds);
   hipLaunchKernelGGL((k_thomas<T, NT>), dim3(nn), dim3(NT), lds, s, (const cx<T>*)rhs, (cx<T>*)out,
                      (cx<T>*)uz, fac, lower, sign, fx, nz, K);
 }
