@@ -676,12 +676,16 @@ int mlv_velocity(mlv_plan* p, const void* w, void* psi, void* ux_spec, void* uz_
     return MLV_OK;
   }
   if (ux_spec) return fail(MLV_ERR_ARG, "FD-z: ux comes from the physical z-derivative of psi");
+  int nt, K;
+  thomas_layout(p->nz, &nt, &K);
+  void* uz = nt ? uz_spec : nullptr;
   e = DISPATCH(p,
-               launch_thomas<float>(w, psi, uz_spec, p->work, p->fac, p->lower, -1.0, p->fx, p->nn,
+               launch_thomas<float>(w, psi, uz, p->work, p->fac, p->lower, -1.0, p->fx, p->nn,
                                     p->nz, s),
-               launch_thomas<double>(w, psi, uz_spec, p->work, p->fac, p->lower, -1.0, p->fx, p->nn,
+               launch_thomas<double>(w, psi, uz, p->work, p->fac, p->lower, -1.0, p->fx, p->nn,
                                      p->nz, s));
   if (e != hipSuccess) return hip_fail(e, "velocity poisson");
+  if (uz_spec && !uz) return mlv_spec_op(p, MLV_SPEC_DDX, psi, uz_spec, stream);
   return MLV_OK;
 }
 

@@ -44,8 +44,8 @@ hipError_t launch_combine(const void* hist, void* out, size_t n, int q, int curr
 template <typename T>
 hipError_t launch_velocity(const void* w, void* psi, void* ux, void* uz, int rows, int cols, int nn,
                            double fx, double fz, double fx2, double fz2, hipStream_t s);
-// Tridiagonal Poisson solve per x mode: out = solve(sign rhs) and, with uz,
-// uz = i fx n out.  fac holds (cp_j, 1/den_j) per element, rows of K nt
+// Tridiagonal Poisson solve per x mode: out = solve(sign rhs) and, with uz
+// (rows of a block, nt > 0, only), uz = i fx n out.  fac holds (cp_j, 1/den_j) per element, rows of K nt
 // entries in the chunk-major layout of thomas_layout(nz) -- entry i nt + t is
 // element t K + i, padding (0, 1) -- or row-major where nt = 0 (dwork then
 // holds (nn, nz) complex128).

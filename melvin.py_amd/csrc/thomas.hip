@@ -129,19 +129,18 @@ __global__ void __launch_bounds__(NT) k_thomas(const cx<T>* __restrict__ rhs,
 }
 
 // Rows longer than a block's threads hold (thomas_layout): one thread per
-// mode sweeps its row; factors row-major.
+// mode sweeps its row; factors row-major.  uz is not formed here: the store
+// lengthens each step of the sweep (64 x 5000 FP64 1881 -> 1954 us), a pass of
+// its own is short beside it.
 template <typename T>
 __global__ void __launch_bounds__(64) k_thomas_serial(const cx<T>* __restrict__ rhs,
                                                       cx<T>* __restrict__ out,
-                                                      cx<T>* __restrict__ uz,
                                                       double2* __restrict__ dwork,
                                                       const double2* __restrict__ fac,
-                                                      double lower, double sign, double fx, int nn,
-                                                      int nz) {
+                                                      double lower, double sign, int nn, int nz) {
   const int n = blockIdx.x * 64 + threadIdx.x;
   if (n >= nn) return;
   const size_t row = (size_t)n * nz;
-  const T y = (T)(fx * n);
   double2 d = make_double2(0.0, 0.0);
   for (int j = 0; j < nz; ++j) {
     const cx<T> r = rhs[row + j];
@@ -155,9 +154,7 @@ __global__ void __launch_bounds__(64) k_thomas_serial(const cx<T>* __restrict__ 
     const double c = fac[row + j].x;
     const double2 dj = dwork[row + j];
     x = make_double2(dj.x - c * x.x, dj.y - c * x.y);
-    const cx<T> p = mk<T>((T)x.x, (T)x.y);
-    out[row + j] = p;
-    if (uz) uz[row + j] = mk<T>(-(y * p.y), y * p.x);
+    out[row + j] = mk<T>((T)x.x, (T)x.y);
   }
 }
 
@@ -184,8 +181,7 @@ hipError_t launch_thomas(const void* rhs, void* out, void* uz, void* dwork, cons
     case 1024: launch_nt<T, 1024>(rhs, out, uz, fac, lower, sign, fx, nn, nz, K, s); break;
     default:
       hipLaunchKernelGGL(k_thomas_serial<T>, dim3((nn + 63) / 64), dim3(64), 0, s,
-                         (const cx<T>*)rhs, (cx<T>*)out, (cx<T>*)uz, (double2*)dwork, fac, lower,
-                         sign, fx, nn, nz);
+                         (const cx<T>*)rhs, (cx<T>*)out, (double2*)dwork, fac, lower, sign, nn, nz);
   }
   return hipGetLastError();
 }

@@ -32,3 +32,17 @@ def test_fdz_advection_beyond_1024_points(mlv, nx, nz, order, precision):
     want = b.vec_dot_nabla(ux, uz, out=torch.empty_like(b.getp()))
     assert torch.equal(a.vec_dot_nabla(ux, uz), want)
     assert torch.equal(a.getp(), b.getp())
+
+
+@pytest.mark.parametrize("precision", ["double", "single"])
+def test_velocity_of_rows_beyond_a_block(mlv, precision):
+    import torch
+
+    p, sim, bfs, s = _fdz(mlv, 32, 4099, precision, 2)
+    w, psi, ux, uz = (sim.make_variable(n, bfs) for n in ("w", "psi", "ux", "uz"))
+    w.sets(s)
+    sim.init_laplacian_solver(bfs)
+    mlv.utility.calc_velocity_from_vorticity(w, psi, ux, uz, sim.get_laplacian_solver())
+    assert torch.equal(psi.gets(), sim.get_laplacian_solver().solve(-w.gets()))
+    assert torch.equal(uz.gets(), psi.sddx())
+    assert torch.equal(ux.getp(), -psi.pddz())
