@@ -740,8 +740,6 @@ int mlv_advect(mlv_plan* p, const void* ux, const void* uz, const void* f_spec, 
   CHECK_PTR(f_phys);
   CHECK_PTR(out_spec);
   hipStream_t s = (hipStream_t)stream;
-  // the stencils wrap at most once
-  if (p->nz < 5) return fail(MLV_ERR_ARG, "FD axis shorter than 5 points");
   if (f_spec) {
     const int rc = mlv_to_physical(p, f_spec, f_phys, stream);
     if (rc) return rc;

@@ -287,14 +287,14 @@ __host__ __device__ constexpr bool bsplit_fits(int logn, int v) {
 }
 // Plans of the z pass (BatchLaunch::planB).  kPlanTwoSweep runs the sizes
 // that bsplit_fits names on the LDS-staged pass in 16,16,R passes both ways,
-// the products in a sweep of their own.  kPlanSplit runs them with the
-// products between the last inverse and the first forward pass (single
-// precision), or on the register pass (double precision, stepZ_body).
+// the products in a sweep of their own.  kPlanSplit runs them on the register
+// pass (stepZ_body) where z_reg_fits, else with the products between the last
+// inverse and the first forward pass.
 constexpr int kPlanSplit = 0, kPlanTwoSweep = 1;
 
 // The register z pass: 2^logn points over z_tps threads (a wavefront, or
-// part of one: 8 points per thread up to 512, 16 at 1024, 32 at 2048), one
-// wavefront per input channel or output, whichever are more.
+// part of one: 8 points per thread up to 512, 16 at 1024), one wavefront per
+// input channel or output, whichever are more.
 __host__ __device__ constexpr int z_tps(int logn) { return logn >= 9 ? 64 : 1 << (logn - 3); }
 __host__ __device__ constexpr int z_loge(int logn) { return logn >= 9 ? logn - 6 : 3; }
 __host__ __device__ constexpr int z_waves(int v) {
@@ -306,20 +306,18 @@ template <typename T>
 __host__ __device__ constexpr size_t z_lds_bytes(int logn, int v) {
   return (size_t)z_waves(v) * (64 / z_tps(logn)) * rf_len(logn, z_loge(logn)) * sizeof(cx<T>);
 }
-// Sizes the register pass takes, in double precision; the rest (4096 points,
-// and programs of six regions at 2048) run the two-sweep pass under either
-// plan.
+// Sizes the register pass takes, in double precision.  At 2048 points, 32 per
+// thread and 250 registers, it loses to the split pass (us per launch, register
+// and split: vortex 2048^2 62 and 52, 4 of them 234 and 227, with a scalar 81
+// and 70; at 1024^2 16 and 17, MHD 24.3 and 26.4).
 template <typename T>
 __host__ __device__ constexpr bool z_reg_fits(int logn, int v) {
-  return sizeof(T) == 8 && logn <= 11 && z_lds_bytes<T>(logn, v) <= kLdsMax;
+  return sizeof(T) == 8 && logn <= 10 && z_lds_bytes<T>(logn, v) <= kLdsMax;
 }
 // Whether register m of a thread holds a kept coefficient or its mirror.
 __host__ __device__ constexpr bool z_any(int m, int tps, int n) {
   return m * tps < xp_nn(n) || (m + 1) * tps - 1 > n - xp_nn(n);
 }
-// Kernels compiled for z extents up to 2^kZLo and up to 2^11.
-constexpr int kZLo = 10;
-
 // workspace channel of equation e's Px (k=0) / Pz (k=1) output; the
 // z-pass inputs occupy channels [0, base)
 __host__ __device__ constexpr int pchan(int base, int e, int k) { return base + 2 * e + k; }

@@ -3,10 +3,8 @@
 
 namespace mlv {
 
-// The register pass (double precision).  LO: the largest z extent (log2) of
-// the launch's jobs that this kernel is compiled for: 2048 points take 32 per
-// thread and would set every size's registers.
-template <typename T, int V, int LO>
+// The register pass (double precision).
+template <typename T, int V>
 __global__ void __launch_bounds__(64 * z_waves(V))
     k_stepZ(const JobDev<T>* __restrict__ jobs, const int* __restrict__ pref, int njobs,
             int stage, int flags, const cx<T>* __restrict__ tw) {
@@ -20,10 +18,10 @@ __global__ void __launch_bounds__(64 * z_waves(V))
   switch (J.lognz) {
 #define X(L)                                                                \
   case L:                                                                   \
-    if constexpr (L <= LO && z_reg_fits<T>(L, V))                                            \
+    if constexpr (z_reg_fits<T>(L, V))                                      \
       stepZ_body<T, L, V>(J, J.st[stage], local, flags, tw, lds);           \
     break;
-    X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11)
+    X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10)
 #undef X
     default:
       break;
@@ -48,12 +46,12 @@ __global__ void __launch_bounds__(kNT)
 // --------------------------------------------------------------------------
 // Launchers
 // --------------------------------------------------------------------------
-template <typename T, int V, int LO>
+template <typename T, int V>
 static void launchZ(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int flags,
                     const cx<T>* tw, hipStream_t s) {
   const ZLaunch& z = bl.z[bl.planB];
-  MLV_SET_LDS_ONCE((k_stepZ<T, V, LO>), z.lds[V]);
-  hipLaunchKernelGGL((k_stepZ<T, V, LO>), dim3(xcd_grid(z.n[stage][V])), dim3(64 * z_waves(V)),
+  MLV_SET_LDS_ONCE((k_stepZ<T, V>), z.lds[V]);
+  hipLaunchKernelGGL((k_stepZ<T, V>), dim3(xcd_grid(z.n[stage][V])), dim3(64 * z_waves(V)),
                      z.lds[V], s, jobs, (const int*)z.pref[stage][V], bl.njobs, stage, flags, tw);
 }
 
@@ -69,26 +67,20 @@ static void launchB_plan(const JobDev<T>* jobs, const BatchLaunch& bl, int stage
 template <typename T, int V>
 static void launchB(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int flags,
                     const cx<T>* tw, hipStream_t s) {
-  const bool swept = bl.zsweep[bl.planB].n[stage][V] != 0;
-  if constexpr (sizeof(T) == 8) {
-    if (bl.z[bl.planB].n[stage][V]) {
-      if (bl.lognz_max <= kZLo)
-        launchZ<T, V, kZLo>(jobs, bl, stage, flags, tw, s);
-      else
-        launchZ<T, V, 11>(jobs, bl, stage, flags, tw, s);
-    }
-    if (swept) launchB_plan<T, V, 0, kPlanTwoSweep>(jobs, bl, stage, flags, tw, s);
-  } else {
-    if (!swept) return;
+  if constexpr (sizeof(T) == 8)
+    if (bl.z[bl.planB].n[stage][V]) launchZ<T, V>(jobs, bl, stage, flags, tw, s);
+  if (bl.zsweep[bl.planB].n[stage][V] == 0) return;
+  const bool two = bl.planB == kPlanTwoSweep;
+  if constexpr (sizeof(T) == 4) {
     if (fixed_logn(bl.lognz_all)) return launch_zpass_fixed(V, jobs, bl, stage, flags, tw, s);
-    const bool two = bl.planB == kPlanTwoSweep;
-    if (bl.split)  // some job carries mean profiles
+    if (bl.split) {  // some job carries mean profiles
       two ? launchB_plan<T, V, 1, kPlanTwoSweep>(jobs, bl, stage, flags, tw, s)
           : launchB_plan<T, V, 1, kPlanSplit>(jobs, bl, stage, flags, tw, s);
-    else
-      two ? launchB_plan<T, V, 0, kPlanTwoSweep>(jobs, bl, stage, flags, tw, s)
-          : launchB_plan<T, V, 0, kPlanSplit>(jobs, bl, stage, flags, tw, s);
+      return;
+    }
   }
+  two ? launchB_plan<T, V, 0, kPlanTwoSweep>(jobs, bl, stage, flags, tw, s)
+      : launchB_plan<T, V, 0, kPlanSplit>(jobs, bl, stage, flags, tw, s);
 }
 
 template <typename T>
@@ -105,13 +97,12 @@ template <typename T, int V>
 static void prepareB(const BatchLaunch& bl) {
   for (int p = 0; p < 2; ++p) {
     const size_t zl = bl.z[p].lds[V], bs = bl.zsweep[p].lds[V];
-    if constexpr (sizeof(T) == 8) {
-      if (zl && bl.lognz_max <= kZLo) MLV_SET_LDS_ONCE((k_stepZ<T, V, kZLo>), zl);
-      if (zl && bl.lognz_max > kZLo) MLV_SET_LDS_ONCE((k_stepZ<T, V, 11>), zl);
-      if (bs) MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanTwoSweep>), bs);
-    } else if (bs) {
-      MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanSplit>), bs);
-      MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanTwoSweep>), bs);
+    if constexpr (sizeof(T) == 8)
+      if (zl) MLV_SET_LDS_ONCE((k_stepZ<T, V>), zl);
+    if (!bs) continue;
+    MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanSplit>), bs);
+    MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanTwoSweep>), bs);
+    if constexpr (sizeof(T) == 4) {
       MLV_SET_LDS_ONCE((k_stepB<T, V, 1, kPlanSplit>), bs);
       MLV_SET_LDS_ONCE((k_stepB<T, V, 1, kPlanTwoSweep>), bs);
     }

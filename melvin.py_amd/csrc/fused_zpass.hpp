@@ -223,7 +223,8 @@ __device__ __forceinline__ void stepZ_body(const JobDev<T>& J, const StageDev& S
 // rows and its products, between two fused passes, cost no LDS trip of their
 // own: 106 against 120 us at 16 x 1024^2 with the register pass, 12 against 15
 // on tearing at 4 x 512^2, 43 against 58 on a mixed batch of double
-// diffusion), double precision the two-sweep plan and z_reg_fits' exceptions.
+// diffusion), double precision the two-sweep plan and the sizes that
+// z_reg_fits leaves out.
 // --------------------------------------------------------------------------
 // SPLIT (single precision): jobs with split carry mean profiles (kernel M)
 // and mean-free channels; a batch without such jobs runs SPLIT = 0.
@@ -598,7 +599,7 @@ __device__ __forceinline__ void roleB(const JobDev<T>* __restrict__ jobs, const 
   switch (J.lognz) {
 #define X(L)                                                          \
   case L:                                                             \
-    if constexpr (sizeof(T) == 8 && L < 9)                            \
+    if constexpr (sizeof(T) == 8 && (L < 9 || (PLAN == kPlanSplit && z_reg_fits<T>(L, V)))) \
       break; /* the register pass's */                                \
     else if constexpr (PLAN == kPlanSplit && bsplit_ok<T, L, V>())    \
       stepB_split<T, L, V, SPLIT>(J, J.st[stage], local, flags, tw, lds); \
