@@ -409,9 +409,17 @@ struct BatchLaunch {
   int lognx_max, lognz_max;            // the largest sizes (log2)
 };
 
-// Kernels A and C are compiled for x sizes up to 2^kXpLo and for all: the
-// larger sizes' points per thread would set every size's registers.
+// Kernels A and C are compiled for x sizes up to 2^kXpLo and for all, in
+// double precision also for up to 2^11: the larger sizes' points per thread
+// would set every size's registers.  (2048^2 FP64 in kernel C compiled for 4096
+// points, 402 registers, one wavefront per SIMD: 39.7 us a launch, with a
+// scalar 76 and 4 of them 293; compiled for 2048, 243 registers: 30.0, 64 and
+// 240.)
 constexpr int kXpLo = 10;
+template <typename T>
+constexpr int xp_lo(int logn) {
+  return logn <= kXpLo ? kXpLo : (sizeof(T) == 8 && logn == 11 ? 11 : 12);
+}
 
 // One-size batches that take kernel C's shape 2, kernel A's mixed tiles and
 // single precision's z-pass kernels of one size.

@@ -64,10 +64,13 @@ static void launchA_lo(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, 
 template <typename T, int NT, bool MIXED>
 static void launchA(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int step,
                     const cx<T>* tw, hipStream_t s) {
-  if (bl.lognx_max <= kXpLo)
-    launchA_lo<T, NT, kXpLo, MIXED>(jobs, bl, stage, step, tw, s);
-  else if constexpr (!MIXED)
+  const int lo = xp_lo<T>(bl.lognx_max);
+  if (lo == kXpLo) return launchA_lo<T, NT, kXpLo, MIXED>(jobs, bl, stage, step, tw, s);
+  if constexpr (!MIXED && xp_fits<T>(11, NT)) {  // (no smaller block holds a column)
+    if constexpr (sizeof(T) == 8)
+      if (lo == 11) return launchA_lo<T, NT, 11, MIXED>(jobs, bl, stage, step, tw, s);
     launchA_lo<T, NT, 12, MIXED>(jobs, bl, stage, step, tw, s);
+  }
 }
 
 template <typename T>
@@ -88,10 +91,13 @@ void launch_xinv(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int st
 
 template <typename T, int NT>
 static void prepareA(const BatchLaunch& bl, size_t lds) {
-  if (bl.lognx_max <= kXpLo)
-    MLV_SET_LDS_ONCE((k_stepA<T, NT, kXpLo, false>), lds);
-  else
-    MLV_SET_LDS_ONCE((k_stepA<T, NT, 12, false>), lds);
+  const int lo = xp_lo<T>(bl.lognx_max);
+  if (lo == kXpLo) MLV_SET_LDS_ONCE((k_stepA<T, NT, kXpLo, false>), lds);
+  if constexpr (xp_fits<T>(11, NT)) {
+    if constexpr (sizeof(T) == 8)
+      if (lo == 11) MLV_SET_LDS_ONCE((k_stepA<T, NT, 11, false>), lds);
+    if (lo == 12) MLV_SET_LDS_ONCE((k_stepA<T, NT, 12, false>), lds);
+  }
 }
 
 template <typename T>

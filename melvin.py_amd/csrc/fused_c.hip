@@ -54,10 +54,13 @@ static void launchC_lo(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, 
 template <typename T, int NT>
 static void launchC(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int step,
                     const cx<T>* tw, hipStream_t s) {
-  if (bl.lognx_max <= kXpLo)
-    launchC_lo<T, NT, kXpLo>(jobs, bl, stage, step, tw, s);
-  else
+  const int lo = xp_lo<T>(bl.lognx_max);
+  if (lo == kXpLo) return launchC_lo<T, NT, kXpLo>(jobs, bl, stage, step, tw, s);
+  if constexpr (xp_fits<T>(11, NT)) {  // (no smaller block holds a column)
+    if constexpr (sizeof(T) == 8)
+      if (lo == 11) return launchC_lo<T, NT, 11>(jobs, bl, stage, step, tw, s);
     launchC_lo<T, NT, 12>(jobs, bl, stage, step, tw, s);
+  }
 }
 
 template <typename T>
@@ -74,10 +77,13 @@ void launch_update(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int 
 
 template <typename T, int NT>
 static void prepareC(const BatchLaunch& bl, size_t lds) {
-  if (bl.lognx_max <= kXpLo)
-    MLV_SET_LDS_ONCE((k_stepC<T, NT, kXpLo>), lds);
-  else
-    MLV_SET_LDS_ONCE((k_stepC<T, NT, 12>), lds);
+  const int lo = xp_lo<T>(bl.lognx_max);
+  if (lo == kXpLo) MLV_SET_LDS_ONCE((k_stepC<T, NT, kXpLo>), lds);
+  if constexpr (xp_fits<T>(11, NT)) {
+    if constexpr (sizeof(T) == 8)
+      if (lo == 11) MLV_SET_LDS_ONCE((k_stepC<T, NT, 11>), lds);
+    if (lo == 12) MLV_SET_LDS_ONCE((k_stepC<T, NT, 12>), lds);
+  }
 }
 
 template <typename T>
