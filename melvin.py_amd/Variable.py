@@ -110,13 +110,13 @@ class Variable:
                     isinstance(u, torch.Tensor) and plain(u, pl.real, (pl.nx, pl.nz))
                     for u in (ux, uz)):
                 return self._advect(pl, ux, uz, convert_to_physical)
-            out = hip.zeros_like(self._pdata)
+            out = torch.empty_like(self._pdata)
         if convert_to_physical:
             self.to_physical()
         a = as_input(ux, pl.real, (pl.nx, pl.nz))
         b = as_input(uz, pl.real, (pl.nx, pl.nz))
         f = as_input(self._pdata, pl.real, (pl.nx, pl.nz))
-        dst = out if (out.is_contiguous() and out.dtype == pl.real) else hip.zeros_like(f)
+        dst = out if (out.is_contiguous() and out.dtype == pl.real) else torch.empty_like(f)
         _lib.call("mlv_flux_divergence", pl.handle, ptr(a), ptr(b), ptr(f), ptr(dst),
                   _lib.stream_handle())
         if dst is not out:
@@ -128,8 +128,9 @@ class Variable:
         as the plan's kernels take it, transformed by this package's own
         methods (a subclass or an instance may have others)."""
         bx, bz = self._basis_functions
-        return (type(self._st) is SpectralTransformer and self._st._plan is pl
-                and own(self._st, SpectralTransformer, "to_physical", "to_spectral")
+        st = self._st
+        return (type(st) is SpectralTransformer and st._plan is pl
+                and "to_physical" not in st.__dict__ and "to_spectral" not in st.__dict__
                 and own(self, Variable, "to_physical")
                 and bx is BasisFunctions.COMPLEX_EXP
                 and bz is (BasisFunctions.COMPLEX_EXP if pl.fully else BasisFunctions.FDM)
@@ -139,8 +140,10 @@ class Variable:
     def _own_pddz(self, pl):
         """Whether pddz is this package's difference of this field's own
         physical array."""
-        return (own(self, Variable, "pddz", "getp") and type(self._sd) is SpatialDifferentiator
-                and self._sd._plan is pl and own(self._sd, SpatialDifferentiator, "pddz", "_fd"))
+        sd = self._sd
+        return (type(sd) is SpatialDifferentiator and sd._plan is pl
+                and "pddz" not in sd.__dict__ and "_fd" not in sd.__dict__
+                and own(self, Variable, "pddz") and own(self, Variable, "getp"))
 
     def _advect(self, pl, ux, uz, convert_to_physical):
         """vec_dot_nabla whose flux divergence is formed inside the forward

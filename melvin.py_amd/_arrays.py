@@ -33,14 +33,14 @@ def output(out, dtype, shape, device=None):
 
 def plain(t, dtype, shape):
     """Whether a kernel can read and write ``t`` in place as such an array."""
-    return (t.is_cuda and t.dtype == dtype and tuple(t.shape) == tuple(shape)
-            and t.is_contiguous())
+    return t.is_cuda and t.dtype == dtype and t.shape == shape and t.is_contiguous()
 
 
-def own(obj, cls, *names):
-    """Whether these methods of ``obj`` are ``cls``'s: neither a subclass nor
-    the instance puts another in their place."""
-    return all(getattr(getattr(obj, n), "__func__", None) is getattr(cls, n) for n in names)
+def own(obj, cls, name):
+    """Whether this method of ``obj`` is ``cls``'s: neither a subclass nor the
+    instance puts another in its place."""
+    return ((type(obj) is cls or getattr(type(obj), name, None) is getattr(cls, name))
+            and name not in obj.__dict__)
 
 
 def finish(tmp, out):

@@ -49,15 +49,20 @@ def calc_velocity_from_vorticity(vorticity, streamfunction, ux, uz,
     if not (w.is_contiguous() and psi.is_contiguous()):
         raise ValueError("vorticity and streamfunction must be contiguous")
     fdm_z = streamfunction._basis_functions[1] is BasisFunctions.FDM
-    one = ((vorticity, streamfunction, ux, uz) if fdm_z or not pl.fully else (ux, uz))
-    # (FD z forms ux in place of ux.setp(-streamfunction.pddz()))
-    if (all(v._fourier(pl) for v in one)
-            and (not fdm_z or (streamfunction._own_pddz(pl) and own(ux, Variable, "setp")))
-            and plain(w, pl.cplx, (pl.rows, pl.cols))
-            and plain(psi, pl.cplx, (pl.rows, pl.cols))
-            and len({w.data_ptr(), psi.data_ptr(), ux._sdata.data_ptr(),
-                     uz._sdata.data_ptr()}) == 4
-            and len({v._pdata.data_ptr() for v in (streamfunction, ux, uz)}) == 3):
+    fused = (uz._fourier(pl) and plain(w, pl.cplx, (pl.rows, pl.cols))
+             and plain(psi, pl.cplx, (pl.rows, pl.cols)))
+    if fused and fdm_z:
+        # (ux is formed in place of ux.setp(-streamfunction.pddz()))
+        fused = (streamfunction._fourier(pl) and streamfunction._own_pddz(pl)
+                 and own(ux, Variable, "setp") and plain(ux._pdata, pl.real, (pl.nx, pl.nz))
+                 and len({w.data_ptr(), psi.data_ptr(), uz._sdata.data_ptr()}) == 3
+                 and len({v._pdata.data_ptr() for v in (streamfunction, ux, uz)}) == 3)
+    elif fused:
+        fused = (pl.fully and ux._fourier(pl)
+                 and len({w.data_ptr(), psi.data_ptr(), ux._sdata.data_ptr(),
+                          uz._sdata.data_ptr()}) == 4
+                 and ux._pdata.data_ptr() != uz._pdata.data_ptr())
+    if fused:
         _lib.call("mlv_velocity_physical", pl.handle, ptr(w), ptr(psi),
                   null if fdm_z else ptr(ux._sdata), ptr(uz._sdata),
                   ptr(streamfunction._pdata) if fdm_z else null, ptr(ux._pdata),
