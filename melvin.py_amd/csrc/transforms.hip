@@ -166,7 +166,58 @@ struct ZShape {
   static constexpr int N = 1 << LOGN, LOGE = tr_loge(LOGN), E = 1 << LOGE, TPS = N / E;
   static constexpr int SL = TPS >= 64 ? 1 : 64 / TPS, NT = SL * TPS;
   static constexpr int LDSN = rf_len(LOGN, LOGE);
+  // LDS elements a row pair: the transform's, or (STAGED) its coefficients,
+  // at most N + 2, or its points, padded
+  static constexpr int slot(bool staged) { return staged && N + 2 > LDSN ? N + 2 : LDSN; }
 };
+// Launches of many rows of at most 32 points (STAGED) pass them through LDS
+// on their way in and out: a wavefront holds 32 to 128 of them, and with each
+// thread loading its own row's points a load touches as many lines as it has
+// lanes.  Below this many rows the two more trips cost more than the lines
+// (us per launch, direct and staged, FP64 c2r, then FP32 r2c: 2^16 rows of 8
+// points 5.1 and 5.3, 5.0 and 4.2; of 16 7.3 and 6.6, 6.4 and 5.1; of 32 10.2
+// and 9.8, 6.5 and 6.2; 2^19 rows of 8 points 38 and 14, 21 and 8; 2^14 rows
+// 3.4 and 4.8, 3.3 and 3.8).
+constexpr int kStagedRows = 65536;
+template <int LOGN>
+static bool staged_rows(int rows) {
+  return LOGN <= 5 && rows >= kStagedRows;
+}
+
+// Position in LDS of the point n of row r of pair sl, rows of 2^LOGN points:
+// one spare element a pair, so that lanes on consecutive pairs differ in bank.
+template <int LOGN>
+__device__ __forceinline__ int pts_at(int sl, int r, int n) {
+  return sl * (2 << LOGN) + sl + (r << LOGN) + n;
+}
+// A block's run of `n` elements, at most MOST, between memory and LDS (PAD:
+// with the spare element after every 2^PAD), all of a thread's loads in
+// flight at once.
+template <int MOST, int NT, int PAD, typename V>
+__device__ __forceinline__ void run_load(const V* __restrict__ p, V* __restrict__ lds, int n) {
+  constexpr int IT = (MOST + NT - 1) / NT;
+  V v[IT];
+  // (unconditional, clamped: predicated element by element they are waited
+  // for one by one)
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int e = threadIdx.x + i * NT;
+    v[i] = p[e < n ? e : 0];
+  }
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int e = threadIdx.x + i * NT;
+    if (e < n) lds[PAD > 0 ? e + (e >> PAD) : e] = v[i];
+  }
+}
+template <int MOST, int NT, int PAD, typename V>
+__device__ __forceinline__ void run_store(V* __restrict__ p, const V* __restrict__ lds, int n) {
+#pragma unroll
+  for (int i = 0; i < (MOST + NT - 1) / NT; ++i) {
+    const int e = threadIdx.x + i * NT;
+    if (e < n) p[e] = lds[PAD > 0 ? e + (e >> PAD) : e];
+  }
+}
 
 // The packed spectrum a + i b at x of two real sequences whose coefficients
 // k < nk are at(k, a, b); zero beyond.
@@ -180,7 +231,7 @@ __device__ __forceinline__ cx<T> herm_at(int x, int N, int nk, F at) {
   return x == k ? mk<T>(a.x - b.y, a.y + b.x) : mk<T>(a.x + b.y, b.x - a.y);
 }
 
-template <typename T, int LOGN, bool PAIRS>
+template <typename T, int LOGN, bool PAIRS, bool STAGED>
 __global__ void __launch_bounds__((ZShape<LOGN>::NT))
     k_zc2r(const cx<T>* __restrict__ in0, const cx<T>* __restrict__ in1, T* __restrict__ out0,
            T* __restrict__ out1, int nx, int nm, T scale, const cx<T>* __restrict__ tw) {
@@ -190,24 +241,49 @@ __global__ void __launch_bounds__((ZShape<LOGN>::NT))
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw) + sl * S::LDSN;
   const cx<T>* __restrict__ in = blockIdx.y ? in1 : in0;
   T* __restrict__ out = blockIdx.y ? out1 : out0;
-  const int xa = 2 * (blockIdx.x * S::SL + sl), xb = xa + 1;
+  const int x0 = 2 * blockIdx.x * S::SL, xa = x0 + 2 * sl, xb = xa + 1;
   const bool live = xa < nx, two = xb < nx;
+  const int nrow = min(2 * S::SL, nx - x0);
   cx<T> v[S::E];
-  // (each coefficient is read for k and for N - k; the second read hits L1)
+  static_assert(!(PAIRS && STAGED), "rows in order");
+  if constexpr (STAGED) {
+    cx<T>* run = reinterpret_cast<cx<T>*>(smem_raw);
+    run_load<S::SL * (S::N + 2), S::NT, 0>(in + (size_t)x0 * nm, run, nrow * nm);
+    rf_sync<S::NT>();
 #pragma unroll
-  for (int m = 0; m < S::E; ++m)
-    v[m] = herm_at<T>(t + m * S::TPS, S::N, live ? nm : 0, [&](int k, cx<T>& a, cx<T>& b) {
-      if constexpr (PAIRS) {
-        const cx<T>* __restrict__ p = in + pair_at(xa, k, nm);
-        a = p[0];
-        b = p[1];
-      } else {
-        a = in[(size_t)xa * nm + k];
-        b = two ? in[(size_t)xb * nm + k] : czero<T>();
-      }
-    });
+    for (int m = 0; m < S::E; ++m)
+      v[m] = herm_at<T>(t + m * S::TPS, S::N, live ? nm : 0, [&](int k, cx<T>& a, cx<T>& b) {
+        a = run[2 * sl * nm + k];
+        b = two ? run[(2 * sl + 1) * nm + k] : czero<T>();
+      });
+    rf_sync<S::NT>();
+  } else {
+    // (each coefficient is read for k and for N - k; the second read hits L1)
+#pragma unroll
+    for (int m = 0; m < S::E; ++m)
+      v[m] = herm_at<T>(t + m * S::TPS, S::N, live ? nm : 0, [&](int k, cx<T>& a, cx<T>& b) {
+        if constexpr (PAIRS) {
+          const cx<T>* __restrict__ p = in + pair_at(xa, k, nm);
+          a = p[0];
+          b = p[1];
+        } else {
+          a = in[(size_t)xa * nm + k];
+          b = two ? in[(size_t)xb * nm + k] : czero<T>();
+        }
+      });
+  }
   rf_fft<T, LOGN, S::LOGE, +1, 1, S::NT>(v, lds, t, tw);
-  if (live) {
+  if constexpr (STAGED) {
+    T* pts = reinterpret_cast<T*>(smem_raw);
+    rf_sync<S::NT>();
+#pragma unroll
+    for (int m = 0; m < S::E; ++m) {
+      pts[pts_at<LOGN>(sl, 0, t + m * S::TPS)] = v[m].x * scale;
+      pts[pts_at<LOGN>(sl, 1, t + m * S::TPS)] = v[m].y * scale;
+    }
+    rf_sync<S::NT>();
+    run_store<2 * S::SL * S::N, S::NT, LOGN + 1>(out + (size_t)x0 * S::N, pts, nrow * S::N);
+  } else if (live) {
 #pragma unroll
     for (int m = 0; m < S::E; ++m) {
       const int n = t + m * S::TPS;
@@ -225,6 +301,7 @@ __global__ void __launch_bounds__((ZShape<LOGN>::NT))
 // positions on the other axis ("cross"), element (p, i) at p sp + i si.
 template <typename T>
 struct PlainSrc {
+  static constexpr bool PLAIN = true;
   const T* __restrict__ f;
   size_t sp, si;
   template <int LOGN, int LOGE, int STRIDE, int NT>
@@ -246,6 +323,7 @@ struct PlainSrc {
 // ORDER / 2 of its ends.
 template <typename T, int ORDER>
 struct FluxSrc {
+  static constexpr bool PLAIN = false;
   const T *__restrict__ uc, *__restrict__ uo, *__restrict__ f;
   size_t sp, si;
   int nc, per;
@@ -315,40 +393,68 @@ struct FluxSrc {
   }
 };
 
-template <typename T, int LOGN, bool PAIRS, typename Src>
+template <typename T, int LOGN, bool PAIRS, bool STAGED, typename Src>
 __global__ void __launch_bounds__((ZShape<LOGN>::NT))
     k_zr2c(Src src, cx<T>* __restrict__ out, int nx, int nm, const cx<T>* __restrict__ tw) {
   using S = ZShape<LOGN>;
   extern __shared__ char smem_raw[];
   const int sl = threadIdx.x / S::TPS, t = threadIdx.x % S::TPS;
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw) + sl * S::LDSN;
-  const int xa = 2 * (blockIdx.x * S::SL + sl), xb = xa + 1;
+  const int x0 = 2 * blockIdx.x * S::SL, xa = x0 + 2 * sl, xb = xa + 1;
   const bool live = xa < nx, two = xb < nx;
+  const int nrow = min(2 * S::SL, nx - x0);
   cx<T> v[S::E];
-  src.template load<LOGN, S::LOGE, 1, S::NT>(v, lds, t, xa, live, two);
+  if constexpr (STAGED) {
+    T* pts = reinterpret_cast<T*>(smem_raw);
+    run_load<2 * S::SL * S::N, S::NT, LOGN + 1>(src.f + (size_t)x0 * S::N, pts, nrow * S::N);
+    rf_sync<S::NT>();
+#pragma unroll
+    for (int m = 0; m < S::E; ++m)
+      v[m] = mk<T>(live ? pts[pts_at<LOGN>(sl, 0, t + m * S::TPS)] : T(0),
+                   two ? pts[pts_at<LOGN>(sl, 1, t + m * S::TPS)] : T(0));
+    rf_sync<S::NT>();
+  } else {
+    src.template load<LOGN, S::LOGE, 1, S::NT>(v, lds, t, xa, live, two);
+  }
   rf_fft<T, LOGN, S::LOGE, -1, 1, S::NT>(v, lds, t, tw);
   rf_sync<S::NT>();
 #pragma unroll
   for (int m = 0; m < S::E; ++m) lds[rf_pad<S::LOGE>(t, m * S::TPS)] = v[m];
   rf_sync<S::NT>();
   // coefficients k <= N / 2 of both rows (a half-spectrum ends at N / 2)
+  cx<T> va[S::E / 2 + 1], vb[S::E / 2 + 1];
 #pragma unroll
   for (int m = 0; m <= S::E / 2; ++m) {
     const int k = t + m * S::TPS;
     if (live && k < nm) {
       const cx<T> y = lds[rf_pad<S::LOGE>(t, m * S::TPS)];
       const cx<T> ym = lds[rf_mirror<LOGN, S::LOGE>(t, m)];
-      const cx<T> a = mk<T>(T(0.5) * (y.x + ym.x), T(0.5) * (y.y - ym.y));
-      const cx<T> b = mk<T>(T(0.5) * (y.y + ym.y), T(0.5) * (ym.x - y.x));
+      va[m] = mk<T>(T(0.5) * (y.x + ym.x), T(0.5) * (y.y - ym.y));
+      vb[m] = mk<T>(T(0.5) * (y.y + ym.y), T(0.5) * (ym.x - y.x));
+      if constexpr (STAGED) continue;
       if constexpr (PAIRS) {
         cx<T>* __restrict__ p = out + pair_at(xa, k, nm);
-        p[0] = a;
-        p[1] = b;
+        p[0] = va[m];
+        p[1] = vb[m];
       } else {
-        out[(size_t)xa * nm + k] = a;
-        if (two) out[(size_t)xb * nm + k] = b;
+        out[(size_t)xa * nm + k] = va[m];
+        if (two) out[(size_t)xb * nm + k] = vb[m];
       }
     }
+  }
+  if constexpr (STAGED) {
+    cx<T>* run = reinterpret_cast<cx<T>*>(smem_raw);
+    rf_sync<S::NT>();
+#pragma unroll
+    for (int m = 0; m <= S::E / 2; ++m) {
+      const int k = t + m * S::TPS;
+      if (live && k < nm) {
+        run[2 * sl * nm + k] = va[m];
+        if (two) run[(2 * sl + 1) * nm + k] = vb[m];
+      }
+    }
+    rf_sync<S::NT>();
+    run_store<S::SL * (S::N + 2), S::NT, 0>(out + (size_t)x0 * nm, run, nrow * nm);
   }
 }
 
@@ -437,22 +543,29 @@ __global__ void __launch_bounds__((XShape<LOGN, TC>::NT))
   return hipGetLastError()
 
 // Columns (or column pairs) per block of an x pass of `n` of them: two, or
-// four in single precision once that still leaves a block per CU: the rows
-// of a tile are then read in runs of 32 bytes instead of 16.
-template <typename T>
-static bool four_cols(int n) {
-  return sizeof(T) == 4 && n >= 4 * 256;
+// four once that still leaves a block per CU: the rows of a tile are then
+// read in runs of twice the length (FP64 inverse of 256 x 16384 reals 20.7 us a
+// call with two, 15.2 with four, 1024 x 4096 20.3 and 16.7).  Double precision
+// takes four up to 1024 points, beyond which they pass the LDS or the
+// registers, and not where it forms a flux, whose operands spill.
+template <typename T, bool FLUX>
+constexpr bool four_cols(int logn) {
+  return sizeof(T) == 4 || (logn <= 10 && !FLUX);
 }
 
 #define MLV_COLS(L, n, KERN, ...)                                                                 \
   do {                                                                                            \
-    if (four_cols<T>(n)) {                                                                        \
-      using S = XShape<L, 4>;                                                                     \
-      const size_t lds = tr_lds_bytes<T>(L, S::C);                                                \
-      const int nt = ((n) + S::C - 1) / S::C;                                                     \
-      MLV_SET_LDS_ONCE((KERN(L, 4)), lds);                                                        \
-      hipLaunchKernelGGL((KERN(L, 4)), dim3(xcd_grid(nt), ny), dim3(S::NT), lds, s, __VA_ARGS__, nt); \
-    } else {                                                                                      \
+    if constexpr (four_cols<T, flux>(L)) {                                                        \
+      if ((n) >= 4 * 256) {                                                                       \
+        using S = XShape<L, 4>;                                                                   \
+        const size_t lds = tr_lds_bytes<T>(L, S::C);                                              \
+        const int nt = ((n) + S::C - 1) / S::C;                                                   \
+        MLV_SET_LDS_ONCE((KERN(L, 4)), lds);                                                      \
+        hipLaunchKernelGGL((KERN(L, 4)), dim3(xcd_grid(nt), ny), dim3(S::NT), lds, s, __VA_ARGS__, nt); \
+        break;                                                                                    \
+      }                                                                                           \
+    }                                                                                             \
+    {                                                                                             \
       using S = XShape<L, 2>;                                                                     \
       const size_t lds = tr_lds_bytes<T>(L, S::C);                                                \
       const int nt = ((n) + S::C - 1) / S::C;                                                     \
@@ -461,10 +574,10 @@ static bool four_cols(int n) {
     }                                                                                             \
   } while (0)
 
-#define MLV_ROWS(L, KERN, ...)                                                                    \
+#define MLV_ROWS(L, STAGED, KERN, ...)                                                            \
   do {                                                                                            \
     using S = ZShape<L>;                                                                          \
-    const size_t lds = tr_lds_bytes<T>(L, S::SL);                                                 \
+    const size_t lds = (size_t)S::SL * S::slot(STAGED) * sizeof(cx<T>);                           \
     const int nb = ((nx + 1) / 2 + S::SL - 1) / S::SL;                                            \
     MLV_SET_LDS_ONCE((KERN(L)), lds);                                                             \
     hipLaunchKernelGGL((KERN(L)), dim3(nb, ny), dim3(S::NT), lds, s, __VA_ARGS__);                \
@@ -474,6 +587,7 @@ template <typename T>
 hipError_t launch_xinv(int logn, const void* in, void* out, int nn, int nm, const void* tw,
                        hipStream_t s, int nrow, double scale) {
   if (nrow < 0) nrow = 2 * nn + 1;
+  constexpr bool flux = false;
   const int ny = 1;
 #define KX(L, C) k_xinv<T, L, C>
 #define X(L)                                                                                \
@@ -489,6 +603,7 @@ hipError_t launch_xinv(int logn, const void* in, void* out, int nn, int nm, cons
 template <typename T>
 hipError_t launch_xinv_vel(int logn, const VelArgs& a, void* out, int nn, int nm, const void* tw,
                            hipStream_t s) {
+  constexpr bool flux = false;
   const int ny = 2;
 #define KX(L, C) k_xinv_vel<T, L, C>
 #define X(L)                                                                                \
@@ -505,6 +620,7 @@ template <typename T>
 hipError_t launch_xfwd(int logn, const void* in, void* out, int nn, int nm, double scale,
                        const void* tw, hipStream_t s, int nrow) {
   if (nrow < 0) nrow = 2 * nn + 1;
+  constexpr bool flux = false;
   const int ny = 1;
 #define KX(L, C) k_xfwd<T, L, C>
 #define X(L)                                                                                \
@@ -523,33 +639,45 @@ hipError_t launch_zc2r(int logn, const Two& a, int nx, int nm, const void* tw, h
   const int ny = a.n;
   const cx<T>*i0 = (const cx<T>*)a.in[0], *i1 = (const cx<T>*)a.in[1];
   T *o0 = (T*)a.out[0], *o1 = (T*)a.out[1];
-#define KP(L) k_zc2r<T, L, true>
-#define KR(L) k_zc2r<T, L, false>
+#define KP(L) k_zc2r<T, L, true, false>
+#define KR(L) k_zc2r<T, L, false, false>
+#define KS(L) k_zc2r<T, (L <= 5 ? L : 3), false, true>
 #define X(L)                                                                                \
   case L:                                                                                   \
     if (pairs)                                                                              \
-      MLV_ROWS(L, KP, i0, i1, o0, o1, nx, nm, (T)scale, (const cx<T>*)tw);                  \
+      MLV_ROWS(L, false, KP, i0, i1, o0, o1, nx, nm, (T)scale, (const cx<T>*)tw);           \
+    else if (staged_rows<L>(nx))                                                            \
+      MLV_ROWS(L, true, KS, i0, i1, o0, o1, nx, nm, (T)scale, (const cx<T>*)tw);            \
     else                                                                                    \
-      MLV_ROWS(L, KR, i0, i1, o0, o1, nx, nm, (T)scale, (const cx<T>*)tw);                  \
+      MLV_ROWS(L, false, KR, i0, i1, o0, o1, nx, nm, (T)scale, (const cx<T>*)tw);           \
     break;
   MLV_BY_LOGN(logn);
 #undef X
 #undef KP
 #undef KR
+#undef KS
 }
 
 template <typename T, bool PAIRS, typename Src>
 static hipError_t zr2c_src(int logn, const Src& src, void* out, int nx, int nm, const void* tw,
                            hipStream_t s) {
   const int ny = 1;
-#define KR(L) k_zr2c<T, L, PAIRS, Src>
+#define KR(L) k_zr2c<T, L, PAIRS, false, Src>
+#define KS(L) k_zr2c<T, (L <= 5 ? L : 3), false, true, PlainSrc<T>>
 #define X(L)                                                                                \
   case L:                                                                                   \
-    MLV_ROWS(L, KR, src, (cx<T>*)out, nx, nm, (const cx<T>*)tw);                            \
+    if constexpr (!PAIRS) {                                                                 \
+      if (staged_rows<L>(nx)) {                                                             \
+        MLV_ROWS(L, true, KS, src, (cx<T>*)out, nx, nm, (const cx<T>*)tw);                  \
+        break;                                                                              \
+      }                                                                                     \
+    }                                                                                       \
+    MLV_ROWS(L, false, KR, src, (cx<T>*)out, nx, nm, (const cx<T>*)tw);                     \
     break;
   MLV_BY_LOGN(logn);
 #undef X
 #undef KR
+#undef KS
 }
 
 // The flux source of a z pass (own axis z) or of an FD-z x pass (own axis x).
@@ -580,6 +708,7 @@ hipError_t launch_zr2c_flux(int logn, const FluxArgs& a, void* out, int nx, int 
 template <typename T>
 hipError_t launch_xc2r_cols(int logn, const Two& a, int nn, int nz, const void* tw, hipStream_t s,
                             double scale) {
+  constexpr bool flux = false;
   const int ny = a.n, np = (nz + 1) / 2;
 #define KX(L, C) k_xc2r_cols<T, L, C>
 #define X(L)                                                                                \
@@ -595,6 +724,7 @@ hipError_t launch_xc2r_cols(int logn, const Two& a, int nn, int nz, const void* 
 template <typename T, typename Src>
 static hipError_t xr2c_src(int logn, const Src& src, void* out, int nn, int nz, double scale,
                            const void* tw, hipStream_t s) {
+  constexpr bool flux = !Src::PLAIN;
   const int ny = 1, np = (nz + 1) / 2;
 #define KX(L, C) k_xr2c_cols<T, L, C, Src>
 #define X(L)                                                                                \
