@@ -281,22 +281,26 @@ int mlv_batch_graph_step(mlv_batch* batch, int nsteps, void* stream);
 int mlv_batch_set_dt(mlv_batch* batch, int job, double dt, void* stream);
 /* Pick each fused kernel's variant for this batch by measurement (the
  * tuning the reference leaves to its array library's FFT plans,
- * SpectralTransformer.py:58,85,132,191): kernel A's block shape (0: 512 threads in
- * single precision, 256 in double; 1: half that, where every job's x
- * transform fits; 2: shape 0's block holding two columns of every op of
- * the stage side by side, so the ops derived from one field read it once --
- * single precision, batches of one x size, 512 or 1024), kernel B's plan
- * (0: split-pass -- inverse 16,16,R with
- * the products in its last pass, forward R,16,16 -- where a job's z
- * transform takes it, else the two-sweep plan; 1: the two-sweep plan
- * everywhere) and kernel C's tile shape (0 narrow, 1 wide: 32 points per
- * thread where it applies, 2 narrow in 512-thread blocks: single
- * precision, batches of one x size in [512, 2048]).  Runs nsteps real steps with every kernel at
- * its first option, its second, .. up to the most options any kernel has,
- * then back down (half of nsteps per segment; a kernel with fewer options
- * stays at its first in the extra segments), with events around each
- * kernel, so the steps advance the simulations as mlv_batch_step would; a
- * kernel's option figure is its fastest segment per step.  Keeps each kernel's faster option and remembers the choice for
+ * SpectralTransformer.py:58,85,132,191): kernel A's block shape (0: blocks of
+ * up to 512 threads in single precision, 256 in double; 1: half of shape 0's;
+ * 2: blocks of 1024 holding two columns of every op of the stage side by
+ * side, so the ops derived from one field read it once -- single precision,
+ * batches of one x size, 512 or 1024), kernel B's plan (0: up to 1024 points in
+ * double precision a wavefront per channel, in registers; else, where a job's
+ * z transform takes it, inverse 16,16,R with the products in its last pass,
+ * forward R,16,16; else as 1: the inverse, the products and the forward
+ * transforms one after the other in LDS, at 512 points and above) and kernel
+ * C's tile shape (0 narrow: blocks of up to 256 threads; 1 wide: 512; 2: whole
+ * column groups with a wavefront per column -- single precision, batches of
+ * one x size, 512 or 1024; at 2048 accepted and the same as 1).  Launches that
+ * would leave the chip idle take smaller blocks in A's shapes 0 and 1 and C's
+ * shape 0; options that launch the same blocks are timed once.  Runs nsteps
+ * real steps with every kernel at its first option, its second, .. up to the
+ * most options any kernel has, then back down (half of nsteps per segment; a
+ * kernel with fewer options stays at its first in the extra segments), with
+ * events around each kernel, so the steps advance the simulations as
+ * mlv_batch_step would; a kernel's option figure is its fastest segment per
+ * step.  Keeps each kernel's faster option and remembers the choice for
  * batches created later for the same set of job shapes (process-wide).
  * chosen (3 ints, or NULL) receives {shape A, plan B, shape C}.  A's shapes
  * and C's shapes give bit-identical results; B's plans agree to rounding.

@@ -1151,10 +1151,15 @@ static int plan_batch_t(const mlv_job_desc* jobs, int njobs, int device, BatchPl
                        : a == 2 ? (r.nm + kMixCols - 1) / kMixCols
                                 : blocksA(r, s, bl.ntA[a]);
         P.pA[a][s][j + 1] = P.pA[a][s][j] + na;
-        P.pC[a][s][j + 1] = P.pC[a][s][j] + (on ? blocksC(r, s, bl.ntC[a]) : 0);
+        const bool group = a == 2 && bl.okC[2] && group_shape(bl.lognx_all);
+        const int nc = !on ? 0
+                       : group ? r.neq[s] * ((r.nm + kGroupCols - 1) / kGroupCols)
+                               : blocksC(r, s, bl.ntC[a]);
+        P.pC[a][s][j + 1] = P.pC[a][s][j] + nc;
         if (bl.okA[a])
           bl.ldsAp[a] = std::max(bl.ldsAp[a], xp_lds_bytes<T>(r.lognx, bl.ntA[a]));
-        bl.ldsCp[a] = std::max(bl.ldsCp[a], xp_lds_bytes<T>(r.lognx, bl.ntC[a]));
+        bl.ldsCp[a] = std::max(bl.ldsCp[a], group ? kGroupCols * group_len(r.lognx) * sizeof(cx<T>)
+                                                  : xp_lds_bytes<T>(r.lognx, bl.ntC[a]));
         if (on && J[j].split && bl.okA[a])
           bl.ldsAp[a] = std::max(bl.ldsAp[a], mean_lds_bytes(r.lognz, bl.ntA[a]));
       }
@@ -1200,11 +1205,14 @@ static int plan_batch_t(const mlv_job_desc* jobs, int njobs, int device, BatchPl
     }
   }
   bl.planB = kPlanSplit;
-  // defaults: 256-thread blocks in both kernels (single precision kernel A's
-  // shape 1: 38 against 43 us on a mixed batch up to 2048^2, 73 and 74 at 16 x
-  // 1024^2; FP64's shape 0 at 1024^2: 14.3 against 15.1)
+  // defaults: kernel A's 256-thread blocks in single precision (shape 1: 38
+  // against 43 us on a mixed batch up to 2048^2, 73 and 74 at 16 x 1024^2; FP64's
+  // shape 0 at 1024^2: 14.3 against 15.1)
   bl.shapeA = f64 ? 0 : 1;
-  bl.wideC = 0;
+  // Kernel C: shape 2 from two and a half blocks per CU on (shapes 0 and 2:
+  // 16 x 1024^2 with a scalar 145 and 138, 64 of them 527 and 496, 64 x 512^2
+  // 147 and 137; 4 x 1024^2 vortex 19.0 and 21.0, 1024^2 12.0 and 16.9).
+  bl.wideC = bl.okC[2] && group_shape(bl.lognx_all) && 2 * P.pC[2][0][njobs] >= 5 * cus ? 2 : 0;
   // choices picked by mlv_batch_autotune for the same set of jobs win
   P.signature = batch_signature(f64 ? MLV_F64 : MLV_F32, jobs, njobs);
   std::lock_guard<std::mutex> lk(g_tuned_mu);
@@ -1550,14 +1558,18 @@ int mlv_batch_autotune(mlv_batch* bp, int nsteps, void* stream, int* chosen) {
   // idle period, and a kernel's first launch, from deciding the choice.
   // The kernels read and write whole buffers in HBM between launches, so
   // one kernel's choice does not change another's time.
-  // the values each kernel can take
+  // the values each kernel can take, without those that launch the same blocks
+  // as another
+  const BatchLaunch& bl = b->bl;
   int opts[3][3], nopt[3] = {0, 0, 0};
-  for (int a = 0; a < 3; ++a)
-    if (b->bl.okA[a]) opts[0][nopt[0]++] = a;
+  opts[0][nopt[0]++] = 0;
+  if (bl.okA[1] && bl.ntA[1] != bl.ntA[0]) opts[0][nopt[0]++] = 1;
+  if (bl.okA[2]) opts[0][nopt[0]++] = 2;
   opts[1][nopt[1]++] = kPlanSplit;
-  if (b->bl.splitB) opts[1][nopt[1]++] = kPlanTwoSweep;
-  for (int c = 0; c < 3; ++c)
-    if (b->bl.okC[c]) opts[2][nopt[2]++] = c;
+  if (bl.splitB) opts[1][nopt[1]++] = kPlanTwoSweep;
+  opts[2][nopt[2]++] = 0;
+  if (bl.okC[1] && bl.ntC[1] != bl.ntC[0]) opts[2][nopt[2]++] = 1;
+  if (bl.okC[2] && group_shape(bl.lognx_all)) opts[2][nopt[2]++] = 2;
   const int maxopt = std::max(nopt[0], std::max(nopt[1], nopt[2]));
   const int h1 = nsteps >= 2 ? nsteps / 2 : nsteps, h2 = nsteps - h1;
   // option indices 0, 1, .., maxopt - 1, then back down

@@ -239,8 +239,8 @@ inline size_t mean_lds_bytes(int logn, int nt) {
 // (stepA_body's MIXED), single precision at 2^9 and 2^10 points with xmix_nt
 // threads, when kMixCols columns of every op of any stage fit the block.
 // Kernel C's tile shapes (BatchLaunch::wideC): 0 (narrow) of at most 256
-// threads, 1 (wide) and, single precision in a batch of one x size
-// (fixed_logn), 2, of 512.
+// threads; 1 (wide) of 512; 2, single precision in a batch of one x size, whole
+// column groups (group_shape; at 2^11 points shape 1's blocks).
 // "At most": a batch whose blocks would leave the chip idle takes smaller
 // ones (fill_threads in capi.cpp).
 constexpr int kMixCols = 2;
@@ -357,6 +357,18 @@ constexpr int kPGroup = 8;
 __host__ __device__ constexpr size_t pidx(int x, int k, int nx) {
   return (size_t)(k / kPGroup) * ((size_t)nx * kPGroup) + (size_t)x * kPGroup + (size_t)(k % kPGroup);
 }
+// Kernel C's shape 2 (stepC_body's GROUP): a group's columns per block, and a
+// column's points per thread (log2) and LDS elements.
+constexpr int kGroupCols = kPGroup;
+constexpr int kGroupPad = 4;  // spare elements a column: the eight differ in bank
+__host__ __device__ constexpr int group_loge(int logn) { return logn - 6; }
+__host__ __device__ constexpr int group_len(int logn) {
+  return rf_len(logn, group_loge(logn)) + kGroupPad;
+}
+// Sizes it is compiled for: 64 threads a column, and the transform's radices
+// (xp_loge) at most its points per thread.
+__host__ __device__ constexpr bool group_shape(int logn) { return logn == 9 || logn == 10; }
+
 // Elements per workspace channel: (nx, nm), nm rounded up to whole groups.
 __host__ __device__ constexpr size_t work_chs(int nx, int nm) {
   return (size_t)nx * (size_t)((nm + kPGroup - 1) / kPGroup * kPGroup);

@@ -17,6 +17,19 @@ __global__ void __launch_bounds__(NT)
   roleC<T, NT, LO>(jobs, clock, pref, njobs, lb, stage, step, tw, lds);
 }
 
+// Shape 2, for a batch whose jobs all have 2^LOGN points along x.
+template <int LOGN>
+__global__ void __launch_bounds__(64 * kGroupCols) __attribute__((amdgpu_waves_per_eu(4)))
+    k_stepC_group(const JobDev<float>* __restrict__ jobs, JobDev<float>* clock,
+                  const int* __restrict__ pref, int njobs, int stage, int step,
+                  const cx<float>* __restrict__ tw) {
+  extern __shared__ char smem_raw[];
+  cx<float>* lds = reinterpret_cast<cx<float>*>(smem_raw);
+  const int lb = xcd_logical(pref[njobs]);
+  if (lb < 0) return;
+  roleC_group<float, LOGN>(jobs, clock, pref, njobs, lb, stage, step, tw, lds);
+}
+
 template <typename T>
 __global__ void k_set_dt(JobDev<T>* jobs, int j, double dt) {
   if (threadIdx.x == 0 && blockIdx.x == 0) jobs[j].dt = dt;
@@ -63,10 +76,23 @@ static void launchC(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int
   }
 }
 
+template <int LOGN>
+static void launchC_group(const JobDev<float>* jobs, const BatchLaunch& bl, int stage, int step,
+                          const cx<float>* tw, hipStream_t s) {
+  MLV_SET_LDS_ONCE((k_stepC_group<LOGN>), bl.ldsC);
+  hipLaunchKernelGGL((k_stepC_group<LOGN>), dim3(xcd_grid(bl.nC[stage])), dim3(64 * kGroupCols),
+                     bl.ldsC, s, jobs, const_cast<JobDev<float>*>(jobs),
+                     (const int*)bl.prefC[stage], bl.njobs, stage, step, tw);
+}
+
 template <typename T>
 void launch_update(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int step,
                    const cx<T>* tw, hipStream_t s) {
   if (bl.nC[stage] == 0) return;
+  if constexpr (sizeof(T) == 4) {
+    if (bl.wideC == 2 && bl.lognx_all == 9) return launchC_group<9>(jobs, bl, stage, step, tw, s);
+    if (bl.wideC == 2 && bl.lognx_all == 10) return launchC_group<10>(jobs, bl, stage, step, tw, s);
+  }
   switch (bl.ntC[bl.wideC]) {
     case 64: return launchC<T, 64>(jobs, bl, stage, step, tw, s);
     case 128: return launchC<T, 128>(jobs, bl, stage, step, tw, s);
@@ -91,6 +117,13 @@ void prepare_update(const BatchLaunch& bl) {
   for (int c = 0; c < 3; ++c) {
     if (!bl.okC[c]) continue;
     const size_t lds = bl.ldsCp[c];
+    if constexpr (sizeof(T) == 4) {
+      if (c == 2 && group_shape(bl.lognx_all)) {
+        if (bl.lognx_all == 9) MLV_SET_LDS_ONCE((k_stepC_group<9>), lds);
+        if (bl.lognx_all == 10) MLV_SET_LDS_ONCE((k_stepC_group<10>), lds);
+        continue;
+      }
+    }
     if (bl.ntC[c] == 64) prepareC<T, 64>(bl, lds);
     if (bl.ntC[c] == 128) prepareC<T, 128>(bl, lds);
     if (bl.ntC[c] == 256) prepareC<T, 256>(bl, lds);

@@ -31,12 +31,26 @@ __device__ __forceinline__ T modk(const cx<T>* __restrict__ tw, int k, int logn,
 // 20.5 -> 18.6.  512-thread blocks, whose Px / Pz runs are twice as long,
 // measured 154 us at 16 x 1024^2 and 38.7 against 30.3 on a mixed batch of
 // double diffusion: more, shorter blocks hide each other's barriers.
-template <typename T, int LOGN, int NT>
+//
+// GROUP (shape 2: single precision, batches of one x size of 512 or 1024
+// points): blocks of a whole column group, 64 threads a column, one wavefront
+// per column from the transform on.  The group's rows are loaded and
+// differenced as above, pass through LDS to their columns' wavefronts and,
+// transformed with the same radices, through LDS again, to be updated row by
+// row: 512 bytes of each array at a time, four rows of a thread in flight
+// where its registers would hold two.  What bounds it: the launch's memory
+// traffic, once it is large: 64 x 1024^2 with a scalar 496 us (4.8 TB/s of its
+// 2.39 GB, where a copy reaches 5.2) against 527 in blocks of two columns,
+// which touch each group's lines four times over, and 16 of them 138 against
+// 145.  Below two and a half
+// blocks per CU the chain of one block is longer: 1024^2 16.9 against 12.0.
+template <typename T, int LOGN, int NT, bool GROUP = false>
 __device__ __forceinline__ void stepC_body(const JobDev<T>& J, const StageDev& S, int local, int cur,
                                            int par, const cx<T>* __restrict__ tw, cx<T>* lds) {
 #pragma clang fp contract(off)  // fused operations are spelled out (fma1)
-  constexpr int N = 1 << LOGN, LOGE = xp_loge<T>(LOGN), E = 1 << LOGE, TPS = N / E;
-  constexpr int TC = NT / TPS;
+  constexpr int N = 1 << LOGN, LOGE = GROUP ? group_loge(LOGN) : xp_loge<T>(LOGN);
+  constexpr int E = 1 << LOGE, TPS = N / E, TC = NT / TPS;
+  static_assert(!GROUP || (TPS == 64 && TC == kGroupCols), "a wavefront per column of a group");
   constexpr int nn = xp_nn(N), rows = 2 * nn + 1;
   const int nm = J.nm;
   const size_t chs = work_chs(N, nm);
@@ -45,7 +59,7 @@ __device__ __forceinline__ void stepC_body(const JobDev<T>& J, const StageDev& S
   const int eqi = local / ntile, tile = local % ntile;
   const int field = S.eq_field[eqi];
   const int c = threadIdx.x % TC, t = TPS == 1 ? 0 : threadIdx.x / TC;
-  const int col = tile * TC + c;
+  int col = tile * TC + c;
   const bool cok = col < nm;
   const cx<T>* __restrict__ pxc = glb(J.work) + (size_t)pchan(J.pbase, eqi, 0) * chs;
   const cx<T>* __restrict__ pzc = glb(J.work) + (size_t)pchan(J.pbase, eqi, 1) * chs;
@@ -64,13 +78,15 @@ __device__ __forceinline__ void stepC_body(const JobDev<T>& J, const StageDev& S
     zv[m] = at32(pzc, o);
   }
   const T szc = modk<T>(tw, cok ? col : 0, J.lognz, order, J.dz);
-  cx<T>* __restrict__ slot = lds + c;
+  // a column's elements in LDS, beside the other columns' or (GROUP) apart
+  constexpr int SD = GROUP ? 1 : TC;
+  cx<T>* __restrict__ slot = lds + (GROUP ? c * group_len(LOGN) : c);
 #pragma unroll
-  for (int m = 0; m < E; ++m) slot[rf_pad<LOGE>(t, m * TPS) * TC] = v[m];
+  for (int m = 0; m < E; ++m) slot[rf_pad<LOGE>(t, m * TPS) * SD] = v[m];
   rf_sync<NT>();
 #pragma unroll
   for (int m = 0; m < E; ++m) {
-    auto at = [&](int d) { return slot[rf_near<LOGN, LOGE>(t, m, d) * TC]; };
+    auto at = [&](int d) { return slot[rf_near<LOGN, LOGE>(t, m, d) * SD]; };
     const cx<T> a1 = at(1), b1 = at(-1);
     cx<T> d;
     if (order == 2) {
@@ -83,8 +99,28 @@ __device__ __forceinline__ void stepC_body(const JobDev<T>& J, const StageDev& S
     v[m] = mk<T>(fma1(-szc, zv[m].y, d.x), fma1(szc, zv[m].x, d.y));
   }
   rf_sync<NT>();
-  rf_fft<T, LOGN, LOGE, -1, TC, NT>(v, slot, t, tw);
-  if (!cok) return;
+  const int lane = threadIdx.x & 63;
+  if constexpr (GROUP) {
+#pragma unroll
+    for (int m = 0; m < E; ++m) slot[rf_pad<LOGE>(t, m * TPS)] = v[m];
+    rf_sync<NT>();
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    col = tile * TC + wv;
+    if (col >= nm) return;
+    slot = lds + wv * group_len(LOGN);
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = slot[rf_pad<LOGE>(lane, m * TPS)];
+    rf_sync<64>();
+    rf_fft<T, LOGN, LOGE, -1, 1, 64, xp_loge<T>(LOGN)>(v, slot, lane, tw);
+    rf_sync<64>();
+#pragma unroll
+    for (int m = 0; m < E; ++m)
+      if (xp_any(m, TPS, N)) slot[rf_pad<LOGE>(lane, m * TPS)] = v[m];
+    rf_sync<64>();
+  } else {
+    rf_fft<T, LOGN, LOGE, -1, TC, NT>(v, slot, t, tw);
+    if (!cok) return;
+  }
 
   const int q = J.q;
   const double dt = J.dt, alpha = J.alpha;
@@ -108,17 +144,24 @@ __device__ __forceinline__ void stepC_body(const JobDev<T>& J, const StageDev& S
   const uint32_t cbase = (uint32_t)col * rows;
   // rows updated U at a time, their loads issued before any is used (single
   // precision: all of them at once spill, 176 against 150 us at 16 x 1024^2)
-  constexpr int U = E >= 16 && sizeof(T) == 4 ? 2 : 4;
-#pragma unroll
-  for (int m0 = 0; m0 < E; m0 += U) {
+  constexpr int U = E >= 16 && sizeof(T) == 4 && !GROUP ? 2 : 4;
+  // row groups: the points a thread holds, or runs of 64 rows
+  constexpr int G = GROUP ? (rows + 63) / 64 : E;
+  auto any = [](int m) { return GROUP || xp_any(m, TPS, N); };
+  auto row_of = [&](int m) {
+    if constexpr (GROUP) return lane + 64 * m < rows ? lane + 64 * m : -1;
+    else return xp_row(t + m * TPS, N);
+  };
+#pragma unroll(GROUP ? 1 : E)
+  for (int m0 = 0; m0 < G; m0 += U) {
     // (a group's loads stay behind the group before: hoisted, they spill)
     if constexpr (sizeof(T) == 4) __builtin_amdgcn_sched_barrier(0);
     cx<T> vv[U], h1[U], h2[U], h3[U], e1[U], e2[U];
     uint32_t lo[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (!xp_any(m0 + u, TPS, N)) continue;
-      const int r = xp_row(t + (m0 + u) * TPS, N);
+      if (!any(m0 + u)) continue;
+      const int r = row_of(m0 + u);
       if (r < 0) continue;
       const uint32_t o = (cbase + r) * (uint32_t)sizeof(cx<T>);
       vv[u] = at32(sin_, o);
@@ -133,12 +176,16 @@ __device__ __forceinline__ void stepC_body(const JobDev<T>& J, const StageDev& S
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (!xp_any(m0 + u, TPS, N)) continue;
-      const int r = xp_row(t + (m0 + u) * TPS, N);
+      if (!any(m0 + u)) continue;
+      const int r = row_of(m0 + u);
       if (r < 0) continue;
       const int n = r <= nn ? r : r - rows, m = col;
       const uint32_t o = (cbase + r) * (uint32_t)sizeof(cx<T>);
-      const cx<T> D = v[m0 + u];
+      cx<T> D;
+      if constexpr (GROUP)
+        D = slot[rf_pad<LOGE>(r <= nn ? r : r + N - rows)];
+      else
+        D = v[m0 + u];
       cx<T> rhs = mk<T>(D.x * scale, D.y * scale);
       if (ddc) {
         const double Pr = J.param[0], R0 = J.param[1];
@@ -238,6 +285,23 @@ __device__ __forceinline__ void roleC(const JobDev<T>* __restrict__ jobs, JobDev
     default:
       break;
   }
+}
+
+// Shape 2's work for logical block lb, in a batch of 2^LOGN points along x.
+template <typename T, int LOGN>
+__device__ __forceinline__ void roleC_group(const JobDev<T>* __restrict__ jobs, JobDev<T>* clock,
+                                            const int* __restrict__ pref, int njobs, int lb,
+                                            int stage, int step, const cx<T>* __restrict__ tw,
+                                            cx<T>* lds) {
+  const int j = find_job(pref, njobs, lb);
+  const JobDev<T>& J = jobs[j];
+  const int local = lb - pref[j];
+  if (stage == J.nstage - 1 && local == 0 && threadIdx.x == 0) {
+    clock[j].t = clock[j].t + J.dt;
+    clock[j].loops = clock[j].loops + 1;
+  }
+  stepC_body<T, LOGN, 64 * kGroupCols, true>(J, J.st[stage], local, ring(J.curr0, step, J.q),
+                                             (J.par0 + step) & 1, tw, lds);
 }
 
 }  // namespace mlv

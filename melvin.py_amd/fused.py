@@ -350,10 +350,10 @@ class Batch(DeviceRun):
         _lib.call("mlv_batch_set_dt", self.handle, int(index), float(dt),
                   _lib.stream_handle(stream))
 
-    # names of the kernel choices (mlv_batch_autotune)
-    _SHAPE_A = ("512 threads", "256 threads", "512 threads, mixed ops")
+    # names of the kernel choices (mlv_batch_autotune says what each runs)
+    _SHAPE_A = ("full blocks", "half blocks", "mixed ops")
     _PLAN_B = ("split-pass", "two-sweep")
-    _SHAPE_C = ("narrow", "wide", "narrow, 512 threads")
+    _SHAPE_C = ("narrow", "wide", "column groups")
 
     def _advance(self, n):
         for j in self.jobs:
@@ -365,8 +365,8 @@ class Batch(DeviceRun):
     def autotune(self, steps=4, stream=None):
         """Pick each fused kernel's variant by timing ``steps`` real steps
         with each option (mlv_batch_autotune); the jobs advance by 2 * steps
-        (3 * steps where the x-inverse has three shapes).  Returns the
-        chosen plan (see ``plan``)."""
+        (3 * steps where a kernel has three options).  Returns the chosen
+        plan (see ``plan``)."""
         chosen = (ctypes.c_int * 3)()
         before = _lib.lib().mlv_batch_steps(self.handle)
         _lib.call("mlv_batch_autotune", self.handle, int(steps), _lib.stream_handle(stream), chosen)
@@ -379,9 +379,7 @@ class Batch(DeviceRun):
         tile shape, and which alternatives this job set admits."""
         p = (ctypes.c_int * 7)()
         _lib.call("mlv_batch_plan", self.handle, p)
-        double = self.jobs[0].dtype == "f64"
-        shape_a = ("256 threads", "128 threads", "256 threads, mixed ops") if double else self._SHAPE_A
-        return {"x_inverse": shape_a[p[0]], "z_pass": self._PLAN_B[p[1]],
+        return {"x_inverse": self._SHAPE_A[p[0]], "z_pass": self._PLAN_B[p[1]],
                 "x_forward_update": self._SHAPE_C[p[2]],
                 "x_inverse_small_block_available": bool(p[3]),
                 "z_pass_split_available": bool(p[4]),
