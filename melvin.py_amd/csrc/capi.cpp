@@ -1205,10 +1205,17 @@ static int plan_batch_t(const mlv_job_desc* jobs, int njobs, int device, BatchPl
     }
   }
   bl.planB = kPlanSplit;
-  // defaults: kernel A's 256-thread blocks in single precision (shape 1: 38
-  // against 43 us on a mixed batch up to 2048^2, 73 and 74 at 16 x 1024^2; FP64's
-  // shape 0 at 1024^2: 14.3 against 15.1)
-  bl.shapeA = f64 ? 0 : 1;
+  // Kernel A, single precision: shape 1 (half of shape 0's block) while it
+  // still holds two columns and the launch is not large; shape 0 from ten
+  // blocks per CU on where shape 1's columns are fewer than fill a line, which
+  // neighbouring blocks then fetch again (us per launch, shapes 0 and 1: mixed
+  // vortex batch up to 2048^2 43.0 and 38.9, 2048^2 25.0 and 21.3, 64 x 256^2
+  // 20.5 and 18.5; 64 x 1024^2 288 and 295, 4 x 2048^2 with a scalar 79 and 87,
+  // 64 x 512^2 double diffusion 91 and 96; one column a block: 1024^2 with a
+  // scalar 12.1 and 12.6, double diffusion 13.1 and 14.2).  Double precision's
+  // shape 0 at 1024^2: 14.3 against 15.1.
+  const bool whole = xp_cols<T>(bl.lognx_max, bl.ntA[1]) >= 8;
+  bl.shapeA = !f64 && bl.ntA[1] >= two && (whole || total(blocksA, bl.ntA[0]) < 10 * cus) ? 1 : 0;
   // Kernel C: shape 2 from two and a half blocks per CU on (shapes 0 and 2:
   // 16 x 1024^2 with a scalar 145 and 138, 64 of them 527 and 496, 64 x 512^2
   // 147 and 137; 4 x 1024^2 vortex 19.0 and 21.0, 1024^2 12.0 and 16.9).

@@ -1,7 +1,10 @@
 """The single-precision update in blocks of a whole column group (shape 2, x
 sizes of 512 and 1024) gives the other shapes' bits: column counts that fill
 their last group and that do not, both orders, every problem, with and without
-the carry, several jobs of different z sizes."""
+the carry, several jobs of different z sizes; and the shapes that a batch
+starts with."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -55,3 +58,25 @@ def test_group_update_of_mixed_z_sizes(mlv, ab, compensated):
     for a, b in zip(got, want):
         for x, y in zip(a, b):
             np.testing.assert_array_equal(x, y)
+
+
+def _default_plan(mlv, sizes, problem="vorticity", coeff=(1e-3, 1e-3)):
+    jobs = [mlv.fused.Job(problem, n, n, 2.0, 2.0, dtype="f32", coeff=coeff, param=[7.0, 1.5])
+            for n in sizes]
+    b = mlv.fused.Batch(jobs)
+    p = (ctypes.c_int * 7)()
+    mlv._lib.call("mlv_batch_plan", b.handle, p)
+    b.close()
+    return p[0], p[2]
+
+
+def test_default_shapes(mlv):
+    """(x-inverse, update): one column a block is not taken, nor the smaller
+    x-inverse block on a large launch of partial lines."""
+    ddc = dict(problem="ddc", coeff=(7.0, 1.0, 0.01))
+    assert _default_plan(mlv, [512]) == (0, 0)
+    assert _default_plan(mlv, [1024]) == (0, 0)
+    assert _default_plan(mlv, [2048, 256, 512, 256]) == (1, 0)
+    assert _default_plan(mlv, [256] * 64) == (1, 0)
+    assert _default_plan(mlv, [512] * 64, **ddc) == (0, 2)
+    assert _default_plan(mlv, [1024] * 16) == (0, 2)
