@@ -180,6 +180,8 @@ int create_impl(FdzHost* b, const mlv_fdz_job_desc* jobs, int njobs) {
     FdzJob<T>& J = host_job<T>(b, j);
     int rc = build_fdz_job<T>(jobs[j], J, j);
     if (rc) return rc;
+    const int var = fdz_row_var(J.K, J.wpr);
+    fl.rowvar = (j == 0 || fl.rowvar == var) && var < kFdzRowVars - 1 ? var : -1;
     const int size = fdz_col_size(J.lognx);
     const size_t ldsc = fdz_cols_lds_bytes<T>(J.lognx);
     if (ldsc > lds_max)

@@ -351,13 +351,17 @@ __device__ __forceinline__ void fdz_row(const FdzJob<T>& J, int stage, int n, in
 
 // Blocks of 128 threads: two rows of one wavefront, or one row of two.  One
 // launch runs every job's rows, each wavefront taking the branch of its job's
-// K.  (A launch per K left a batch of ragged sizes with up to five launches
-// that each filled a fraction of the chip: six FP64 jobs of nz 33 to 257 took
-// 39.6 us of row kernels per step, 14.4 in one launch.  The kernel holds 124
-// VGPRs: reading all operands and factors up front costs 149 and a wavefront
-// per SIMD, 81.8 against 75.9 us for eight jobs of 1024x513, with no gain for
-// one.)
-template <typename T>
+// variant (fdz_row_var).  (A launch per variant left a batch of ragged sizes
+// with up to five launches that each filled a fraction of the chip: six FP64
+// jobs of nz 33 to 257 took 39.6 us of row kernels per step, 14.4 in one
+// launch.  The kernel holds 124 VGPRs: reading all operands and factors up
+// front costs 149 and a wavefront per SIMD, 81.8 against 75.9 us for eight jobs
+// of 1024x513, with no gain for one.)
+// VAR >= 0: a batch of one variant runs the kernel compiled for it alone, whose
+// 68 to 98 VGPRs leave room for a wavefront or three more per SIMD (us per
+// launch, all variants' kernel and its own: 100 FP32 jobs of 256x129 47.6 and
+// 42.5, 16 of 2048x17 31.9 and 25.3, 64 of 256x257 96 and 85).
+template <typename T, int VAR>
 __global__ void __launch_bounds__(kFdzRowThreads)
     k_fdz_rows(const FdzJob<T>* __restrict__ jobs, FdzJob<T>* clock, const int* __restrict__ pref,
                int njobs, int phase, int step, const double2* __restrict__ tw64) {
@@ -367,7 +371,7 @@ __global__ void __launch_bounds__(kFdzRowThreads)
   if (lb < 0) return;
   const int jb = find_job(pref, njobs, lb);
   const FdzJob<T>& J = jobs[jb];
-  const int wpr = J.wpr, lr = 64 * wpr;
+  const int wpr = VAR >= 0 ? kFdzRowWpr[VAR < 0 ? 0 : VAR] : J.wpr, lr = 64 * wpr;
   const int rib = threadIdx.x / lr, t = threadIdx.x % lr;  // row in block, thread in row
   const int lw = (lb - pref[jb]) * fdz_rows_per_block(wpr) + rib;
   int stage, nwf;
@@ -391,7 +395,9 @@ __global__ void __launch_bounds__(kFdzRowThreads)
   double2* buf = reinterpret_cast<double2*>(smem_raw) + (size_t)(2 * rib) * zstride;
   double2* vrow = buf + zstride;
 #define MLV_ROW(KT, WPR) fdz_row<T, KT, WPR>(J, stage, n, f, step, buf, vrow, t, tot, tw64)
-  if (wpr == 1) {
+  if constexpr (VAR >= 0) {
+    MLV_ROW(kFdzRowKt[VAR], kFdzRowWpr[VAR]);
+  } else if (wpr == 1) {
     if (J.K <= 1)
       MLV_ROW(1, 1);
     else if (J.K <= 2)
@@ -756,15 +762,29 @@ __global__ void k_fdz_set_dt(FdzJob<T>* jobs, int j, double dt, double lo_w, dou
 // --------------------------------------------------------------------------
 // Host side
 // --------------------------------------------------------------------------
+template <typename T, int VAR>
+static void launch_rows_var(const FdzJob<T>* jobs, const FdzLaunch& fl, int phase, int step,
+                            hipStream_t s) {
+  const int p = phase < 0 ? 2 : phase;
+  MLV_SET_LDS_ONCE((k_fdz_rows<T, VAR>), fl.ldsrow);
+  hipLaunchKernelGGL((k_fdz_rows<T, VAR>), dim3(xcd_grid(fl.nrow[p])), dim3(kFdzRowThreads),
+                     fl.ldsrow, s, jobs, const_cast<FdzJob<T>*>(jobs), (const int*)fl.prefrow[p],
+                     fl.njobs, phase, step, fl.tw64);
+}
+
+#define MLV_ROW_VARS(X) X(-1) X(0) X(1) X(2) X(3)
+
 template <typename T>
 static void launch_rows(const FdzJob<T>* jobs, const FdzLaunch& fl, int phase, int step,
                         hipStream_t s) {
-  const int p = phase < 0 ? 2 : phase;
-  if (fl.nrow[p] <= 0) return;
-  MLV_SET_LDS_ONCE(k_fdz_rows<T>, fl.ldsrow);
-  hipLaunchKernelGGL(k_fdz_rows<T>, dim3(xcd_grid(fl.nrow[p])), dim3(kFdzRowThreads), fl.ldsrow, s,
-                     jobs, const_cast<FdzJob<T>*>(jobs), (const int*)fl.prefrow[p], fl.njobs,
-                     phase, step, fl.tw64);
+  if (fl.nrow[phase < 0 ? 2 : phase] <= 0) return;
+  switch (fl.rowvar) {
+#define X(V) \
+  case V: return launch_rows_var<T, V>(jobs, fl, phase, step, s);
+    MLV_ROW_VARS(X)
+#undef X
+    default: break;
+  }
 }
 
 // Column blocks of the jobs whose blocks have NT threads.
@@ -824,7 +844,15 @@ template <typename T>
 hipError_t fdz_prepare(const FdzLaunch& fl) {
   if (fl.ldscol[0]) MLV_SET_LDS_ONCE((k_fdz_cols<T, 256>), fl.ldscol[0]);
   if (fl.ldscol[1]) MLV_SET_LDS_ONCE((k_fdz_cols<T, 512>), fl.ldscol[1]);
-  MLV_SET_LDS_ONCE(k_fdz_rows<T>, fl.ldsrow);
+  switch (fl.rowvar) {
+#define X(V)                                             \
+  case V:                                                \
+    MLV_SET_LDS_ONCE((k_fdz_rows<T, V>), fl.ldsrow);     \
+    break;
+    MLV_ROW_VARS(X)
+#undef X
+    default: break;
+  }
   return hipGetLastError();
 }
 

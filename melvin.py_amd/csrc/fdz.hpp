@@ -49,6 +49,14 @@ constexpr int kFdzRowThreads = 128;
 constexpr int kFdzMaxNz = 768;
 __host__ __device__ constexpr int fdz_wpr(int nz) { return nz > 256 ? 2 : 1; }
 __host__ __device__ constexpr int fdz_rows_per_block(int wpr) { return 2 / wpr; }
+// Compiled variants of a row: elements per lane at most, wavefronts per row;
+// a job's is the smallest that holds it.
+constexpr int kFdzRowVars = 5;
+constexpr int kFdzRowKt[kFdzRowVars] = {1, 2, 4, 4, 6};
+constexpr int kFdzRowWpr[kFdzRowVars] = {1, 1, 1, 2, 2};
+__host__ __device__ constexpr int fdz_row_var(int K, int wpr) {
+  return wpr == 1 ? (K <= 1 ? 0 : K <= 2 ? 1 : 2) : (K <= 4 ? 3 : 4);
+}
 
 template <typename T>
 struct FdzJob {
@@ -103,6 +111,10 @@ struct FdzLaunch {
   int njobs;
   int ncol[kFdzColSizes][2];         // column blocks of 256 and 512 threads, phases 0 and 1
   int nrow[3];                       // row blocks of phases 0, 1 and the prologue
+  // the row variant of every job; -1 when they differ, and for the largest,
+  // which gains no wavefront in a kernel of its own (eight 1024x513 FP32 jobs
+  // 249 us a step in all variants' kernel, 255 in its own)
+  int rowvar;
   size_t ldsrow, ldscol[kFdzColSizes];
   const double2* tw64;               // FP64 twiddles exp(-2 pi i k / NMAX)
   int *prefcol[kFdzColSizes][2];
