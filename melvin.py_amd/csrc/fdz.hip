@@ -471,7 +471,7 @@ __device__ __forceinline__ void fdz_cols_body(const FdzJob<T>& J, int local, int
   const bool corr = J.scheme == MLV_FDZ_PC && phase == 1;
   const int vs = corr ? 2 : par;
   const int f = __builtin_amdgcn_readfirstlane(threadIdx.x / GT);
-  const int g = threadIdx.x % GT, sub = g % PB, t = TPS == 1 ? 0 : g / PB;
+  const int g = threadIdx.x % GT, sub = g % PB, t = rf_thread<TPS>(g / PB);
   const int c0 = 2 * (local * PB + sub);  // the pair's first column
   const bool live = c0 < Z, two = c0 + 1 < Z;
   auto region = [&](int fld, int sb) { return lds + fld * REG + sb; };

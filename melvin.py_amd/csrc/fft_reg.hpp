@@ -68,6 +68,15 @@ __host__ __device__ constexpr int rf_len(int logn, int loge) {
   return (1 << logn) + ((1 << logn) >> loge);
 }
 
+// A transform's thread among TPS, from its index.  Spelled out as 0 where it
+// is the only one: with the index only known to be 0 from its range, the
+// compiler drops n from the test "n == 0 and column 0" of a row n = t - 1 (the
+// x inverse at 8 points: its assembly tests the column alone).
+template <int TPS>
+__device__ __forceinline__ int rf_thread(int t) {
+  return TPS == 1 ? 0 : t;
+}
+
 // Synchronisation of the threads that share LDS: a block of one wavefront
 // needs no barrier.
 template <int NT>

@@ -58,7 +58,7 @@ __device__ __forceinline__ void stepC_body(const JobDev<T>& J, const StageDev& S
   const int ntile = (nm + TC - 1) / TC;
   const int eqi = local / ntile, tile = local % ntile;
   const int field = S.eq_field[eqi];
-  const int c = threadIdx.x % TC, t = TPS == 1 ? 0 : threadIdx.x / TC;
+  const int c = threadIdx.x % TC, t = rf_thread<TPS>(threadIdx.x / TC);
   int col = tile * TC + c;
   const bool cok = col < nm;
   const cx<T>* __restrict__ pxc = glb(J.work) + (size_t)pchan(J.pbase, eqi, 0) * chs;

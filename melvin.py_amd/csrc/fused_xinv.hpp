@@ -59,9 +59,7 @@ __device__ __forceinline__ void stepA_body(const JobDev<T>& J, const StageDev& S
   constexpr int TC = NT / TPS;
   constexpr int nn = xp_nn(N), rows = 2 * nn + 1;
   const int nm = J.nm;
-  const int c = threadIdx.x % TC, t = TPS == 1 ? 0 : threadIdx.x / TC;
-  // (t is spelled out as 0 at N = 8: where the compiler only knows its range
-  // to be 0, it folds n == 0 wrongly for n = t - 1)
+  const int c = threadIdx.x % TC, t = rf_thread<TPS>(threadIdx.x / TC);
   int opi, col;
   bool ok;
   if constexpr (MIXED) {

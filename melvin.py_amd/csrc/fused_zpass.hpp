@@ -97,7 +97,7 @@ __device__ __forceinline__ void stepZ_body(const JobDev<T>& J, const StageDev& S
   const int nx = J.nx;
   const uint32_t chs = (uint32_t)work_chs(nx, nm);
   const int ch = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63, sub = lane / TPS, t = TPS == 1 ? 0 : lane % TPS;
+  const int lane = threadIdx.x & 63, sub = lane / TPS, t = rf_thread<TPS>(lane % TPS);
   const int x0 = 2 * (local * PB + sub);
   const bool live = x0 < nx;
   auto region = [&](int c, int sb) { return lds + (c * PB + sb) * LDSN; };

@@ -62,7 +62,7 @@ __global__ void __launch_bounds__((XShape<LOGN, TC>::NT))
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int tile = xcd_logical(ntile);
   if (tile < 0) return;
-  const int c = threadIdx.x % S::C, t = threadIdx.x / S::C;
+  const int c = threadIdx.x % S::C, t = rf_thread<S::TPS>(threadIdx.x / S::C);
   const int col = tile * S::C + c;
   cx<T> v[S::E];
 #pragma unroll
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__((XShape<LOGN, TC>::NT))
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int tile = xcd_logical(ntile);
   if (tile < 0) return;
-  const int c = threadIdx.x % S::C, t = threadIdx.x / S::C;
+  const int c = threadIdx.x % S::C, t = rf_thread<S::TPS>(threadIdx.x / S::C);
   const int col = tile * S::C + c, rows = 2 * nn + 1;
   const bool isz = blockIdx.y != 0;
   cx<T> v[S::E];
@@ -143,7 +143,7 @@ __global__ void __launch_bounds__((XShape<LOGN, TC>::NT))
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int tile = xcd_logical(ntile);
   if (tile < 0) return;
-  const int c = threadIdx.x % S::C, t = threadIdx.x / S::C;
+  const int c = threadIdx.x % S::C, t = rf_thread<S::TPS>(threadIdx.x / S::C);
   const int col = tile * S::C + c;
   cx<T> v[S::E];
 #pragma unroll
@@ -474,7 +474,7 @@ __global__ void __launch_bounds__((XShape<LOGN, TC>::NT))
   if (tile < 0) return;
   const cx<T>* __restrict__ in = blockIdx.y ? in1 : in0;
   T* __restrict__ out = blockIdx.y ? out1 : out0;
-  const int c = threadIdx.x % S::C, t = threadIdx.x / S::C;
+  const int c = threadIdx.x % S::C, t = rf_thread<S::TPS>(threadIdx.x / S::C);
   const int za = 2 * (tile * S::C + c);
   const bool live = za < nz, two = za + 1 < nz;
   cx<T> v[S::E];
@@ -504,7 +504,7 @@ __global__ void __launch_bounds__((XShape<LOGN, TC>::NT))
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int tile = xcd_logical(ntile);
   if (tile < 0) return;
-  const int c = threadIdx.x % S::C, t = threadIdx.x / S::C;
+  const int c = threadIdx.x % S::C, t = rf_thread<S::TPS>(threadIdx.x / S::C);
   const int za = 2 * (tile * S::C + c);
   const bool live = za < nz, two = za + 1 < nz;
   cx<T> v[S::E];
