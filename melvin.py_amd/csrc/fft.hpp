@@ -275,18 +275,4 @@ __host__ __device__ constexpr int fft_slots() {
   return (NT * P) >> LOGN;
 }
 
-// Points per thread.  Column passes (along x, strided) want enough slots per
-// block that every row is read in runs of at least 64 bytes (8 float or 4
-// double complex values), so single precision uses 32 points from N = 1024.
-// Row passes read contiguous rows and keep 16 points up to N = 1024, which
-// leaves more blocks and a smaller register file.
-template <typename T>
-__host__ __device__ constexpr int fft_points_col(int logn) {
-  return sizeof(T) == 4 ? (logn >= 10 ? 32 : 16) : (logn >= 11 ? 32 : 16);
-}
-template <typename T>
-__host__ __device__ constexpr int fft_points_row(int logn) {
-  return logn >= 11 ? 32 : 16;
-}
-
 }  // namespace mlv

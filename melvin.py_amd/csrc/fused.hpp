@@ -265,15 +265,13 @@ __host__ __device__ constexpr int brows(int nin, int neq, int slots) {
 __host__ __device__ constexpr bool bfits(int nin, int neq, int slots) {
   return ((nin + 1) / 2 <= slots) && (neq <= slots);
 }
-// Points per thread of the z pass of a program with nin inputs and neq
-// equations: 16 up to N = 1024, and at N = 2048 when the program fits the
-// two slots that leaves (for the reason given at fused_points); otherwise
-// the row policy's 32.
+// Points per thread of the LDS-staged z pass of a program with nin inputs and
+// neq equations: 16 up to N = 1024, which leaves more blocks and a smaller
+// register file, and at N = 2048 when the program fits the two slots that
+// leaves; otherwise 32.
 template <typename T>
 __host__ __device__ constexpr int bpoints(int logn, int nin, int neq) {
-  return (logn <= 10 || (logn == 11 && bfits(nin, neq, (kNT * 16) >> 11)))
-             ? 16
-             : fft_points_row<T>(logn);
+  return (logn <= 10 || (logn == 11 && bfits(nin, neq, (kNT * 16) >> 11))) ? 16 : 32;
 }
 __host__ __device__ constexpr int bvar_nin(int v) { return v <= BV_VORT3 ? v + 3 : 6; }
 __host__ __device__ constexpr int bvar_neq(int v) { return v <= BV_VORT3 ? v + 1 : 1; }

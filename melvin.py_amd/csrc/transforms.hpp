@@ -10,8 +10,10 @@ namespace mlv {
 constexpr int kNT = 256;
 
 // The operator-level transforms' split (fft_reg.hpp): log2 of the points per
-// thread, 8 up to 1024 points and 16 above, where a block of a few columns
-// would otherwise pass 1024 threads.
+// thread, 8 up to 1024 points and 16 above.  At 4096 a block of four columns
+// would pass 1024 threads with 8; at 2048 they measure no better (us per
+// launch, 16 and 8: 2048 x 1024 FP32 inverse 8.6 and 8.6, forward 7.8 and 7.8,
+// 2048^2 FP64 14.6 and 15.3, 11.8 and 13.0; 4096 columns FP32 22.2 and 25.0).
 __host__ __device__ constexpr int tr_loge(int logn) { return logn >= 11 ? 4 : 3; }
 // LDS of `slots` transforms of 2^logn points.
 template <typename T>
