@@ -304,13 +304,23 @@ template <typename T>
 __host__ __device__ constexpr size_t z_lds_bytes(int logn, int v) {
   return (size_t)z_waves(v) * (64 / z_tps(logn)) * rf_len(logn, z_loge(logn)) * sizeof(cx<T>);
 }
-// Sizes the register pass takes, in double precision.  At 2048 points, 32 per
-// thread and 250 registers, it loses to the split pass (us per launch, register
-// and split: vortex 2048^2 62 and 52, 4 of them 234 and 227, with a scalar 81
-// and 70; at 1024^2 16 and 17, MHD 24.3 and 26.4).
+// Sizes the register pass takes, in double precision: up to 1024 points, 512
+// for MHD, four of whose six wavefronts have no product to transform back.
+// Above, it loses to the split pass (us per launch, register and split: vortex
+// 2048^2 62 and 52, 4 of them 234 and 227, with a scalar 81 and 70; MHD 1024^2
+// 24.2 and 23.2, 4 of them 77 and 65; MHD 4 x 512^2 21 and 22, vortex 1024^2
+// 16 and 17).
 template <typename T>
 __host__ __device__ constexpr bool z_reg_fits(int logn, int v) {
-  return sizeof(T) == 8 && logn <= 10 && z_lds_bytes<T>(logn, v) <= kLdsMax;
+  return sizeof(T) == 8 && logn <= (v >= BV_MHD1 ? 9 : 10);
+}
+// The LDS-staged pass of double precision is compiled for z extents up to
+// 2^kZLo and for all.
+constexpr int kZLo = 10;
+// Whether program v has a size up to 2^kZLo on that pass under a plan.
+template <typename T>
+__host__ __device__ constexpr bool z_staged_lo(int v, int plan) {
+  return plan == kPlanTwoSweep || !z_reg_fits<T>(kZLo, v);
 }
 // Whether register m of a thread holds a kept coefficient or its mirror.
 __host__ __device__ constexpr bool z_any(int m, int tps, int n) {

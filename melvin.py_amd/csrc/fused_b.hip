@@ -30,8 +30,11 @@ __global__ void __launch_bounds__(64 * z_waves(V))
 
 // The LDS-staged pass.  Single precision is held to 128 VGPRs: four
 // wavefronts per SIMD, as many as the four blocks per CU its LDS allows at
-// 1024 points.
-template <typename T, int V, int SPLIT, int PLAN>
+// 1024 points.  Double precision has the extents up to 1024 in a kernel of
+// their own (LO): the larger ones' 32 points per thread take 178 VGPRs, which
+// leave two of the three blocks per CU that MHD's LDS allows there (4 x 1024^2
+// 81 us a launch, 65 in the kernel of its own).
+template <typename T, int V, int SPLIT, int PLAN, int LO>
 __global__ void __launch_bounds__(kNT)
     __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 1)))
     k_stepB(const JobDev<T>* __restrict__ jobs, const int* __restrict__ pref, int njobs,
@@ -40,7 +43,7 @@ __global__ void __launch_bounds__(kNT)
   cx<T>* lds = reinterpret_cast<cx<T>*>(smem_raw);
   const int lb = xcd_logical(pref[njobs]);
   if (lb < 0) return;
-  roleB<T, V, SPLIT, PLAN>(jobs, pref, njobs, lb, stage, flags, tw, lds);
+  roleB<T, V, SPLIT, PLAN, LO>(jobs, pref, njobs, lb, stage, flags, tw, lds);
 }
 
 // --------------------------------------------------------------------------
@@ -55,13 +58,22 @@ static void launchZ(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int
                      z.lds[V], s, jobs, (const int*)z.pref[stage][V], bl.njobs, stage, flags, tw);
 }
 
+template <typename T, int V, int SPLIT, int PLAN, int LO>
+static void launchB_lo(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int flags,
+                       const cx<T>* tw, hipStream_t s) {
+  const ZLaunch& b = bl.zsweep[bl.planB];
+  MLV_SET_LDS_ONCE((k_stepB<T, V, SPLIT, PLAN, LO>), b.lds[V]);
+  hipLaunchKernelGGL((k_stepB<T, V, SPLIT, PLAN, LO>), dim3(xcd_grid(b.n[stage][V])), dim3(kNT),
+                     b.lds[V], s, jobs, (const int*)b.pref[stage][V], bl.njobs, stage, flags, tw);
+}
+
 template <typename T, int V, int SPLIT, int PLAN>
 static void launchB_plan(const JobDev<T>* jobs, const BatchLaunch& bl, int stage, int flags,
                          const cx<T>* tw, hipStream_t s) {
-  const ZLaunch& b = bl.zsweep[bl.planB];
-  MLV_SET_LDS_ONCE((k_stepB<T, V, SPLIT, PLAN>), b.lds[V]);
-  hipLaunchKernelGGL((k_stepB<T, V, SPLIT, PLAN>), dim3(xcd_grid(b.n[stage][V])), dim3(kNT),
-                     b.lds[V], s, jobs, (const int*)b.pref[stage][V], bl.njobs, stage, flags, tw);
+  if constexpr (sizeof(T) == 8 && z_staged_lo<T>(V, PLAN))
+    if (bl.lognz_max <= kZLo)
+      return launchB_lo<T, V, SPLIT, PLAN, kZLo>(jobs, bl, stage, flags, tw, s);
+  launchB_lo<T, V, SPLIT, PLAN, 12>(jobs, bl, stage, flags, tw, s);
 }
 
 template <typename T, int V>
@@ -100,12 +112,19 @@ static void prepareB(const BatchLaunch& bl) {
     if constexpr (sizeof(T) == 8)
       if (zl) MLV_SET_LDS_ONCE((k_stepZ<T, V>), zl);
     if (!bs) continue;
-    MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanSplit>), bs);
-    MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanTwoSweep>), bs);
-    if constexpr (sizeof(T) == 4) {
-      MLV_SET_LDS_ONCE((k_stepB<T, V, 1, kPlanSplit>), bs);
-      MLV_SET_LDS_ONCE((k_stepB<T, V, 1, kPlanTwoSweep>), bs);
+    if constexpr (sizeof(T) == 8) {
+      if (bl.lognz_max <= kZLo) {
+        if constexpr (z_staged_lo<T>(V, kPlanSplit))
+          MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanSplit, kZLo>), bs);
+        MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanTwoSweep, kZLo>), bs);
+        continue;
+      }
+    } else {
+      MLV_SET_LDS_ONCE((k_stepB<T, V, 1, kPlanSplit, 12>), bs);
+      MLV_SET_LDS_ONCE((k_stepB<T, V, 1, kPlanTwoSweep, 12>), bs);
     }
+    MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanSplit, 12>), bs);
+    MLV_SET_LDS_ONCE((k_stepB<T, V, 0, kPlanTwoSweep, 12>), bs);
   }
 }
 

@@ -588,8 +588,9 @@ __host__ __device__ constexpr bool bsplit_ok() {
 }
 
 // Kernel B's work for logical block lb of a launch over the job table's
-// z-pass blocks of program V (prefix array pref), in plan PLAN.
-template <typename T, int V, int SPLIT, int PLAN>
+// z-pass blocks of program V (prefix array pref), in plan PLAN.  LO: the
+// largest z extent (log2) of the launch's jobs it is compiled for.
+template <typename T, int V, int SPLIT, int PLAN, int LO>
 __device__ __forceinline__ void roleB(const JobDev<T>* __restrict__ jobs, const int* __restrict__ pref,
                                       int njobs, int lb, int stage, int flags,
                                       const cx<T>* __restrict__ tw, cx<T>* lds) {
@@ -599,7 +600,7 @@ __device__ __forceinline__ void roleB(const JobDev<T>* __restrict__ jobs, const 
   switch (J.lognz) {
 #define X(L)                                                          \
   case L:                                                             \
-    if constexpr (sizeof(T) == 8 && (L < 9 || (PLAN == kPlanSplit && z_reg_fits<T>(L, V)))) \
+    if constexpr (L > LO || (sizeof(T) == 8 && (L < 9 || (PLAN == kPlanSplit && z_reg_fits<T>(L, V))))) \
       break; /* the register pass's */                                \
     else if constexpr (PLAN == kPlanSplit && bsplit_ok<T, L, V>())    \
       stepB_split<T, L, V, SPLIT>(J, J.st[stage], local, flags, tw, lds); \
