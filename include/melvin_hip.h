@@ -184,9 +184,14 @@ int mlv_velocity_physical(mlv_plan* plan, const void* w, void* psi, void* ux_spe
 /* Variable.vec_dot_nabla (Variable.py:119-128): f_phys = to_physical(f_spec)
  * unless f_spec is NULL, then out_spec = to_spectral(pddx(ux f) + pddz(uz f));
  * ux, uz, f_phys are physical fields.  (FD-z plans beyond nx = 1024 are
- * faster as mlv_to_physical, mlv_flux_divergence and mlv_to_spectral.) */
+ * faster through mlv_advect_stencil.) */
 int mlv_advect(mlv_plan* plan, const void* ux, const void* uz, const void* f_spec, void* f_phys,
                void* out_spec, void* stream);
+/* The same as mlv_to_physical (unless f_spec is NULL), mlv_flux_divergence
+ * and mlv_to_spectral: flux_phys, a physical field that is none of the
+ * others, receives the flux divergence. */
+int mlv_advect_stencil(mlv_plan* plan, const void* ux, const void* uz, const void* f_spec,
+                       void* f_phys, void* flux_phys, void* out_spec, void* stream);
 /* FP64 reduction of n values of type dtype (b used by SUMSQ2/DOT); writes
  * scale * result to out_f64 (device).  plan may be NULL: the call then uses
  * its device's shared partials buffer, which the first *_create call on the

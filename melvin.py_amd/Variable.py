@@ -99,14 +99,7 @@ class Variable:
     def vec_dot_nabla(self, ux, uz, out=None, convert_to_physical=True):
         pl = plan_for(self._params)
         if out is None:
-            # FD z beyond 1024 points along x: a thread of the transform that
-            # forms the flux holds 16 points with the operands of six to eight
-            # columns and spills (us a call, fused against stencil then
-            # transform: 2048x65 FP64 31 and 23 at order 2, 40 and 23 at order
-            # 4; 2048x700 37 and 39, 49 and 39; 4096x512 100 and 60, 156 and
-            # 62; at 1024x513 20 and 24, 22 and 25)
-            fused = pl.fully or pl.nx <= 1024
-            if fused and self._fourier(pl) and all(
+            if self._fourier(pl) and all(
                     isinstance(u, torch.Tensor) and plain(u, pl.real, (pl.nx, pl.nz))
                     for u in (ux, uz)):
                 return self._advect(pl, ux, uz, convert_to_physical)
@@ -146,14 +139,26 @@ class Variable:
                 and own(self, Variable, "pddz") and own(self, Variable, "getp"))
 
     def _advect(self, pl, ux, uz, convert_to_physical):
-        """vec_dot_nabla whose flux divergence is formed inside the forward
-        transform, so the caller's ``out`` is the only thing it leaves out.
-        ux and uz are read in place: one may be this field's own physical
-        array, which the conversion writes first."""
+        """vec_dot_nabla in one call, its flux divergence formed inside the
+        forward transform, so the caller's ``out`` is the only thing it leaves
+        out.  ux and uz are read in place: one may be this field's own
+        physical array, which the conversion writes first."""
         spec = torch.empty((pl.rows, pl.cols), dtype=pl.cplx, device=self._pdata.device)
-        _lib.call("mlv_advect", pl.handle, ptr(ux), ptr(uz),
-                  ptr(self._sdata) if convert_to_physical else ctypes.c_void_p(0),
-                  ptr(self._pdata), ptr(spec), _lib.stream_handle())
+        src = ptr(self._sdata) if convert_to_physical else ctypes.c_void_p(0)
+        if pl.fully or pl.nx <= 1024:
+            _lib.call("mlv_advect", pl.handle, ptr(ux), ptr(uz), src, ptr(self._pdata), ptr(spec),
+                      _lib.stream_handle())
+        else:
+            # FD z beyond 1024 points along x: a thread of the transform that
+            # forms the flux holds 16 points with the operands of six to eight
+            # columns and spills, so the flux is written first (us a call, FP64,
+            # fused and so: 2048x65 31 and 23, 2048x700 37 and 38, at order 4
+            # 48 and 38, 4096x512 97 and 59, at order 4 153 and 61; 1024x513
+            # 20 and 24.  It costs the host 2 us: a loop body at 2048x60 that
+            # waits for its calls alone 181 and 185)
+            flux = torch.empty_like(self._pdata)
+            _lib.call("mlv_advect_stencil", pl.handle, ptr(ux), ptr(uz), src, ptr(self._pdata),
+                      ptr(flux), ptr(spec), _lib.stream_handle())
         return spec
 
     def save(self, dump_counter):

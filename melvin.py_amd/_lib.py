@@ -36,7 +36,8 @@ EXPORTS = (
     "mlv_plan_info", "mlv_to_physical", "mlv_to_spectral", "mlv_spec_op",
     "mlv_fd_op", "mlv_flux_divergence", "mlv_poisson", "mlv_update",
     "mlv_reduce", "mlv_reduce_noalloc", "mlv_combine", "mlv_velocity",
-    "mlv_velocity_physical", "mlv_advect", "mlv_job_work_bytes", "mlv_batch_create", "mlv_batch_rebuild",
+    "mlv_velocity_physical", "mlv_advect", "mlv_advect_stencil", "mlv_job_work_bytes",
+    "mlv_batch_create", "mlv_batch_rebuild",
     "mlv_batch_destroy", "mlv_batch_step", "mlv_batch_graph_step", "mlv_batch_set_dt",
     "mlv_batch_steps", "mlv_batch_profile", "mlv_batch_profile_read",
     "mlv_batch_run", "mlv_batch_job_time", "mlv_batch_tracker", "mlv_batch_autotune",
@@ -138,6 +139,7 @@ def _declare(lib):
         "mlv_velocity": ([vp, vp, vp, vp, vp, vp], i),
         "mlv_velocity_physical": ([vp, vp, vp, vp, vp, vp, vp, vp, vp], i),
         "mlv_advect": ([vp, vp, vp, vp, vp, vp, vp], i),
+        "mlv_advect_stencil": ([vp, vp, vp, vp, vp, vp, vp, vp], i),
         "mlv_job_work_bytes": ([i, i, i, i, i, ctypes.POINTER(sz)], i),
         "mlv_batch_create": ([pp, i, ctypes.POINTER(JobDesc), i], i),
         "mlv_batch_rebuild": ([vp, ctypes.POINTER(JobDesc), i], i),

@@ -763,6 +763,24 @@ int mlv_advect(mlv_plan* p, const void* ux, const void* uz, const void* f_spec, 
   return MLV_OK;
 }
 
+int mlv_advect_stencil(mlv_plan* p, const void* ux, const void* uz, const void* f_spec,
+                       void* f_phys, void* flux_phys, void* out_spec, void* stream) {
+  CHECK_PLAN(p);
+  CHECK_PTR(ux);
+  CHECK_PTR(uz);
+  CHECK_PTR(f_phys);
+  CHECK_PTR(flux_phys);
+  CHECK_PTR(out_spec);
+  if (flux_phys == ux || flux_phys == uz || flux_phys == f_phys)
+    return fail(MLV_ERR_ARG, "flux_phys must be an array of its own");
+  if (f_spec) {
+    const int rc = mlv_to_physical(p, f_spec, f_phys, stream);
+    if (rc) return rc;
+  }
+  const int rc = mlv_flux_divergence(p, ux, uz, f_phys, flux_phys, stream);
+  return rc ? rc : mlv_to_spectral(p, flux_phys, out_spec, stream);
+}
+
 }  // extern "C"
 
 // ---------------------------------------------------------------------------

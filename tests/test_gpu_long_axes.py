@@ -46,3 +46,24 @@ def test_velocity_of_rows_beyond_a_block(mlv, precision):
     assert torch.equal(psi.gets(), sim.get_laplacian_solver().solve(-w.gets()))
     assert torch.equal(uz.gets(), psi.sddx())
     assert torch.equal(ux.getp(), -psi.pddz())
+
+
+def test_flux_of_the_advection_is_an_array_of_its_own(mlv):
+    import torch
+    from melvin_amd import _lib
+    from melvin_amd._plans import plan_for, ptr
+
+    p, sim, bfs, s = _fdz(mlv, 64, 17, "double", 2)
+    pl = plan_for(p)
+    f, ux, uz, flux = (torch.ones((64, 17), device="cuda", dtype=torch.float64) for _ in range(4))
+    spec = torch.empty((pl.rows, pl.cols), device="cuda", dtype=pl.cplx)
+    for bad in (f, ux, uz):
+        with pytest.raises(ValueError, match="flux_phys"):
+            _lib.call("mlv_advect_stencil", pl.handle, ptr(ux), ptr(uz), ptr(s), ptr(f), ptr(bad),
+                      ptr(spec), _lib.stream_handle())
+    _lib.call("mlv_advect_stencil", pl.handle, ptr(ux), ptr(uz), ptr(s), ptr(f), ptr(flux),
+              ptr(spec), _lib.stream_handle())
+    want = torch.empty_like(spec)
+    _lib.call("mlv_advect", pl.handle, ptr(ux), ptr(uz), ptr(s), ptr(f), ptr(want),
+              _lib.stream_handle())
+    assert torch.allclose(spec, want, rtol=0, atol=1e-12 * float(want.abs().max()))
