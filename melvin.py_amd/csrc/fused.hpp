@@ -305,14 +305,17 @@ __host__ __device__ constexpr size_t z_lds_bytes(int logn, int v) {
   return (size_t)z_waves(v) * (64 / z_tps(logn)) * rf_len(logn, z_loge(logn)) * sizeof(cx<T>);
 }
 // Sizes the register pass takes, in double precision: up to 1024 points, 512
-// for MHD, four of whose six wavefronts have no product to transform back.
-// Above, it loses to the split pass (us per launch, register and split: vortex
-// 2048^2 62 and 52, 4 of them 234 and 227, with a scalar 81 and 70; MHD 1024^2
-// 24.2 and 23.2, 4 of them 77 and 65; MHD 4 x 512^2 21 and 22, vortex 1024^2
-// 16 and 17).
+// for three fields and for MHD, four of whose six wavefronts have no product
+// to transform back.  Above, it loses to the split pass (us per launch,
+// register and split: vortex 2048^2 62 and 52, 4 of them 234 and 227, with a
+// scalar 81 and 70; MHD 1024^2 24.2 and 23.2, 4 of them 77 and 65; three
+// fields 1024^2 29.5 and 29.3, 4 of them 95 and 85; MHD 4 x 512^2 21 and 22,
+// vortex 1024^2 16 and 17, three fields 512^2 13 and 15).  The kernel's
+// registers are its largest size's: without 1024 points three fields' other
+// sizes gain too (32 x 512^2 196 -> 160, 128 x 256^2 204 -> 160).
 template <typename T>
 __host__ __device__ constexpr bool z_reg_fits(int logn, int v) {
-  return sizeof(T) == 8 && logn <= (v >= BV_MHD1 ? 9 : 10);
+  return sizeof(T) == 8 && logn <= (v >= BV_VORT3 ? 9 : 10);
 }
 // The LDS-staged pass of double precision is compiled for z extents up to
 // 2^kZLo and for all.

@@ -41,3 +41,27 @@ def test_every_plan_vs_oracle(mlv, nx, nz, name):
             assert rel(g, st[f]) <= 1e-12, (a, z, c, f)
         for g, w in zip(got, shapes.setdefault(z, got)):
             np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("name", ["ddc", "mhd"])
+def test_batch_over_both_z_passes(mlv, name):
+    """One batch on both sides of the register pass's limit: each job's bits
+    are its own run's."""
+    def jobs():
+        out = []
+        for nx, nz in ((16, 512), (16, 1024), (32, 32), (64, 512)):
+            p, start, coeff, _ = _problem(name, nx, nz, 4)
+            out.append(_job(mlv, name, p, start, coeff, "f64"))
+        return out
+
+    together, alone = jobs(), jobs()
+    b = mlv.fused.Batch(together)
+    b.step(2)
+    for j in alone:
+        one = mlv.fused.Batch([j])
+        one.step(2)
+        one.close()
+    for j, k in zip(together, alone):
+        for g, w in zip(j.state(), k.state()):
+            np.testing.assert_array_equal(g, w)
+    b.close()
