@@ -25,12 +25,13 @@ __device__ __forceinline__ T modk(const cx<T>* __restrict__ tw, int k, int logn,
 // the transform are the rows it updates, so the result never goes back
 // through LDS (it did, twice, when a wavefront's columns were transformed in
 // LDS and updated from it).
-// What bounds it: at 16 x 1024^2 FP32 (two fields, AB4) its 597 MB, 150 us =
-// 4.0 TB/s of the 5.2 a copy reaches (148 before); on small grids the chain of
-// one block: 256^2 FP64 14.1 -> 6.8 us, 4 x 512^2 FP32 20.2 -> 9.4, 1024^2 FP64
-// 20.5 -> 18.6.  512-thread blocks, whose Px / Pz runs are twice as long,
-// measured 154 us at 16 x 1024^2 and 38.7 against 30.3 on a mixed batch of
-// double diffusion: more, shorter blocks hide each other's barriers.
+// What bounds it: at 16 x 1024^2 FP32 (two fields, AB4) its 597 MB, 145 us =
+// 4.1 TB/s of the 5.2 a copy reaches (shape 2, below: 138); on small grids the
+// chain of one block: 256^2 FP64 14.1 -> 6.8 us, 4 x 512^2 FP32 20.2 -> 9.4,
+// 1024^2 FP64 20.5 -> 18.6.  512-thread blocks, whose Px / Pz runs are twice
+// as long, measured 4 us more at 16 x 1024^2 and 38.7 against 30.3 us on a
+// mixed batch of double diffusion: more, shorter blocks hide each other's
+// barriers.
 //
 // GROUP (shape 2: single precision, batches of one x size of 512 or 1024
 // points): blocks of a whole column group, 64 threads a column, one wavefront
@@ -41,9 +42,10 @@ __device__ __forceinline__ T modk(const cx<T>* __restrict__ tw, int k, int logn,
 // where its registers would hold two.  What bounds it: the launch's memory
 // traffic, once it is large: 64 x 1024^2 with a scalar 496 us (4.8 TB/s of its
 // 2.39 GB, where a copy reaches 5.2) against 527 in blocks of two columns,
-// which touch each group's lines four times over, and 16 of them 138 against
-// 145.  Below two and a half
-// blocks per CU the chain of one block is longer: 1024^2 16.9 against 12.0.
+// which touch each group's lines four times over (46.5 million requests at the
+// L2 against 26.1, for the same misses), and 16 of them 138 against 145.  Below
+// two and a half blocks per CU the chain of one block is longer: 1024^2 16.9
+// against 12.0.
 template <typename T, int LOGN, int NT, bool GROUP = false>
 __device__ __forceinline__ void stepC_body(const JobDev<T>& J, const StageDev& S, int local, int cur,
                                            int par, const cx<T>* __restrict__ tw, cx<T>* lds) {
